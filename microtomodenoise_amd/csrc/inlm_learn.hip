@@ -13,8 +13,9 @@
 // and the gradient with respect to their input) are implicit GEMMs on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation: a wavefront computes 16
 // consecutive voxels x 16 output channels, K = 27 taps x 16 channels in 14
-// chunks of two taps.  The weight gradients (a reduction over all voxels) and
-// the first layer (one input channel) run on the vector ALUs in FP32.
+// chunks of two taps.  Their weight gradients (a reduction
+// over all voxels) run there too; the first layer (one input channel) runs on
+// the vector ALUs in FP32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -129,16 +130,135 @@ __global__ __launch_bounds__(256) void conv16_mfma(const __bf16 *__restrict__ X,
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradients on the vector ALUs (FP32): dW[tap][k][n] += sum_v
-// X[v + tap][k] * G[v][n] and dB[n] += sum_v G[v][n].  A block of 256 threads
-// = (k, n) pairs takes a chunk of 64 voxels of one row at a time through LDS.
-// Cin is 16 (BF16 activations) or 1 (the FP32 input, layer 1).  Each of the
-// kWgradBlocks blocks writes its partial sums (part[block][tap][k][n], then
-// part[block][NTAP CIN C + n] for the bias) and wgrad_reduce adds them in
-// block order, so training repeats bit for bit.
+// Weight gradients: dW[tap][k][n] = sum_v X[v + tap][k] * G[v][n] and
+// dB[n] = sum_v G[v][n].  Each of at most kWgradBlocks blocks writes its
+// partial sums (part[block][tap][k][n], then part[block][NTAP CIN C + n] for
+// the bias) and wgrad_reduce adds them in a fixed order, so training repeats
+// bit for bit.
 // ---------------------------------------------------------------------------
-constexpr int kWgradBlocks = 2048;
+constexpr int kWgradBlocks = 512;               // two per CU
 constexpr int kWgradStride = NTAP * C * C + C;  // floats per block's partials
+
+// 16 -> 16 channels on v_mfma_f32_16x16x32_bf16: per tap a 16x16 product
+// whose K dimension runs over 32 voxels of an x row, A[k][v] = X[v + tap][k]
+// and B[v][n] = G[v][n], summed in FP32.  A wave keeps the 27 products and
+// the bias (A = 1) in registers over all rows it visits.  Both operands need
+// eight voxels of one channel per lane, the transpose of the channels-last
+// layout: ds_read_b64_tr_b16 reads four voxels of 16 channels per 16 lanes
+// that way, so a shift in x is a shift of 32 bytes and every read of a wave
+// covers 512 contiguous bytes.  (The order of the 32 voxels within K is free:
+// lane group q holds voxels 4q..4q+3 and 16+4q..16+4q+3 in both operands.)
+//
+// A block stages X over a 32x4x4 tile and its halo (2.4 voxels per output,
+// 39 KB) and G (16 KB) per tile, two blocks per CU.  The form before it, one
+// thread per (k, n) pair with 27 shifted copies of X in LDS, read one LDS
+// dword per multiply-add and one block filled a CU's LDS: 37.7 ms a layer on
+// a 256^3 volume against 0.34 ms (680 TFLOP/s), which the tiles' loads
+// through L2 (1.8 GB) and the LDS reads (56 per 28 MFMAs) bound together.
+constexpr int WTX = 32, WTY = 4, WTZ = 4;
+constexpr int WRX = WTX + 2, WRY = WTY + 2, WRZ = WTZ + 2;
+typedef short short4v __attribute__((ext_vector_type(4)));
+
+// eight voxels of this lane's channel: p is the LDS address of the first of
+// 32 voxels of a row, the lane's share of it included
+__device__ __forceinline__ bf16x8 read_voxels(const __bf16 *p)
+{
+    typedef __attribute__((address_space(3))) short4v lds4;
+    const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+    const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 16 * C));
+    bf16x8 r;
+    __builtin_memcpy(&r, &a, 8);
+    __builtin_memcpy(reinterpret_cast<char *>(&r) + 8, &b, 8);
+    return r;
+}
+
+__global__ __launch_bounds__(256, 2) void conv16_wgrad(const __bf16 *__restrict__ X, const __bf16 *__restrict__ G,
+                                                       float *__restrict__ part, ActGeom g)
+{
+    constexpr int XCH = WRX * WRY * WRZ * 2, GCH = WTX * WTY * WTZ * 2;  // 16-byte chunks
+    constexpr int XPT = (XCH + 255) / 256, GPT = GCH / 256;
+    static_assert(GCH % 256 == 0 && WTY * WTZ % 4 == 0, "whole chunks and rows per thread and wave");
+    __shared__ __attribute__((aligned(16))) __bf16 xs[WRZ * WRY * WRX * C];
+    __shared__ __attribute__((aligned(16))) __bf16 gs[WTZ * WTY * WTX * C];
+    static_assert(sizeof(xs) >= NTAP * C * C * sizeof(float), "the block's sums reuse the X tile");
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int ntx = (g.nx + WTX - 1) / WTX, nty = (g.ny + WTY - 1) / WTY, ntz = (g.nz + WTZ - 1) / WTZ;
+    const long tiles = (long)ntx * nty * ntz;
+    const long t0 = tiles * blockIdx.x / gridDim.x, t1 = tiles * (blockIdx.x + 1) / gridDim.x;
+
+    floatx4 acc[NTAP], accb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NTAP; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.f;
+    // this lane's share of a 32-voxel read: voxel 4 q + (lane % 16) / 4, channels 4 (lane % 4) ..
+    const int share = (4 * (lane >> 4) + ((lane & 15) >> 2)) * C + 4 * (lane & 3);
+
+    for (long tile = t0; tile < t1; tile++) {
+        const int x0 = (int)(tile % ntx) * WTX, y0 = (int)(tile / ntx % nty) * WTY, z0 = (int)(tile / ((long)ntx * nty)) * WTZ;
+        // region voxel (rx, ry, rz) is the padded voxel (x0 + rx, y0 + ry, z0 + rz); past the padded volume it is zero
+        const __bf16 *xo = X + ((long)z0 * g.sy + (long)y0 * g.sx + x0) * C;
+        const __bf16 *go = G + g.vox(x0, y0, z0) * C;
+        uint4 xr[XPT], gr[GPT];
+#pragma unroll
+        for (int i = 0; i < XPT; i++) {
+            const int ch = t + i * 256, v = ch >> 1;
+            const int rx = v % WRX, ry = v / WRX % WRY, rz = v / (WRX * WRY);
+            xr[i] = uint4{0, 0, 0, 0};
+            if (ch < XCH && x0 + rx < g.nx + 2 && y0 + ry < g.ny + 2 && z0 + rz < g.nz + 2)
+                xr[i] = *reinterpret_cast<const uint4 *>(xo + ((long)rz * g.sy + (long)ry * g.sx + rx) * C + 8 * (ch & 1));
+        }
+#pragma unroll
+        for (int i = 0; i < GPT; i++) {
+            const int ch = t + i * 256, v = ch >> 1;
+            const int rx = v % WTX, ry = v / WTX % WTY, rz = v / (WTX * WTY);
+            gr[i] = uint4{0, 0, 0, 0};
+            if (x0 + rx < g.nx && y0 + ry < g.ny && z0 + rz < g.nz)
+                gr[i] = *reinterpret_cast<const uint4 *>(go + ((long)rz * g.sy + (long)ry * g.sx + rx) * C + 8 * (ch & 1));
+        }
+        __syncthreads();  // the tile before this one has been read
+#pragma unroll
+        for (int i = 0; i < XPT; i++)
+            if (t + i * 256 < XCH) *reinterpret_cast<uint4 *>(xs + 8 * (t + i * 256)) = xr[i];
+#pragma unroll
+        for (int i = 0; i < GPT; i++) *reinterpret_cast<uint4 *>(gs + 8 * (t + i * 256)) = gr[i];
+        __syncthreads();
+        for (int r = wave; r < WTY * WTZ; r += 4) {
+            const int ry = r % WTY, rz = r / WTY;
+            const bf16x8 b = read_voxels(gs + r * WTX * C + share);
+            accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b, accb, 0, 0, 0);
+            const __bf16 *xrow = xs + ((rz * WRY + ry) * WRX) * C + share;
+#pragma unroll
+            for (int tap = 0; tap < NTAP; tap++) {
+                const bf16x8 a = read_voxels(xrow + ((tap / 9) * WRY * WRX + (tap / 3 % 3) * WRX + tap % 3) * C);
+                acc[tap] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[tap], 0, 0, 0);
+            }
+        }
+    }
+    // the block's sums, wave after wave: lane l holds rows k = 4 (l / 16) + i of column n = l % 16
+    float *sum = reinterpret_cast<float *>(xs), *sumb = reinterpret_cast<float *>(gs);
+    const int n = lane & 15, q = lane >> 4;
+    for (int w = 0; w < 4; w++) {
+        __syncthreads();
+        if (wave == w) {
+#pragma unroll
+            for (int tap = 0; tap < NTAP; tap++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float *d = sum + (tap * C + 4 * q + i) * C + n;
+                    *d = w == 0 ? acc[tap][i] : *d + acc[tap][i];
+                }
+            if (q == 0) sumb[n] = w == 0 ? accb[0] : sumb[n] + accb[0];
+        }
+    }
+    __syncthreads();
+    float *pb = part + (long)blockIdx.x * kWgradStride;
+    for (int i = t; i < NTAP * C * C; i += 256) pb[i] = sum[i];
+    if (t < C) pb[NTAP * C * C + t] = sumb[t];
+}
+
+// The first layer (one FP32 input channel): dW[tap][n] = sum_v X[v + tap] G[v][n].
 template <int CIN>
 __global__ __launch_bounds__(256) void conv_wgrad(const void *__restrict__ Xv, const __bf16 *__restrict__ G,
                                                   float *__restrict__ part, ActGeom g, int rows_per_block)
@@ -191,17 +311,27 @@ __global__ __launch_bounds__(256) void conv_wgrad(const void *__restrict__ Xv, c
     }
 }
 
-// dW[e] += sum over blocks b (in order) of part[b][e], e < NTAP CIN C, and
-// dB likewise from the bias partials
+// dW[e] = sum over blocks of part[block][e], e < NTAP CIN C, and dB likewise
+// from the bias partials.  Four threads share an element (blocks b, b + 4,
+// ...), 64 consecutive elements a block, so a block's reads are 256
+// contiguous bytes and the chain of one thread is a quarter of the partials.
 __global__ __launch_bounds__(256) void wgrad_reduce(const float *__restrict__ part, int nblocks, int nw,
                                                     float *__restrict__ dW, float *__restrict__ dB)
 {
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= nw + C) return;
+    __shared__ float sh[4][64];
+    const int e = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
     float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += part[(long)b * kWgradStride + e];
-    if (e < nw) dW[e] += s;
-    else dB[e - nw] += s;
+    if (e < nw + C) {
+#pragma unroll 8
+        for (int b = w; b < nblocks; b += 4) s += part[(long)b * kWgradStride + e];
+    }
+    sh[w][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (w == 0 && e < nw + C) {
+        s = (sh[0][e & 63] + sh[1][e & 63]) + (sh[2][e & 63] + sh[3][e & 63]);
+        if (e < nw) dW[e] = s;
+        else dB[e - nw] = s;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -745,24 +875,25 @@ hipError_t ProposalNet::run(const float *vol, const int shape[3], const float *m
         const long nrows = g.ny * (long)g.nz;
         const int rpb = (int)((nrows + kWgradBlocks - 1) / kWgradBlocks);
         const unsigned wgb = (unsigned)((nrows + rpb - 1) / rpb);
-        auto reduce = [&](int cin, float *dW, float *dB) {
+        const long wtiles = (long)((g.nx + WTX - 1) / WTX) * ((g.ny + WTY - 1) / WTY) * ((g.nz + WTZ - 1) / WTZ);
+        const unsigned wtb = (unsigned)std::min<long>(wtiles, kWgradBlocks);
+        auto reduce = [&](int cin, int nblocks, float *dW, float *dB) {
             const int nw = NTAP * cin * C;
-            hipLaunchKernelGGL(wgrad_reduce, dim3((unsigned)((nw + C + 255) / 256)), dim3(256), 0, m.st, m.wpart,
-                               (int)wgb, nw, dW, dB);
+            hipLaunchKernelGGL(wgrad_reduce, dim3((unsigned)((nw + C + 63) / 64)), dim3(256), 0, m.st, m.wpart,
+                               nblocks, nw, dW, dB);
         };
         int cur = 0;
         for (int l = 2; l >= 0; l--) {
             // convolution l+2: input act[l], gradient at its output gbuf[cur]
-            hipLaunchKernelGGL(conv_wgrad<C>, dim3(wgb), dim3(256), 0, m.st, (const void *)m.act[l], m.gbuf[cur],
-                               m.wpart, g, rpb);
-            reduce(C, G + m.off_w[l], G + m.off_b[l]);
+            hipLaunchKernelGGL(conv16_wgrad, dim3(wtb), dim3(256), 0, m.st, m.act[l], m.gbuf[cur], m.wpart, g);
+            reduce(C, (int)wtb, G + m.off_w[l], G + m.off_b[l]);
             hipLaunchKernelGGL(conv16_mfma, dim3(cb), dim3(256), 0, m.st, m.gbuf[cur], m.wb[l],
                                (const float *)nullptr, m.act[l], m.gbuf[cur ^ 1], g, 1);
             cur ^= 1;
         }
         hipLaunchKernelGGL(conv_wgrad<1>, dim3(wgb), dim3(256), 0, m.st, (const void *)m.in, m.gbuf[cur], m.wpart,
                            g, rpb);
-        reduce(1, G + m.off_w1, G + m.off_b1);
+        reduce(1, (int)wgb, G + m.off_w1, G + m.off_b1);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (loss_host) {

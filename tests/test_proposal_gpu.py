@@ -99,6 +99,36 @@ def test_proposal_gradients_match_oracle(gpu_available):
         assert e_x <= 1e-1, name
 
 
+@pytest.mark.parametrize("shape", [(3, 5, 33), (4, 4, 32), (9, 5, 31), (1, 9, 65), (5, 1, 2), (8, 12, 100)])
+def test_gradients_at_tile_edges(gpu_available, shape):
+    """Volumes around the 32x4x4 tiles of the weight gradients, with the
+    budget of the larger volume's test: both sides round the same activations
+    and gradients to BF16, and a sum in another order flips few of them."""
+    ns = 19
+    nz, ny, nx = shape
+    rng = np.random.default_rng(nx)
+    vol = (rng.normal(size=shape) * 300 + 2000).astype(np.float32)
+    _, nt = PO.tile_index(shape)
+    mass = rng.uniform(0.0, 4.0, size=(nt, ns)).astype(np.float32)
+    mass[:, :4] += 20.0
+    net = PR.OffsetProposal(ns, seed=21)
+    params = net.get_params()
+    vd, md = torch.from_numpy(vol).cuda(), torch.from_numpy(mass).cuda()
+    print(f"[gpu] gradients {shape}", flush=True)
+    # a larger volume first, so that the step runs in buffers that held another shape
+    big = torch.from_numpy(rng.normal(size=(9, 17, 70)).astype(np.float32)).cuda()
+    net.predict(big.data_ptr(), [70, 17, 9])
+    loss = net.train_step(vd.data_ptr(), [nx, ny, nz], md.data_ptr(), 0.0)
+    grads = net.grads()
+    net.close()
+    lo, go, _ = PO.forward_backward(vol, params, ns, mass, bf16=True)
+    assert abs(loss - lo) <= 2e-4 * abs(lo)
+    for name, sl in PO.block_slices(ns):
+        err = np.linalg.norm(grads[sl] - go[sl]) / max(np.linalg.norm(go[sl]), 1e-12)
+        print(f"[gpu]   {name}: rel err {err:.2e}", flush=True)
+        assert err <= 2e-2, name
+
+
 def test_adam_update(gpu_available):
     ns, shape, vol, mass = _net_case(2)
     nz, ny, nx = shape
