@@ -13,9 +13,9 @@
 // and the gradient with respect to their input) are implicit GEMMs on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation: a wavefront computes 16
 // consecutive voxels x 16 output channels, K = 27 taps x 16 channels in 14
-// chunks of two taps.  Their weight gradients (a reduction
-// over all voxels) run there too; the first layer (one input channel) runs on
-// the vector ALUs in FP32.
+// chunks of two taps.  Their weight gradients (a reduction over all voxels)
+// run there too; the first layer (one input channel) runs on the vector ALUs
+// in FP32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -138,6 +138,9 @@ __global__ __launch_bounds__(256) void conv16_mfma(const __bf16 *__restrict__ X,
 // ---------------------------------------------------------------------------
 constexpr int kWgradBlocks = 512;               // two per CU
 constexpr int kWgradStride = NTAP * C * C + C;  // floats per block's partials
+constexpr int kHeadShares = 64;                 // partials of the head's gradient
+static_assert(kHeadShares * (C + 1) * (long)kMaxProposalOffsets <= (long)kWgradBlocks * kWgradStride,
+              "the head's partials fit the same buffer");
 
 // 16 -> 16 channels on v_mfma_f32_16x16x32_bf16: per tap a 16x16 product
 // whose K dimension runs over 32 voxels of an x row, A[k][v] = X[v + tap][k]
@@ -258,80 +261,112 @@ __global__ __launch_bounds__(256, 2) void conv16_wgrad(const __bf16 *__restrict_
     if (t < C) pb[NTAP * C * C + t] = sumb[t];
 }
 
-// The first layer (one FP32 input channel): dW[tap][n] = sum_v X[v + tap] G[v][n].
-template <int CIN>
-__global__ __launch_bounds__(256) void conv_wgrad(const void *__restrict__ Xv, const __bf16 *__restrict__ G,
-                                                  float *__restrict__ part, ActGeom g, int rows_per_block)
+// The first layer (one FP32 input channel): dW[tap][n] = sum_v X[v + tap] G[v][n]
+// in FP32.  A wave takes 64 voxels of a row, one a lane, and one dz: nine X
+// values and 16 G values a lane feed 144 multiply-adds into registers, so the
+// vector ALUs bound it (14.5 GFLOP on a 256^3 volume: 0.18 ms at their rate);
+// the loads of the next 64 voxels are in flight meanwhile, two waves a SIMD.
+// A thread per channel with X in LDS read one dword per multiply-add and used
+// 16 of 256 threads: 4.2 ms with 2048 blocks there, 0.77 ms here.
+__global__ __launch_bounds__(192, 2) void conv1_wgrad(const float *__restrict__ X, const __bf16 *__restrict__ G,
+                                                      float *__restrict__ part, ActGeom g)
 {
-    constexpr int CH = 64;                   // voxels per chunk along x
-    __shared__ float xs[NTAP][CH][CIN];     // X at the 27 shifted positions
-    __shared__ float gs[CH][C];
-    const int tid = threadIdx.x;
-    const int k = tid / C, n = tid % C;     // valid for CIN = 16; CIN = 1 uses k = 0 and tid < 16
-    float acc[NTAP];
+    const int lane = threadIdx.x & 63, dz = (threadIdx.x >> 6) - 1;
+    const int nxc = (g.nx + 63) / 64;
+    const long units = (long)nxc * g.ny * g.nz;
+    const long u0 = units * blockIdx.x / gridDim.x, u1 = units * (blockIdx.x + 1) / gridDim.x;
+    int xc = (int)(u0 % nxc), y = (int)(u0 / nxc % g.ny), z = (int)(u0 / ((long)nxc * g.ny));
+    float acc[9][C], accb[C];
 #pragma unroll
-    for (int t = 0; t < NTAP; t++) acc[t] = 0.f;
-    float accb = 0.f;
-    const long nrows = (long)g.ny * g.nz;
-    const long r0 = (long)blockIdx.x * rows_per_block;
-    for (long r = r0; r < r0 + rows_per_block && r < nrows; r++) {
-        const int y = (int)(r % g.ny), z = (int)(r / g.ny);
-        for (int x0 = 0; x0 < g.nx; x0 += CH) {
-            const int nv = g.nx - x0 < CH ? g.nx - x0 : CH;
-            __syncthreads();
-            for (int i = tid; i < CH * C; i += 256) {
-                const int xv = i / C, c = i % C;
-                gs[xv][c] = xv < nv ? bf2f(G[g.vox(x0 + xv, y, z) * C + c]) : 0.f;
-            }
-            for (int i = tid; i < NTAP * CH * CIN; i += 256) {
-                const int t = i / (CH * CIN), rem = i % (CH * CIN), xv = rem / CIN, c = rem % CIN;
-                float val = 0.f;
-                if (xv < nv) {
-                    const long v = g.vox(x0 + xv, y, z) + tap_off(g, t);
-                    if constexpr (CIN == 1) val = static_cast<const float *>(Xv)[v];
-                    else val = bf2f(static_cast<const __bf16 *>(Xv)[v * C + c]);
-                }
-                xs[t][xv][c] = val;
-            }
-            __syncthreads();
-            if (CIN == C || tid < C) {
-                for (int xv = 0; xv < nv; xv++) {
-                    const float gv = gs[xv][n];
-                    accb += gv;
+    for (int i = 0; i < 9; i++)
 #pragma unroll
-                    for (int t = 0; t < NTAP; t++) acc[t] = __builtin_fmaf(xs[t][xv][CIN == 1 ? 0 : k], gv, acc[t]);
-                }
+        for (int c = 0; c < C; c++) acc[i][c] = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; c++) accb[c] = 0.f;
+    float xv[9];
+    uint4 gr[2];
+    // lanes past the row read its last voxel against a zero gradient
+    auto load = [&](float (&xo)[9], uint4 (&go)[2]) __attribute__((always_inline)) {
+        const int x = xc * 64 + lane;
+        const long v = g.vox(x < g.nx ? x : g.nx - 1, y, z);
+        const float *p = X + v + (long)dz * g.sy;
+#pragma unroll
+        for (int i = 0; i < 9; i++) xo[i] = p[(i / 3 - 1) * g.sx + i % 3 - 1];
+        const uint4 *q = reinterpret_cast<const uint4 *>(G + v * C);
+        const uint4 zero = {0, 0, 0, 0};
+        go[0] = x < g.nx ? q[0] : zero;
+        go[1] = x < g.nx ? q[1] : zero;
+    };
+    if (u0 < u1) load(xv, gr);
+    for (long u = u0; u < u1; u++) {
+        if (++xc == nxc) {
+            xc = 0;
+            if (++y == g.ny) {
+                y = 0;
+                z++;
             }
         }
+        float xn[9];
+        uint4 gn[2];
+        if (u + 1 < u1) load(xn, gn);
+        unsigned w[8];
+        __builtin_memcpy(w, gr, sizeof w);
+        float gv[C];
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            gv[c] = __builtin_bit_cast(float, (c & 1) != 0 ? w[c >> 1] & 0xffff0000u : w[c >> 1] << 16);
+#pragma unroll
+        for (int i = 0; i < 9; i++)
+#pragma unroll
+            for (int c = 0; c < C; c++) acc[i][c] = __builtin_fmaf(xv[i], gv[c], acc[i][c]);
+        if (dz == 0)
+#pragma unroll
+            for (int c = 0; c < C; c++) accb[c] += gv[c];
+#pragma unroll
+        for (int i = 0; i < 9; i++) xv[i] = xn[i];
+        gr[0] = gn[0];
+        gr[1] = gn[1];
     }
+    auto wave_total = [](float v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+        return v;
+    };
     float *pb = part + (long)blockIdx.x * kWgradStride;
-    if (CIN == C || tid < C) {
-        for (int t = 0; t < NTAP; t++) pb[(t * CIN + (CIN == 1 ? 0 : k)) * C + n] = acc[t];
-        if (CIN == 1 || k == 0) pb[NTAP * CIN * C + n] = accb;
-    }
+#pragma unroll
+    for (int i = 0; i < 9; i++)
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const float s = wave_total(acc[i][c]);
+            if (lane == 0) pb[((dz + 1) * 9 + i) * C + c] = s;
+        }
+    if (dz == 0)
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const float s = wave_total(accb[c]);
+            if (lane == 0) pb[NTAP * C + c] = s;
+        }
 }
 
-// dW[e] = sum over blocks of part[block][e], e < NTAP CIN C, and dB likewise
-// from the bias partials.  Four threads share an element (blocks b, b + 4,
-// ...), 64 consecutive elements a block, so a block's reads are 256
-// contiguous bytes and the chain of one thread is a quarter of the partials.
-__global__ __launch_bounds__(256) void wgrad_reduce(const float *__restrict__ part, int nblocks, int nw,
-                                                    float *__restrict__ dW, float *__restrict__ dB)
+// out[e] = sum over blocks of part[block][e], e < n, blocks `stride` floats
+// apart (weights and biases lie side by side in both).  Four threads share an
+// element (blocks b, b + 4, ...), 64 consecutive elements a block, so a
+// block's reads are 256 contiguous bytes and the chain of one thread is a
+// quarter of the partials: 0.68 -> 0.01 ms for 512 partials of a 16 -> 16
+// layer.
+__global__ __launch_bounds__(256) void wgrad_reduce(const float *__restrict__ part, long stride, int nblocks, int n,
+                                                    float *__restrict__ out)
 {
     __shared__ float sh[4][64];
     const int e = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
     float s = 0.f;
-    if (e < nw + C) {
+    if (e < n) {
 #pragma unroll 8
-        for (int b = w; b < nblocks; b += 4) s += part[(long)b * kWgradStride + e];
+        for (int b = w; b < nblocks; b += 4) s += part[(long)b * stride + e];
     }
     sh[w][threadIdx.x & 63] = s;
     __syncthreads();
-    if (w == 0 && e < nw + C) {
-        s = (sh[0][e & 63] + sh[1][e & 63]) + (sh[2][e & 63] + sh[3][e & 63]);
-        if (e < nw) dW[e] = s;
-        else dB[e - nw] = s;
-    }
+    if (w == 0 && e < n) out[e] = (sh[0][e & 63] + sh[1][e & 63]) + (sh[2][e & 63] + sh[3][e & 63]);
 }
 
 // ---------------------------------------------------------------------------
@@ -451,7 +486,6 @@ __global__ __launch_bounds__(256) void head_fwd(const float *__restrict__ feat, 
     }
 }
 
-// dWh[c][s] = sum_t feat[t][c] dl[t][s]; dbh[s] = sum_t dl[t][s]
 // loss = sum of the tiles' terms, in a fixed order (strided per thread,
 // then the block's fixed reduction tree)
 __global__ __launch_bounds__(256) void loss_reduce(const float *__restrict__ tile_loss, int ntiles,
@@ -464,23 +498,32 @@ __global__ __launch_bounds__(256) void loss_reduce(const float *__restrict__ til
     if (threadIdx.x == 0) loss[0] = v;
 }
 
+// dWh[c][s] = sum_t feat[t][c] dl[t][s]; dbh[s] = sum_t dl[t][s]:
+// partial sums over a share of the tiles (blockIdx.y of gridDim.y), added by
+// wgrad_reduce: part[share][c * ns + s], then part[share][C ns + s] for the
+// bias.  kHeadShares blocks along the tiles keep the chip busy where ns / 256
+// blocks alone did not: 2.6 ms for 8192 tiles and 1326 offsets against
+// 0.03 ms.
 __global__ __launch_bounds__(256) void head_bwd_w(const float *__restrict__ feat, const float *__restrict__ dl,
-                                                  int ntiles, int ns, float *__restrict__ dWh, float *__restrict__ dbh)
+                                                  int ntiles, int ns, float *__restrict__ part)
 {
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s >= ns) return;
+    const int t0 = (int)((long)ntiles * blockIdx.y / gridDim.y), t1 = (int)((long)ntiles * (blockIdx.y + 1) / gridDim.y);
     float acc[C], ab = 0.f;
 #pragma unroll
     for (int c = 0; c < C; c++) acc[c] = 0.f;
-    for (int t = 0; t < ntiles; t++) {
+#pragma unroll 4
+    for (int t = t0; t < t1; t++) {
         const float d = dl[(long)t * ns + s];
         ab += d;
 #pragma unroll
         for (int c = 0; c < C; c++) acc[c] = __builtin_fmaf(feat[(long)t * C + c], d, acc[c]);
     }
+    float *pb = part + (long)blockIdx.y * (C + 1) * ns;
 #pragma unroll
-    for (int c = 0; c < C; c++) dWh[(long)c * ns + s] += acc[c];
-    dbh[s] += ab;
+    for (int c = 0; c < C; c++) pb[(long)c * ns + s] = acc[c];
+    pb[(long)C * ns + s] = ab;
 }
 
 // dfeat[t][c] = sum_s dl[t][s] Wh[c][s]  (one block per tile)
@@ -865,35 +908,31 @@ hipError_t ProposalNet::run(const float *vol, const int shape[3], const float *m
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (training) {
         float *G = m.grads;
-        if ((e = hipMemsetAsync(G, 0, m.n_params * sizeof(float), m.st)) != hipSuccess) return e;
-        hipLaunchKernelGGL(head_bwd_w, dim3((m.ns + 255) / 256), dim3(256), 0, m.st, m.feat, m.dl, ntiles, m.ns,
-                           G + m.off_wh, G + m.off_bh);
+        auto reduce = [&](long stride, int nblocks, int n, float *out) {
+            hipLaunchKernelGGL(wgrad_reduce, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, m.st, m.wpart, stride,
+                               nblocks, n, out);
+        };
+        const int shares = std::min(ntiles, kHeadShares);
+        hipLaunchKernelGGL(head_bwd_w, dim3((m.ns + 255) / 256, shares), dim3(256), 0, m.st, m.feat, m.dl, ntiles,
+                           m.ns, m.wpart);
+        reduce((long)(C + 1) * m.ns, shares, (C + 1) * m.ns, G + m.off_wh);
         hipLaunchKernelGGL(head_bwd_x, dim3(ntiles), dim3(256), 0, m.st, m.dl, P + m.off_wh, m.ns, m.dfeat);
         // gradient at the pre-activation of the last convolution
         hipLaunchKernelGGL(pool_bwd, dim3(vb), dim3(256), 0, m.st, m.dfeat, m.act[3], m.gbuf[0], g, ntx, nty);
-        // a fixed number of blocks over the rows, each writing its partials
-        const long nrows = g.ny * (long)g.nz;
-        const int rpb = (int)((nrows + kWgradBlocks - 1) / kWgradBlocks);
-        const unsigned wgb = (unsigned)((nrows + rpb - 1) / rpb);
         const long wtiles = (long)((g.nx + WTX - 1) / WTX) * ((g.ny + WTY - 1) / WTY) * ((g.nz + WTZ - 1) / WTZ);
-        const unsigned wtb = (unsigned)std::min<long>(wtiles, kWgradBlocks);
-        auto reduce = [&](int cin, int nblocks, float *dW, float *dB) {
-            const int nw = NTAP * cin * C;
-            hipLaunchKernelGGL(wgrad_reduce, dim3((unsigned)((nw + C + 63) / 64)), dim3(256), 0, m.st, m.wpart,
-                               nblocks, nw, dW, dB);
-        };
+        const int wtb = (int)std::min<long>(wtiles, kWgradBlocks);
         int cur = 0;
         for (int l = 2; l >= 0; l--) {
             // convolution l+2: input act[l], gradient at its output gbuf[cur]
             hipLaunchKernelGGL(conv16_wgrad, dim3(wtb), dim3(256), 0, m.st, m.act[l], m.gbuf[cur], m.wpart, g);
-            reduce(C, (int)wtb, G + m.off_w[l], G + m.off_b[l]);
+            reduce(kWgradStride, wtb, NTAP * C * C + C, G + m.off_w[l]);
             hipLaunchKernelGGL(conv16_mfma, dim3(cb), dim3(256), 0, m.st, m.gbuf[cur], m.wb[l],
                                (const float *)nullptr, m.act[l], m.gbuf[cur ^ 1], g, 1);
             cur ^= 1;
         }
-        hipLaunchKernelGGL(conv_wgrad<1>, dim3(wgb), dim3(256), 0, m.st, (const void *)m.in, m.gbuf[cur], m.wpart,
-                           g, rpb);
-        reduce(1, (int)wgb, G + m.off_w1, G + m.off_b1);
+        const int w1b = (int)std::min<long>((long)((g.nx + 63) / 64) * g.ny * g.nz, kWgradBlocks);
+        hipLaunchKernelGGL(conv1_wgrad, dim3(w1b), dim3(192), 0, m.st, m.in, m.gbuf[cur], m.wpart, g);
+        reduce(kWgradStride, w1b, NTAP * C + C, G + m.off_w1);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (loss_host) {

@@ -99,9 +99,10 @@ def test_proposal_gradients_match_oracle(gpu_available):
         assert e_x <= 1e-1, name
 
 
-@pytest.mark.parametrize("shape", [(3, 5, 33), (4, 4, 32), (9, 5, 31), (1, 9, 65), (5, 1, 2), (8, 12, 100)])
+@pytest.mark.parametrize("shape", [(3, 5, 33), (4, 4, 32), (9, 5, 31), (1, 9, 65), (5, 1, 2), (8, 12, 100), (9, 66, 290)])
 def test_gradients_at_tile_edges(gpu_available, shape):
-    """Volumes around the 32x4x4 tiles of the weight gradients, with the
+    """Volumes around the 32x4x4 tiles and 64-voxel rows of the weight
+    gradients (and one of 180 tiles, in unequal shares of the head's), with the
     budget of the larger volume's test: both sides round the same activations
     and gradients to BF16, and a sum in another order flips few of them."""
     ns = 19
