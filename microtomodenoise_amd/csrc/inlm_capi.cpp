@@ -84,6 +84,42 @@ inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64
     default: err = "unknown noise mode"; return INLM_BAD_ARG;
     }
 }
+
+size_t cluster_bytes(int nz) { return (size_t)nz * 2 * (sizeof(int64_t) + sizeof(double)); }
+
+inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,
+                            const double *std_dev, void *work, hipStream_t st, float *sig, std::string &err)
+{
+    const int nz = shape[2];
+    const bool windows = p.noise_mode == INLM_NOISE_ZADAPTIVE;
+    const int nwin = windows ? nz : 1;
+    int64_t *bounds_dev = static_cast<int64_t *>(work);
+    double *out_dev = reinterpret_cast<double *>(bounds_dev + 2 * (size_t)nz);
+    std::vector<int64_t> bounds;
+    std::vector<double> got(2 * (size_t)nwin);
+    hipError_t e = hipSuccess;
+    if (windows) {
+        zwindow_bounds(samples, n, shape, p.zwindow, bounds);
+        e = hipMemcpyAsync(bounds_dev, bounds.data(), sizeof(int64_t) * bounds.size(), hipMemcpyHostToDevice, st);
+    }
+    if (e == hipSuccess) e = launch_clusters(std_dev, n, windows ? bounds_dev : nullptr, nwin, out_dev, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(got.data(), out_dev, sizeof(double) * got.size(), hipMemcpyDeviceToHost, st);
+    const hipError_t w = hipStreamSynchronize(st);  // also before the vectors go
+    if (e == hipSuccess) e = w;
+    if (e != hipSuccess) {
+        err = std::string("noise clustering: ") + hipGetErrorString(e);
+        return INLM_HIP_ERROR;
+    }
+    std::vector<double> mean((size_t)nwin), stdev((size_t)nwin);
+    for (int i = 0; i < nwin; i++) {
+        mean[i] = got[2 * (size_t)i];
+        stdev[i] = got[2 * (size_t)i + 1];
+    }
+    if (windows) fill_empty_slices(mean, stdev);
+    const double k = p.stds_from_mean;
+    for (int i = 0; i < nz; i++) sig[i] = (float)(mean[windows ? i : 0] + k * stdev[windows ? i : 0]);
+    return INLM_OK;
+}
 }  // namespace inlm
 
 struct inlm_handle {
@@ -118,6 +154,7 @@ struct inlm_handle {
     int64_t *samples_dev = nullptr;
     double *std_dev = nullptr;
     int64_t samples_cap = 0;
+    void *clusters_dev = nullptr;  // window bounds and results of the noise clustering (inlm::cluster_bytes)
     int64_t semi_ref = -1;  // semimanual noise mode: the reference sample of the first estimate
     bool raw_loaded = false, sigma_set = false;
     int last_iter = 0;
@@ -253,7 +290,7 @@ size_t handle_bytes(const inlm_params &pin, const int32_t shape_in[3])
     if (fast) b += sizeof(float) * vox + inlm::kMomentDoubles * sizeof(double);
     const size_t ns = search_offsets(p.radius_searchspace, p.nslices).size();
     b += 2 * ns * sizeof(SearchEntry) + (ns + kStageMovesPad) * sizeof(int);
-    if (p.noise_mode != INLM_NOISE_MANUAL && p.n_samples > 0) b += (size_t)p.n_samples * (sizeof(int64_t) + sizeof(double));
+    if (p.noise_mode != INLM_NOISE_MANUAL && p.n_samples > 0) b += (size_t)p.n_samples * (sizeof(int64_t) + sizeof(double)) + cluster_bytes(g.nz);
     return b;
 }
 }  // namespace inlm
@@ -488,6 +525,7 @@ inlm_status inlm_destroy(inlm_handle *h)
     (void)hipFree(h->search_fast_dev);
     (void)hipFree(h->samples_dev);
     (void)hipFree(h->std_dev);
+    (void)hipFree(h->clusters_dev);
     (void)hipFree(h->lists_dev);
     (void)hipFree(h->counts_dev);
     (void)hipFree(h->probs_dev);
@@ -679,9 +717,14 @@ inlm_status inlm_sigma_from_patchstd(const inlm_params *p, const int32_t shape[3
     return INLM_OK;
 }
 
-inlm_status inlm_patchstd(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n, double *out)
+}  // extern "C"
+
+namespace {
+
+// Checks the samples and leaves their patch standard deviations in
+// h->std_dev, in flight on the handle's stream.
+inlm_status patchstd_on_device(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n)
 {
-    if (!h || (!samples && n > 0) || (!out && n > 0)) return fail(h, INLM_BAD_ARG, "null argument");
     if (which != 0 && which != 1) return fail(h, INLM_BAD_ARG, "which must be 0 (original) or 1 (result)");
     if (which == 0 && !h->raw_loaded) return fail(h, INLM_BAD_ARG, "no original volume loaded");
     if (which == 1 && h->last_iter < 1) return fail(h, INLM_BAD_ARG, "no result yet");
@@ -717,6 +760,18 @@ inlm_status inlm_patchstd(inlm_handle *h, int32_t which, const int64_t *samples,
         slp = nslice;
     }
     HIP_TRY(h, inlm::launch_patchstd(origin, rowp, slp, h->samples_dev, n, g.nx, nslice, ps, h->std_dev, h->stream));
+    return INLM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+inlm_status inlm_patchstd(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n, double *out)
+{
+    if (!h || (!samples && n > 0) || (!out && n > 0)) return fail(h, INLM_BAD_ARG, "null argument");
+    const inlm_status s = patchstd_on_device(h, which, samples, n);
+    if (s != INLM_OK || n == 0) return s;
     HIP_TRY(h, hipMemcpyAsync(out, h->std_dev, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(h, hipStreamSynchronize(h->stream));
     return INLM_OK;
@@ -725,13 +780,22 @@ inlm_status inlm_patchstd(inlm_handle *h, int32_t which, const int64_t *samples,
 inlm_status inlm_estimate_noise(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n, float *sigma_out)
 {
     if (!h || !sigma_out) return fail(h, INLM_BAD_ARG, "null argument");
+    int shape[3] = {h->geo.nx, h->geo.ny, h->geo.nz};
+    std::string err;
+    if (n > 0 && (h->p.noise_mode == INLM_NOISE_GLOBAL || h->p.noise_mode == INLM_NOISE_ZADAPTIVE)) {
+        // the sample statistics stay on the GPU
+        if (!samples) return fail(h, INLM_BAD_ARG, "null argument");
+        inlm_status s = patchstd_on_device(h, which, samples, n);
+        if (s != INLM_OK) return s;
+        if (!h->clusters_dev) HIP_TRY(h, hipMalloc(&h->clusters_dev, inlm::cluster_bytes(h->geo.nz)));
+        s = inlm::sigma_on_device(h->p, shape, samples, n, h->std_dev, h->clusters_dev, h->stream, sigma_out, err);
+        return s != INLM_OK ? fail(h, s, err) : INLM_OK;
+    }
     std::vector<double> sd((size_t)std::max<int64_t>(n, 1));
     if (h->p.noise_mode != INLM_NOISE_MANUAL) {
         inlm_status s = inlm_patchstd(h, which, samples, n, sd.data());
         if (s != INLM_OK) return s;
     }
-    int shape[3] = {h->geo.nx, h->geo.ny, h->geo.nz};
-    std::string err;
     const inlm_status s = inlm::sigma_from_std(h->p, shape, samples, sd.data(), n, which, h->semi_ref, sigma_out, err);
     if (s != INLM_OK) return fail(h, s, err);
     return INLM_OK;

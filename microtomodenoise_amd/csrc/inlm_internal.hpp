@@ -5,6 +5,8 @@
 #include <functional>
 #include <string>
 
+#include <hip/hip_runtime.h>
+
 #include "inlm_capi.h"
 
 namespace inlm {
@@ -18,6 +20,13 @@ void set_global_error(const std::string &msg);
 // semimanual reference sample between estimates.
 inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64_t *samples, const double *sd,
                            int64_t n, int which, int64_t &semi_ref, float *sig, std::string &err);
+
+// The same in the global and z-adaptive modes from standard deviations on the
+// device (n >= 1), clustered there; work: cluster_bytes(nz) of device memory.
+// Returns when sig is written.
+size_t cluster_bytes(int nz);
+inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,
+                            const double *std_dev, void *work, hipStream_t st, float *sig, std::string &err);
 
 // Device bytes a handle of these parameters allocates for `shape`.
 size_t handle_bytes(const inlm_params &p, const int32_t shape[3]);

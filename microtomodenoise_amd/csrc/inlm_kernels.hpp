@@ -69,6 +69,13 @@ hipError_t launch_selftest_div(unsigned first, unsigned count, unsigned long lon
 hipError_t launch_patchstd(const float *origin, int64_t row_pitch, int64_t slice_pitch, const int64_t *samples,
                            int64_t n, int nx, int64_t nslice, int patchsize, double *out, hipStream_t st);
 
+// Two-cluster hard EM (create2clusters) of values[bounds[2 i] .. bounds[2 i + 1]]
+// for each of nwin windows: out[2 i] the mean and out[2 i + 1] the standard
+// deviation of the lower cluster.  Device pointers; bounds may be null for one
+// window over all n values.
+hipError_t launch_clusters(const double *values, int64_t n, const int64_t *bounds, int nwin, double *out,
+                           hipStream_t st);
+
 // Matrix-core forms (FP32_FAST, FP16, BF16).  Rs/Ps are normalised padded
 // volumes in the form's storage type; raw is the unpadded original in float
 // (returned unchanged where every weight vanishes).

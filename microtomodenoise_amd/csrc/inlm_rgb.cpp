@@ -113,7 +113,7 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
     } sg{st};
 
     const size_t padn = (size_t)geo.voxels_p();
-    DevBuf bR, bP, bO, bU, bS, bSm, bSd;
+    DevBuf bR, bP, bO, bU, bS, bSm, bSd, bC;
     RGB_HIP(hipMalloc(&bR.p, 3 * padn * sizeof(float)));
     RGB_HIP(hipMalloc(&bP.p, 3 * padn * sizeof(float)));
     RGB_HIP(hipMalloc(&bO.p, 3 * npix * sizeof(float)));
@@ -140,20 +140,36 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
         if (!draw_samples(sh, ns, p.patchsize, p.sample_seed, samples.data(), p.circular_mask_diameter))
             return rgb_fail(INLM_BAD_ARG, "no noise sample fits the image (or the circular mask)");
         RGB_HIP(hipMalloc(&bSm.p, (size_t)ns * sizeof(int64_t)));
-        RGB_HIP(hipMalloc(&bSd.p, (size_t)ns * sizeof(double)));
+        RGB_HIP(hipMalloc(&bSd.p, 3 * (size_t)ns * sizeof(double)));
         RGB_HIP(hipMemcpyAsync(bSm.p, samples.data(), (size_t)ns * sizeof(int64_t), hipMemcpyHostToDevice, st));
     }
     std::vector<double> sd((size_t)std::max<int64_t>(ns, 1));
     inlm_params pc = p;
     if (pc.noise_mode == INLM_NOISE_ZADAPTIVE) pc.noise_mode = INLM_NOISE_GLOBAL;
     int64_t semi_ref[3] = {-1, -1, -1};
+    const bool cluster = ns > 0 && pc.noise_mode == INLM_NOISE_GLOBAL;
+    if (cluster) {  // a window of the clustering per channel
+        const int64_t bounds[6] = {0, ns - 1, ns, 2 * ns - 1, 2 * ns, 3 * ns - 1};
+        RGB_HIP(hipMalloc(&bC.p, sizeof(bounds) + 6 * sizeof(double)));
+        RGB_HIP(hipMemcpy(bC.p, bounds, sizeof(bounds), hipMemcpyHostToDevice));
+    }
     auto estimate = [&](const float *chans_dev, int which, float sig[3]) -> inlm_status {
         const int one_slice[3] = {nx, ny, 1};
-        for (int ch = 0; ch < 3; ch++) {
+        double *sd_dev = static_cast<double *>(bSd.p);
+        for (int ch = 0; ch < 3 && ns > 0; ch++)
+            RGB_HIP(launch_patchstd(chans_dev + ch * npix, nx, (int64_t)npix, static_cast<int64_t *>(bSm.p), ns, nx,
+                                    (int64_t)npix, p.patchsize, sd_dev + ch * ns, st));
+        if (cluster) {
+            int64_t *bounds_dev = static_cast<int64_t *>(bC.p);
+            double *out_dev = reinterpret_cast<double *>(bounds_dev + 6), got[6];
+            RGB_HIP(launch_clusters(sd_dev, 3 * ns, bounds_dev, 3, out_dev, st));
+            RGB_HIP(hipMemcpyAsync(got, out_dev, sizeof(got), hipMemcpyDeviceToHost, st));
+            RGB_HIP(hipStreamSynchronize(st));
+            for (int ch = 0; ch < 3; ch++) sig[ch] = (float)(got[2 * ch] + (double)p.stds_from_mean * got[2 * ch + 1]);
+        }
+        for (int ch = 0; ch < 3 && !cluster; ch++) {
             if (ns > 0) {
-                RGB_HIP(launch_patchstd(chans_dev + ch * npix, nx, (int64_t)npix, static_cast<int64_t *>(bSm.p), ns,
-                                        nx, (int64_t)npix, p.patchsize, static_cast<double *>(bSd.p), st));
-                RGB_HIP(hipMemcpyAsync(sd.data(), bSd.p, (size_t)ns * sizeof(double), hipMemcpyDeviceToHost, st));
+                RGB_HIP(hipMemcpyAsync(sd.data(), sd_dev + ch * ns, (size_t)ns * sizeof(double), hipMemcpyDeviceToHost, st));
                 RGB_HIP(hipStreamSynchronize(st));
             }
             std::string err;

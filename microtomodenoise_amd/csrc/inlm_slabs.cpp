@@ -38,6 +38,14 @@ struct Handle {
     }
 };
 
+struct DevBuf {
+    void *p = nullptr;
+    ~DevBuf()
+    {
+        if (p) (void)hipFree(p);
+    }
+};
+
 // z reach of one output: search |dz| <= min(nslices/2, rs_z), patch |dz| <= rp_z
 int z_reach(const inlm_params &p, int nz)
 {
@@ -233,7 +241,20 @@ extern "C" inlm_status inlm_denoise_slabs(const inlm_params *p, const int32_t sh
         }
         const int sh[3] = {nx, ny, nz};
         std::string err;
-        s = inlm::sigma_from_std(*p, sh, samples.data(), sd.data(), ns, which, semi_ref, sig, err);
+        if (ns > 0 && (p->noise_mode == INLM_NOISE_GLOBAL || p->noise_mode == INLM_NOISE_ZADAPTIVE)) {
+            DevBuf stds, work;
+            hipError_t e = hipSetDevice(device);
+            if (e == hipSuccess) e = hipMalloc(&stds.p, sizeof(double) * (size_t)ns);
+            if (e == hipSuccess) e = hipMalloc(&work.p, inlm::cluster_bytes(nz));
+            if (e == hipSuccess) e = hipMemcpy(stds.p, sd.data(), sizeof(double) * (size_t)ns, hipMemcpyHostToDevice);
+            if (e != hipSuccess) {
+                inlm::set_global_error(std::string("inlm_denoise_slabs: ") + hipGetErrorString(e));
+                return e == hipErrorOutOfMemory ? INLM_OOM : INLM_HIP_ERROR;
+            }
+            s = inlm::sigma_on_device(*p, sh, samples.data(), ns, static_cast<double *>(stds.p), work.p, nullptr, sig,
+                                      err);
+        } else
+            s = inlm::sigma_from_std(*p, sh, samples.data(), sd.data(), ns, which, semi_ref, sig, err);
         if (s != INLM_OK) inlm::set_global_error("inlm_denoise_slabs: " + err);
         return s;
     };

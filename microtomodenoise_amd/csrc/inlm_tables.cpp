@@ -232,23 +232,30 @@ void create2clusters(const double *values, int n, int fs, int ls, double &mean, 
     else { mean = m2; stdev = std::sqrt(v2); }
 }
 
-void zwindow_clusters(const int64_t *samples, const double *values, int64_t n, const int shape[3], int windowsize,
-                      std::vector<double> &mean, std::vector<double> &stdev)
+void zwindow_bounds(const int64_t *samples, int64_t n, const int shape[3], int windowsize,
+                    std::vector<int64_t> &bounds)
 {
     const int64_t nslice = (int64_t)shape[0] * shape[1];
     const int nz = shape[2];
-    mean.assign(nz, 0.0);
-    stdev.assign(nz, 0.0);
-    if (n <= 0) return;
+    bounds.assign(2 * (size_t)nz, 0);
     int64_t startpos = 0, endpos = 0;
-    double max_mean = -1.0;
-    bool empty = false;
     for (int pos = 0; pos < nz; pos++) {
         // Window of noiselevel.cpp:541-548: slices in (pos-w/2, pos+w/2]
         // plus the first sample beyond (the reference's endpos stops on it).
-        while (startpos < n - 1 && samples[startpos] / nslice <= (pos - windowsize / 2)) startpos++;
-        while (endpos < n - 1 && samples[endpos] / nslice <= (pos + windowsize / 2)) endpos++;
-        create2clusters(values, (int)n, (int)startpos, (int)endpos, mean[pos], stdev[pos]);
+        const int64_t lo = (int64_t)(pos - windowsize / 2 + 1) * nslice, hi = (int64_t)(pos + windowsize / 2 + 1) * nslice;
+        while (startpos < n - 1 && samples[startpos] < lo) startpos++;
+        while (endpos < n - 1 && samples[endpos] < hi) endpos++;
+        bounds[2 * (size_t)pos] = startpos;
+        bounds[2 * (size_t)pos + 1] = endpos;
+    }
+}
+
+void fill_empty_slices(std::vector<double> &mean, std::vector<double> &stdev)
+{
+    const int nz = (int)mean.size();
+    double max_mean = -1.0;
+    bool empty = false;
+    for (int pos = 0; pos < nz; pos++) {
         max_mean = std::max(max_mean, mean[pos]);
         if (mean[pos] == 0.0) empty = true;
     }
@@ -266,6 +273,20 @@ void zwindow_clusters(const int64_t *samples, const double *values, int64_t n, c
             if (mean[i] == 0.0) empty = true;
         }
     }
+}
+
+void zwindow_clusters(const int64_t *samples, const double *values, int64_t n, const int shape[3], int windowsize,
+                      std::vector<double> &mean, std::vector<double> &stdev)
+{
+    const int nz = shape[2];
+    mean.assign(nz, 0.0);
+    stdev.assign(nz, 0.0);
+    if (n <= 0) return;
+    std::vector<int64_t> b;
+    zwindow_bounds(samples, n, shape, windowsize, b);
+    for (int pos = 0; pos < nz; pos++)
+        create2clusters(values, (int)n, (int)b[2 * (size_t)pos], (int)b[2 * (size_t)pos + 1], mean[pos], stdev[pos]);
+    fill_empty_slices(mean, stdev);
 }
 
 }  // namespace inlm

@@ -48,5 +48,11 @@ void create2clusters(const double *values, int n, int fs, int ls, double &mean, 
 // z-adaptive windows (noiselevel.cpp:529-606) in FP64: out[z] = {mean, std}.
 void zwindow_clusters(const int64_t *samples, const double *values, int64_t n, const int shape[3], int windowsize,
                       std::vector<double> &mean, std::vector<double> &std);
+// Its parts, for the clustering on the GPU (launch_clusters): the first and
+// last sample of each slice's window, bounds[2 z] and bounds[2 z + 1] (n >= 1),
+// and the extrapolation into slices whose window had no valid sample.
+void zwindow_bounds(const int64_t *samples, int64_t n, const int shape[3], int windowsize,
+                    std::vector<int64_t> &bounds);
+void fill_empty_slices(std::vector<double> &mean, std::vector<double> &std);
 
 }  // namespace inlm

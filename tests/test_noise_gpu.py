@@ -55,3 +55,44 @@ def test_noise_modes_schedule_vs_oracle(gpu_available, mode, mask):
         assert np.all(log[0] == np.float32(900.0)) and np.unique(log[1]).size == 1
     want = O.iternlm(raw, op, sigma0=log[0], sigma1=log[1])
     assert np.array_equal(bits(out), bits(want))
+
+
+def _noise_volume(kind):
+    rng = np.random.default_rng(7)
+    v = rng.normal(size=(9, 40, 70)).astype(np.float32) * 50 + 1000
+    if kind == "flat":  # no sample varies: every patch std is zero
+        v[:] = 3.0
+    elif kind == "half-flat":  # zeros are left out; windows without a valid sample are filled from their neighbours
+        v[:5] = 1.0
+    elif kind == "two-level":
+        v[:, :, 35:] *= 40
+    elif kind == "outlier":  # a few samples so far off that both densities underflow
+        v[4, 3, 3] = 1e12
+    elif kind == "tiny":  # densities outside the range the logarithms decide
+        v = (v - 1000) * np.float32(1e-30)
+    return np.ascontiguousarray(v)
+
+
+@pytest.mark.parametrize("n", [1, 2, 1023, 1024, 1025, 4096, 4097, 20011])
+@pytest.mark.parametrize("kind", ["plain", "flat", "half-flat", "two-level", "outlier", "tiny"])
+def test_clustering_on_the_gpu_equals_the_host(gpu_available, kind, n):
+    """Both run the same steps in FP64 and differ by the order of at most
+    2e4-term sums (about 1e-12 relative), so the float results agree to one
+    unit in the last place (1.2e-7)."""
+    raw = _noise_volume(kind)
+    nz, ny, nx = raw.shape
+    samples = _capi.draw_samples([nx, ny, nz], n, 15, 5)
+    for mode, window in (("global", 0), ("z-adaptive", 4), ("z-adaptive", 100)):
+        p = DenoiseParameters(radius_searchspace=[2, 2, 2], radius_patchspace=[1, 1, 1])
+        p.noiselevel.mode = mode
+        p.noiselevel.zwindow = window
+        p.noiselevel.n_samples = n
+        print(f"[gpu] clustering {kind} {mode} {window} n={n}", flush=True)
+        g = IterativeNLM_GPU()
+        assert g.configure_device([nx, ny, nz], p) == nz
+        g.load_raw(raw)
+        stds = g.patchstd(samples)
+        got = g.estimate_noise(samples)
+        g.free_device()
+        want = _capi.sigma_from_patchstd(p.to_c(), [nx, ny, nz], samples, stds)
+        assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
