@@ -133,7 +133,8 @@ struct inlm_handle {
     std::vector<unsigned char> search_fast_blob;  // the fast order and its staging moves, as uploaded
     std::vector<int> tap_dxyz;
     inlm::TapTable taps{};
-    int rp_tiled = 0;
+    int rp_tiled = 0;  // matrix-core forms: the patch radius
+    int tiled = 0;     // FP32 form: the tiled kernel's patch shape, 0 for the per-voxel kernel
     size_t pad_elems = 0;  // allocated elements of each padded volume (>= padded voxels)
     long shifted = 0;      // 16-bit forms: elements from a padded volume to its copy shifted by one
     // FP32 parity form: padded original and previous iterate in float.
@@ -423,8 +424,8 @@ inlm_status inlm_create(const inlm_params *pin, const int32_t shape_in[3], int32
             return fail(nullptr, INLM_BAD_ARG, "the matrix-core forms need an isotropic patch of radius 1, 2 or 3");
         }
         h->rp_tiled = rp[0];
-    } else if (p.kernel_select == 0 && iso && inlm::tiled_taps_match(rp[0], h->tap_dxyz.data(), h->taps.w, h->taps.n))
-        h->rp_tiled = rp[0];
+    } else if (p.kernel_select == 0)
+        h->tiled = inlm::tiled_shape(rp, h->tap_dxyz.data(), h->taps.w, h->taps.n);
 
     inlm_status st = INLM_OK;
     auto bail = [&](inlm_status s) {
@@ -634,7 +635,7 @@ inlm_status run_iteration_impl(inlm_handle *h, int32_t iter, const float *raw, f
                                             h->search_dev, h->search_fast_dev, ns, h->min_lin, h->taps,
                                             h->fg, h->stream, pruned ? &ol : nullptr, h->p.kernel_select == 2));
     } else {
-        HIP_TRY(h, inlm::launch_filter(h->p.precision, h->rp_tiled, h->p.weight_fn, h->R_pad,
+        HIP_TRY(h, inlm::launch_filter(h->p.precision, h->tiled, h->p.weight_fn, h->R_pad,
                                        static_cast<const float *>(P), h->result, h->sigma, h->p.beta, h->search_dev,
                                        ns, h->taps, h->fg, h->stream, mass));
     }
@@ -932,7 +933,7 @@ int64_t inlm_tile_count(const inlm_handle *h) { return h ? (int64_t)tile_count(h
 inlm_status inlm_weight_mass(inlm_handle *h, int32_t iter, float *mass, int32_t is_device)
 {
     if (!h || !mass) return fail(h, INLM_BAD_ARG, "null argument");
-    if (h->fast || h->rp_tiled == 0)
+    if (h->fast || (h->tiled != 111 && h->tiled != 222 && h->tiled != 333))
         return fail(h, INLM_BAD_ARG, "weight mass needs the FP32 form on the tiled kernel (isotropic patch r 1..3)");
     HIP_TRY(h, hipSetDevice(h->device));
     const size_t bytes = sizeof(float) * (size_t)tile_count(h->geo) * h->search.size();

@@ -28,11 +28,11 @@ namespace {
 
 constexpr int NT = 256;   // threads per workgroup of the helper kernels
 constexpr int NTF = 512;  // threads per workgroup of the tiled filter (8 wavefronts)
-constexpr int TX = 32, TY = 8, TZ = 8, VX = 4;  // tile; each thread sums a 4-voxel x-run
+constexpr int TX = 32, VX = 4;  // tile width; each thread sums a 4-voxel x-run
 constexpr float kPadeCut = -3.56648f;
 
 // ---------------------------------------------------------------------------
-// Compile-time patch rows of an isotropic ellipsoid of radius R, in the
+// Compile-time patch rows of an ellipsoid of radii (RX, RY, RZ), in the
 // reference scan order z -> y -> x (iternlm_prepare.cpp:152-203).  Each row
 // (dz,dy) holds the taps dx = -j..j; tap0 is the reference index of its first
 // tap (index 0 is the centre, which leads the list).  Every tap also carries a
@@ -44,15 +44,15 @@ struct Row {
     int dz, dy, j, tap0;
 };
 constexpr int kMaxClasses = 48;
-template <int R>
+template <int RX, int RY, int RZ>
 struct Rows {
-    Row r[4 * R * R + 4 * R + 1];
+    Row r[(2 * RY + 1) * (2 * RZ + 1)];
     int n, ntaps, nclass;
     int key_rho[kMaxClasses], key_z[kMaxClasses];
     static constexpr bool inside(int x, int y, int z)
     {
-        const float rr = (float)R;
-        const float fx = (float)x / rr, fy = (float)y / rr, fz = (float)z / rr;
+        const float fx = (float)x / (float)(RX > 1 ? RX : 1), fy = (float)y / (float)(RY > 1 ? RY : 1),
+                    fz = (float)z / (float)(RZ > 1 ? RZ : 1);
         float e = fx * fx;
         e = e + fy * fy;
         e = e + fz * fz;
@@ -68,10 +68,10 @@ struct Rows {
     constexpr Rows() : r(), n(0), ntaps(0), nclass(1), key_rho(), key_z()
     {
         int tap = 1;
-        for (int z = -R; z <= R; ++z)
-            for (int y = -R; y <= R; ++y) {
+        for (int z = -RZ; z <= RZ; ++z)
+            for (int y = -RY; y <= RY; ++y) {
                 int j = -1;
-                for (int x = 0; x <= R; ++x)
+                for (int x = 0; x <= RX; ++x)
                     if (inside(x, y, z)) j = x;
                 if (j < 0) continue;
                 r[n] = Row{z, y, j, tap};
@@ -89,10 +89,17 @@ struct Rows {
         ntaps = tap;
     }
 };
-template <int R>
-struct RowsOf {
-    static constexpr Rows<R> value{};
-    static_assert(value.nclass <= kMaxClasses, "too many weight classes");
+// A patch shape of the tiled kernel.
+template <int RX_, int RY_, int RZ_>
+struct Patch {
+    static constexpr int RX = RX_, RY = RY_, RZ = RZ_;
+    static constexpr Rows<RX, RY, RZ> rows{};
+    static_assert(rows.nclass <= kMaxClasses, "too many weight classes");
+    // one weight for every tap (1/7, or 1/9 in a plane): the staged squares
+    // are multiplied by it once instead of once per tap
+    static constexpr bool kUniform = RX == 1 && RY == 1 && RZ <= 1;
+    // large patches leave whole wavefronts without a weight above the cutoff
+    static constexpr bool kSkip = rows.ntaps > 50;
 };
 
 // Compiler fence that also pins the running sums: the row's arithmetic must
@@ -125,16 +132,23 @@ __constant__ const unsigned char kLaneCell[64] = {
     8,  9,  10, 11, 12, 13, 36, 37, 24, 25, 26, 27, 40, 41, 52, 53, 54, 55, 42, 43, 56, 57,
     30, 31, 44, 45, 58, 59, 60, 61, 46, 47, 34, 35, 48, 49, 38, 39, 62, 63, 50, 51};  // xr | ty << 3
 
-template <int R>
+template <class PT>
 struct Tile {
-    static constexpr int RX = TX + 2 * R, RY = TY + 2 * R, RZ = TZ + 2 * R;
+    static constexpr int TZ = PT::RZ == 0 ? 1 : 8, TY = PT::RZ == 0 ? 64 : 8;  // a flat patch takes flat tiles
+    static constexpr int RY = TY + 2 * PT::RY, RZ = TZ + 2 * PT::RZ;
+    // LDS column of a tile's first voxel.  Patches of one tap per row outside
+    // the middle one (RX = 1) keep each 4-voxel run on one 16-byte read.
+    static constexpr int O = PT::RX == 1 ? 4 : PT::RX;
     static constexpr int PITCH = kPitch;  // LDS row pitch in floats
-    static_assert(RX <= kPitch, "patch radius too large for the LDS row");
+    static_assert(O + TX + PT::RX <= kPitch, "patch radius too large for the LDS row");
     static constexpr int CPR = PITCH / 4;        // 4-float chunks per row
     static constexpr int NCHUNK = RZ * RY * CPR;
     static constexpr int CPT = (NCHUNK + NTF - 1) / NTF;  // chunks staged per thread
-    static constexpr int LDS = RZ * RY * PITCH;         // floats per buffer
-    static constexpr int WIN = ((VX + 2 * R) + 3) & ~3; // floats read per row window
+    static constexpr int LDS = CPT * NTF * 4;  // floats per buffer: slots past NCHUNK write behind the region
+    // chunks a run reads of a row of half-width j: columns O - j .. O + 3 + j
+    static constexpr int lo(int j) { return (O - j) / 4; }
+    static constexpr int hi(int j) { return (O + 3 + j) / 4; }
+    static constexpr int WIN = 4 * (hi(PT::RX) - lo(PT::RX) + 1);
 };
 
 struct TiledArgs {
@@ -153,20 +167,16 @@ struct TiledArgs {
 
 // Correctly rounded n/d for the operands the Pade weight produces
 // (n in [0, 120], d in [120, 600]: no overflow, underflow or special value):
-// a reciprocal refined by one Newton step, then two remainder corrections
-// with exact fused remainders.  This is the IEEE division sequence without the
-// range scaling and special-value fixup that these operands never need;
-// filter_selftest_div checks it against IEEE division on every float in the
-// weight's domain.
+// the quotient by the hardware reciprocal and one correction with the exact
+// fused remainder.  Both are functions of one float, and
+// filter_selftest_div compares the weight with IEEE division on every float
+// of its domain, so neither a refined reciprocal nor a second correction
+// (four more instructions, as a general division needs) is kept.
 __device__ __forceinline__ float div_pade(float n, float d)
 {
-    float y = __builtin_amdgcn_rcpf(d);
-    const float e = __builtin_fmaf(-d, y, 1.0f);
-    y = __builtin_fmaf(e, y, y);
-    float q = n * y;
-    float r = __builtin_fmaf(-d, q, n);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-d, q, n);
+    const float y = __builtin_amdgcn_rcpf(d);
+    const float q = n * y;
+    const float r = __builtin_fmaf(-d, q, n);
     return __builtin_fmaf(r, y, q);
 }
 
@@ -205,17 +215,27 @@ __device__ __forceinline__ int xcd_swizzle(int wg, int nwg)
     return (wg & 7) * (nwg >> 3) + (wg >> 3);
 }
 
-// Occupancy is bounded by LDS to 3 workgroups of 8 waves per CU (R <= 2) or
-// 2 (R = 3), i.e. 6 or 4 waves per SIMD; the register budget is capped to
-// match so that the scheduler does not trade occupancy for hoisted loads.
-template <int R>
-constexpr int waves_per_eu() { return R <= 2 ? 6 : 4; }
+// Occupancy is bounded by LDS to 4, 3 or 2 workgroups of 8 waves per CU (2, 3
+// or 4 chunks per thread); the register budget is capped to match so that
+// the scheduler does not trade occupancy for hoisted loads.
+template <class PT, bool MASS>
+constexpr int waves_per_eu() { return Tile<PT>::CPT <= 2 && !MASS ? 8 : Tile<PT>::CPT <= 3 ? 6 : 4; }
 
-template <int R, int WFN, bool MASS>
-__global__ __launch_bounds__(NTF) __attribute__((amdgpu_waves_per_eu(waves_per_eu<R>(), waves_per_eu<R>()))) void
+// Vector issue bounds this kernel (no fused multiply-add, no packed FP32: at
+// most one instruction every two cycles per SIMD).  Per offset and output it
+// needs two instructions per tap, 21 issue slots for the weight and 4 for the
+// sums.  The offsets of 62 steps lie in one register per lane, so a step
+// has its addresses at once and issues its loads (R of this offset, the chunks
+// of the next) before anything else; with the offsets read from memory each
+// step waited for three loads one after the other.  Before (with the longer
+// division, a multiply per tap at r = 1 and two reads per row there) and now:
+// r = 1, 3102 offsets of 256^3: 54 and 43 ms; r = 2, 1326 offsets of
+// 301x333x131: 41.6 and 37.6 ms; r = 3, 256x256x96: 40.2 and 39.3 ms.
+template <class PT, int WFN, bool MASS>
+__global__ __launch_bounds__(NTF) __attribute__((amdgpu_waves_per_eu(waves_per_eu<PT, MASS>(), waves_per_eu<PT, MASS>()))) void
 filter_tiled_fp32(TiledArgs a)
 {
-    using T = Tile<R>;
+    using T = Tile<PT>;
     __shared__ __attribute__((aligned(16))) float lds[2][T::LDS];
     __shared__ float red[2][NTF / 64];
 
@@ -225,31 +245,29 @@ filter_tiled_fp32(TiledArgs a)
     const int rem = wg / a.ntx;
     const int by = rem % a.nty;
     const int bz = rem / a.nty;
-    const int X0 = bx * TX, Y0 = by * TY, Z0 = bz * TZ;
+    const int X0 = bx * TX, Y0 = by * T::TY, Z0 = bz * T::TZ;
     const FilterGeom g = a.g;
     const long sp = (long)g.nxp * g.nyp;
+    const float w0 = a.wc[0];
 
-    // Staging: region origin (padded coordinates) is the tile origin minus R.
-    const float *Pbase = a.P + ((long)(Z0 + g.pz - R) * sp + (long)(Y0 + g.py - R) * g.nxp + (X0 + g.px - R));
-    int coff[T::CPT];
+    // Staging: LDS column 0 of region row 0 is voxel (X0 - O, Y0 - RY, Z0 - RZ).
+    const float *pc[T::CPT];
     float p0[T::CPT][4];
 #pragma unroll
     for (int c = 0; c < T::CPT; c++) {
-        int ci = t + c * NTF;
-        if (ci >= T::NCHUNK) ci = 0;  // duplicate of chunk 0, never written
+        const int ci = t + c * NTF < T::NCHUNK ? t + c * NTF : 0;  // slots past the region repeat chunk 0
         const int cx = ci % T::CPR, row = ci / T::CPR;
         const int ry = row % T::RY, rz = row / T::RY;
-        coff[c] = (int)(rz * sp + (long)ry * g.nxp + 4 * cx);
-#pragma unroll
-        for (int e = 0; e < 4; e++) p0[c][e] = Pbase[coff[c] + e];
+        pc[c] = a.P + ((long)(Z0 + g.pz - PT::RZ + rz) * sp + (long)(Y0 + g.py - PT::RY + ry) * g.nxp +
+                       (X0 + g.px - T::O + 4 * cx));
+        __builtin_memcpy(p0[c], pc[c], 16);
     }
 
     // This thread's 4-voxel run.
     const int cell = kLaneCell[t & 63];
-    const int xr = cell & 7, ty = cell >> 3, tz = t >> 6;
+    const int xr = cell & 7, ty = (cell >> 3) + (T::TZ == 1 ? 8 * (t >> 6) : 0), tz = T::TZ == 1 ? 0 : t >> 6;
     const int x0 = X0 + VX * xr, y = Y0 + ty, z = Z0 + tz;
-    const long vox = (long)(z + g.pz) * sp + (long)(y + g.py) * g.nxp + (x0 + g.px);
-    const float *Rv = a.R + vox;
+    const float *Rv = a.R + ((long)(z + g.pz) * sp + (long)(y + g.py) * g.nxp + (x0 + g.px));
     const int zc = z < g.nz ? z : g.nz - 1;
     const float sig = a.sigma[zc];
     const float m = -1.f / (sig * sig * a.beta);
@@ -265,105 +283,110 @@ filter_tiled_fp32(TiledArgs a)
         wmax_bits[v] = 0u;
     }
 
-    const int ldsrow = ((tz + R) * T::RY + (ty + R)) * T::PITCH + VX * xr;
+    const int ldsrow = ((tz + PT::RZ) * T::RY + (ty + PT::RY)) * T::PITCH + VX * xr;
     const int nS = a.n_search;
 
-    auto load_window = [](const float *src, float (&win)[T::WIN]) __attribute__((always_inline)) {
+    // chunks lo..hi of a row: whole 16-byte reads (one ds_read_b128 with an
+    // immediate offset), not the narrowed pieces the compiler would pick
+    auto load_window = [](const float *row, auto jj, float (&win)[T::WIN]) __attribute__((always_inline)) {
+        constexpr int j = decltype(jj)::value;
+        typedef float f4v __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int i = 0; i < T::WIN / 4; i++) {
-            typedef float f4v __attribute__((ext_vector_type(4)));
-            f4v q = *reinterpret_cast<const f4v *>(src + 4 * i);
-            // whole 16-byte reads (one ds_read_b128 with an immediate
-            // offset), not the narrowed pieces the compiler would pick
+        for (int i = T::lo(j); i <= T::hi(j); i++) {
+            f4v q = *reinterpret_cast<const f4v *>(row + 4 * i);
             asm("" : "+v"(q));
-            win[4 * i] = q[0];
-            win[4 * i + 1] = q[1];
-            win[4 * i + 2] = q[2];
-            win[4 * i + 3] = q[3];
+#pragma unroll
+            for (int e = 0; e < 4; e++) win[4 * (i - T::lo(j)) + e] = q[e];
         }
     };
-    auto stage = [&](float (&pn)[T::CPT][4], float *buf) __attribute__((always_inline)) {
+    auto stage = [&](const float (&pn)[T::CPT][4], float *buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < T::CPT; c++) {
-            const int ci = t + c * NTF;
-            if (T::NCHUNK % NTF == 0 || ci < T::NCHUNK) {
-                float4 dv;
-                float q;
-                q = pn[c][0] - p0[c][0]; dv.x = q * q;
-                q = pn[c][1] - p0[c][1]; dv.y = q * q;
-                q = pn[c][2] - p0[c][2]; dv.z = q * q;
-                q = pn[c][3] - p0[c][3]; dv.w = q * q;
-                *reinterpret_cast<float4 *>(buf + 4 * ci) = dv;
+            float dv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float q = pn[c][e] - p0[c][e];
+                dv[e] = q * q;
+                if constexpr (PT::kUniform) dv[e] = dv[e] * w0;
             }
+            __builtin_memcpy(__builtin_assume_aligned(buf + 4 * (t + c * NTF), 16), dv, 16);
         }
     };
     auto load_chunks = [&](float (&pn)[T::CPT][4], int lin) __attribute__((always_inline)) {
-        const float *base = Pbase + lin;
 #pragma unroll
-        for (int c = 0; c < T::CPT; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) pn[c][e] = base[coff[c] + e];
+        for (int c = 0; c < T::CPT; c++) __builtin_memcpy(pn[c], pc[c] + lin, 16);
     };
+    auto lin_at = [&](int k) __attribute__((always_inline)) { return a.search[k < nS ? k : nS - 1].lin; };
 
-    {
-        float pn[T::CPT][4];
-        load_chunks(pn, a.search[0].lin);
-        stage(pn, lds[0]);
-    }
-    __syncthreads();
-
-    for (int k = 0; k < nS; k++) {
-        const int lin = a.search[k].lin;
-        const bool more = (k + 1) < nS;
-        float pn[T::CPT][4];
-        if (more) load_chunks(pn, a.search[k + 1].lin);
-        float rs[VX];
-#pragma unroll
-        for (int v = 0; v < VX; v++) rs[v] = Rv[lin + v];
-
-        const float *L = lds[k & 1] + ldsrow;
+    // offset k from LDS buffer rd, while the chunks of offset k + 1 (the last
+    // offset again past the end) go to wr
+    int linv = 0, kb = 0;
+    auto step = [&](int k, const float *rd, float *wr) __attribute__((always_inline)) {
+        float rs[VX], pn[T::CPT][4];
+        __builtin_memcpy(rs, Rv + __builtin_amdgcn_readlane(linv, k - kb), 16);
+        load_chunks(pn, __builtin_amdgcn_readlane(linv, k + 1 - kb));
+        const float *L = rd + ldsrow;
         float d[VX];
+        float win[2][T::WIN];
         {
             // the centre tap leads the sum (iternlm_prepare.cpp:176-177)
-            float win[T::WIN];
-            load_window(L, win);
-            const float w0 = a.wc[0];
+            load_window(L, std::integral_constant<int, 0>{}, win[1]);
 #pragma unroll
-            for (int v = 0; v < VX; v++) d[v] = win[R + v] * w0;
+            for (int v = 0; v < VX; v++) {
+                const float c = win[1][T::O + v - 4 * T::lo(0)];
+                d[v] = PT::kUniform ? c : c * w0;
+            }
         }
         // Rows in reference order; the window of row i+1 is read while row i
         // is summed.  A compiler barrier per row keeps the optimiser from
         // hoisting every window above the arithmetic (which exhausts the
         // register budget and spills).
-        constexpr int NR = RowsOf<R>::value.n;
-        float win[2][T::WIN];
-        load_window(L + (RowsOf<R>::value.r[0].dz * T::RY + RowsOf<R>::value.r[0].dy) * T::PITCH, win[0]);
+        constexpr int NR = PT::rows.n;
+        constexpr Row first = PT::rows.r[0];
+        load_window(L + (first.dz * T::RY + first.dy) * T::PITCH, std::integral_constant<int, first.j>{}, win[0]);
         static_for<0, NR>([&](auto ri) __attribute__((always_inline)) {
             constexpr int i = decltype(ri)::value;
-            constexpr Row rw = RowsOf<R>::value.r[i];
+            constexpr Row rw = PT::rows.r[i];
             if constexpr (i + 1 < NR) {
-                constexpr Row nx = RowsOf<R>::value.r[i + 1];
-                load_window(L + (nx.dz * T::RY + nx.dy) * T::PITCH, win[(i + 1) & 1]);
+                constexpr Row nx = PT::rows.r[i + 1];
+                load_window(L + (nx.dz * T::RY + nx.dy) * T::PITCH, std::integral_constant<int, nx.j>{}, win[(i + 1) & 1]);
             }
             static_for<0, 2 * rw.j + 1>([&](auto kk) __attribute__((always_inline)) {
                 constexpr int dx = decltype(kk)::value - rw.j;
                 if constexpr (!(rw.dz == 0 && rw.dy == 0 && dx == 0)) {
-                    constexpr int cls = RowsOf<R>::value.class_of(dx, rw.dy, rw.dz);
-                    const float wt = a.wc[cls];
+                    constexpr int cls = PT::rows.class_of(dx, rw.dy, rw.dz);
+                    const float wt = PT::kUniform ? 0.f : a.wc[cls];
 #pragma unroll
-                    for (int v = 0; v < VX; v++) d[v] = d[v] + win[i & 1][R + v + dx] * wt;
+                    for (int v = 0; v < VX; v++) {
+                        const float q = win[i & 1][T::O + v + dx - 4 * T::lo(rw.j)];
+                        d[v] = d[v] + (PT::kUniform ? q : q * wt);
+                    }
                 }
             });
             pin(d);
         });
         float sw = 0.f;
+        bool some = true;
+        if constexpr (PT::kSkip && WFN == 0) {
+            bool any = false;
 #pragma unroll
-        for (int v = 0; v < VX; v++) {
-            const float wt = weight_of<WFN>(d[v] * m);
-            fv[v] = fv[v] + wt * rs[v];
-            fw[v] = fw[v] + wt;
-            wmax_bits[v] = __builtin_elementwise_max(wmax_bits[v], __builtin_bit_cast(unsigned, wt));
-            if constexpr (MASS) sw += (valid && x0 + v < g.nx) ? wt : 0.f;
+            for (int v = 0; v < VX; v++) any = any || d[v] * m > kPadeCut;
+            some = __builtin_amdgcn_ballot_w64(any) != 0;
+        }
+        if (some) {
+#pragma unroll
+            for (int v = 0; v < VX; v++) {
+                const float wt = weight_of<WFN>(d[v] * m);
+                fv[v] = fv[v] + wt * rs[v];
+                fw[v] = fw[v] + wt;
+                wmax_bits[v] = __builtin_elementwise_max(wmax_bits[v], __builtin_bit_cast(unsigned, wt));
+                if constexpr (MASS) sw += (valid && x0 + v < g.nx) ? wt : 0.f;
+            }
+        } else {
+            // every weight of the wavefront is zero: only an infinite or NaN
+            // value still reaches the sum
+#pragma unroll
+            for (int v = 0; v < VX; v++) fv[v] = fv[v] + 0.f * rs[v];
         }
         if constexpr (MASS) {
             // weight mass of this offset over the tile: wave sums into LDS,
@@ -372,7 +395,10 @@ filter_tiled_fp32(TiledArgs a)
             for (int o = 32; o >= 1; o >>= 1) sw += __shfl_xor(sw, o, 64);
             if ((t & 63) == 0) red[k & 1][t >> 6] = sw;
         }
-        if (more) stage(pn, lds[(k + 1) & 1]);
+        // the chunks are in flight until here: without the fence their first
+        // use moves up among the window sums and waits for them
+        __builtin_amdgcn_sched_barrier(0);
+        stage(pn, wr);
         __syncthreads();
         if constexpr (MASS) {
             if (t == 0) {
@@ -381,6 +407,21 @@ filter_tiled_fp32(TiledArgs a)
                 for (int w = 0; w < NTF / 64; w++) tot += red[k & 1][w];
                 a.mass[(long)wg * nS + k] = tot;
             }
+        }
+    };
+    {
+        float pn[T::CPT][4];
+        load_chunks(pn, lin_at(0));
+        stage(pn, lds[0]);
+    }
+    __syncthreads();
+    constexpr int kBlock = 62;  // even; a step looks one offset ahead
+    for (kb = 0; kb < nS; kb += kBlock) {
+        linv = lin_at(kb + (t & 63));
+        const int ke = kb + kBlock < nS ? kb + kBlock : nS;
+        for (int k = kb; k < ke; k += 2) {
+            step(k, lds[0], lds[1]);
+            if (k + 1 < ke) step(k + 1, lds[1], lds[0]);
         }
     }
 
@@ -822,10 +863,30 @@ hipError_t launch_selftest_div(unsigned first, unsigned count, unsigned long lon
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-template <int R>
-static bool taps_match_r(const int *dxyz, int n)
+// Per-class weights of the tiled kernel; false when two taps of one class
+// carry different weights (then the per-voxel kernel must run).
+template <class PT>
+static bool class_weights(const int *dxyz, const float *w, int n, float *wc)
 {
-    constexpr const Rows<R> &rows = RowsOf<R>::value;
+    bool seen[kMaxClasses] = {};
+    for (int i = 0; i < n; i++) {
+        const int c = PT::rows.class_of(dxyz[3 * i], dxyz[3 * i + 1], dxyz[3 * i + 2]);
+        if (c < 0) return false;
+        if (!seen[c]) {
+            wc[c] = w[i];
+            seen[c] = true;
+        } else if (__builtin_memcmp(&wc[c], &w[i], sizeof(float)) != 0)
+            return false;
+        if (PT::kUniform && __builtin_memcmp(&w[0], &w[i], sizeof(float)) != 0) return false;
+    }
+    return true;
+}
+
+// Whether the kernel of this shape sums exactly these taps in this order.
+template <class PT>
+static bool taps_match(const int *dxyz, const float *w, int n)
+{
+    constexpr const auto &rows = PT::rows;
     if (n != rows.ntaps) return false;
     if (dxyz[0] != 0 || dxyz[1] != 0 || dxyz[2] != 0) return false;
     for (int ri = 0; ri < rows.n; ri++) {
@@ -837,37 +898,21 @@ static bool taps_match_r(const int *dxyz, int n)
             tap++;
         }
     }
-    return true;
-}
-
-// Per-class weights of the tiled kernel; false when two taps of one class
-// carry different weights (then the per-voxel kernel must run).
-template <int R>
-static bool class_weights_r(const int *dxyz, const float *w, int n, float *wc)
-{
-    constexpr const Rows<R> &rows = RowsOf<R>::value;
-    bool seen[kMaxClasses] = {};
-    for (int i = 0; i < n; i++) {
-        const int c = rows.class_of(dxyz[3 * i], dxyz[3 * i + 1], dxyz[3 * i + 2]);
-        if (c < 0) return false;
-        if (!seen[c]) {
-            wc[c] = w[i];
-            seen[c] = true;
-        } else if (__builtin_memcmp(&wc[c], &w[i], sizeof(float)) != 0)
-            return false;
-    }
-    return true;
-}
-
-bool tiled_taps_match(int rp, const int *dxyz, const float *w, int n)
-{
     float wc[kMaxClasses];
-    switch (rp) {
-    case 1: return taps_match_r<1>(dxyz, n) && class_weights_r<1>(dxyz, w, n, wc);
-    case 2: return taps_match_r<2>(dxyz, n) && class_weights_r<2>(dxyz, w, n, wc);
-    case 3: return taps_match_r<3>(dxyz, n) && class_weights_r<3>(dxyz, w, n, wc);
-    default: return false;
-    }
+    return class_weights<PT>(dxyz, w, n, wc);
+}
+
+// The patch shapes with a tiled kernel: radii as rx * 100 + ry * 10 + rz.
+#define INLM_TILED_SHAPES(X) X(1, 1, 1) X(2, 2, 2) X(3, 3, 3)
+
+int tiled_shape(const int rp[3], const int *dxyz, const float *w, int n)
+{
+#define INLM_SHAPE(RX, RY, RZ)                                                                       \
+    if (rp[0] == RX && rp[1] == RY && rp[2] == RZ)                                                    \
+        return taps_match<Patch<RX, RY, RZ>>(dxyz, w, n) ? RX * 100 + RY * 10 + RZ : 0;
+    INLM_TILED_SHAPES(INLM_SHAPE)
+#undef INLM_SHAPE
+    return 0;
 }
 
 hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, hipStream_t st)
@@ -878,11 +923,12 @@ hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, 
     return hipGetLastError();
 }
 
-template <int R, int WFN>
+template <class PT, int WFN>
 static hipError_t launch_tiled(const float *Rv, const float *P, float *out, const float *sigma, float beta,
                                const SearchEntry *search, int n_search, const TapTable &taps, const FilterGeom &g,
                                float *mass, hipStream_t st)
 {
+    using T = Tile<PT>;
     TiledArgs a;
     a.mass = mass;
     a.R = Rv;
@@ -894,15 +940,19 @@ static hipError_t launch_tiled(const float *Rv, const float *P, float *out, cons
     a.beta = beta;
     a.g = g;
     a.ntx = (g.nx + TX - 1) / TX;
-    a.nty = (g.ny + TY - 1) / TY;
-    a.ntz = (g.nz + TZ - 1) / TZ;
+    a.nty = (g.ny + T::TY - 1) / T::TY;
+    a.ntz = (g.nz + T::TZ - 1) / T::TZ;
     for (int i = 0; i < kMaxClasses; i++) a.wc[i] = 0.f;
-    if (!class_weights_r<R>(taps.dxyz, taps.w, taps.n, a.wc)) return hipErrorInvalidValue;
-    const long nwg = (long)a.ntx * a.nty * a.ntz;
-    if (mass)
-        hipLaunchKernelGGL((filter_tiled_fp32<R, WFN, true>), dim3((unsigned)nwg), dim3(NTF), 0, st, a);
-    else
-        hipLaunchKernelGGL((filter_tiled_fp32<R, WFN, false>), dim3((unsigned)nwg), dim3(NTF), 0, st, a);
+    if (!class_weights<PT>(taps.dxyz, taps.w, taps.n, a.wc)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((long)a.ntx * a.nty * a.ntz)), block(NTF);
+    if constexpr (PT::RX == PT::RY && PT::RX == PT::RZ) {
+        if (mass) {
+            hipLaunchKernelGGL((filter_tiled_fp32<PT, WFN, true>), grid, block, 0, st, a);
+            return hipGetLastError();
+        }
+    }
+    if (mass) return hipErrorInvalidValue;  // weight mass: isotropic patches, 32x8x8 tiles
+    hipLaunchKernelGGL((filter_tiled_fp32<PT, WFN, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
 
@@ -949,21 +999,22 @@ hipError_t launch_filter_rgb(int weight_fn, const float *const R[3], const float
     return hipGetLastError();
 }
 
-hipError_t launch_filter(int form, int rp, int weight_fn, const float *R, const float *P, float *out,
+hipError_t launch_filter(int form, int shape, int weight_fn, const float *R, const float *P, float *out,
                          const float *sigma, float beta, const SearchEntry *search, int n_search,
                          const TapTable &taps, const FilterGeom &g, hipStream_t st, float *mass)
 {
     if (form != FORM_FP32) return hipErrorInvalidValue;
-#define INLM_TILED(RR)                                                                                   \
-    return weight_fn == 0 ? launch_tiled<RR, 0>(R, P, out, sigma, beta, search, n_search, taps, g, mass, st) \
-                          : launch_tiled<RR, 1>(R, P, out, sigma, beta, search, n_search, taps, g, mass, st)
-    switch (rp) {
-    case 1: INLM_TILED(1);
-    case 2: INLM_TILED(2);
-    case 3: INLM_TILED(3);
+    switch (shape) {
+#define INLM_SHAPE(RX, RY, RZ)                                                                                 \
+    case RX * 100 + RY * 10 + RZ:                                                                              \
+        return weight_fn == 0 ? launch_tiled<Patch<RX, RY, RZ>, 0>(R, P, out, sigma, beta, search, n_search, taps, \
+                                                                   g, mass, st)                               \
+                              : launch_tiled<Patch<RX, RY, RZ>, 1>(R, P, out, sigma, beta, search, n_search, taps, \
+                                                                   g, mass, st);
+        INLM_TILED_SHAPES(INLM_SHAPE)
+#undef INLM_SHAPE
     default: break;
     }
-#undef INLM_TILED
     if (mass) return hipErrorInvalidValue;  // weight mass needs the tiled kernel
     return weight_fn == 0 ? launch_pervoxel<0>(R, P, out, sigma, beta, search, n_search, taps, g, st)
                           : launch_pervoxel<1>(R, P, out, sigma, beta, search, n_search, taps, g, st);

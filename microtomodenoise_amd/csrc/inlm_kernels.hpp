@@ -36,12 +36,12 @@ struct TapTable {
 hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, hipStream_t st);
 
 // One filter pass.  R/P are padded volumes; out is unpadded; sigma has nz
-// entries.  Returns hipErrorInvalidValue when no kernel covers the patch.
-// rp is the (isotropic) patch radius served by a tiled kernel, or 0 to force
+// entries.  shape is the patch shape of a tiled kernel (tiled_shape), or 0 for
 // the per-voxel kernel, which runs any tap table.  With mass != nullptr the
-// tiled kernel also writes, per 32x8x8 tile and search offset, the sum of
-// the weights over the tile's voxels ([tile][offset], tiles x-fastest).
-hipError_t launch_filter(int form, int rp, int weight_fn, const float *R, const float *P, float *out,
+// tiled kernel (isotropic patches only) also writes, per 32x8x8 tile and
+// search offset, the sum of the weights over the tile's voxels
+// ([tile][offset], tiles x-fastest).
+hipError_t launch_filter(int form, int shape, int weight_fn, const float *R, const float *P, float *out,
                          const float *sigma, float beta, const SearchEntry *search, int n_search,
                          const TapTable &taps, const FilterGeom &g, hipStream_t st, float *mass = nullptr);
 
@@ -51,10 +51,10 @@ hipError_t launch_filter_rgb(int weight_fn, const float *const R[3], const float
                              const float mult[3], int independent, const SearchEntry *search, int n_search,
                              const TapTable &taps, const FilterGeom &g, hipStream_t st);
 
-// Whether the tiled kernel for isotropic radius rp uses exactly the given tap
-// order (dx,dy,dz per tap, centre first) and whether all taps it groups into
-// one weight class carry the same weight.
-bool tiled_taps_match(int rp, const int *dxyz, const float *w, int n);
+// The shape (radii as rx * 100 + ry * 10 + rz) of the tiled kernel that sums
+// exactly the given taps in the given order (dx,dy,dz per tap, centre first),
+// with one weight per class of taps; 0 when there is none.
+int tiled_shape(const int rp[3], const int *dxyz, const float *w, int n);
 
 // Exhaustive check of the parity kernel's division: counts weights that
 // differ from IEEE division over the float bit patterns 0x80000000+[first,
