@@ -219,7 +219,7 @@ __device__ __forceinline__ int xcd_swizzle(int wg, int nwg)
 // or 4 chunks per thread); the register budget is capped to match so that
 // the scheduler does not trade occupancy for hoisted loads.
 template <class PT, bool MASS>
-constexpr int waves_per_eu() { return Tile<PT>::CPT <= 2 && !MASS ? 8 : Tile<PT>::CPT <= 3 ? 6 : 4; }
+constexpr int waves_per_eu() { return Tile<PT>::CPT <= 2 && PT::RX <= 2 && !MASS ? 8 : Tile<PT>::CPT <= 3 ? 6 : 4; }
 
 // Vector issue bounds this kernel (no fused multiply-add, no packed FP32: at
 // most one instruction every two cycles per SIMD).  Per offset and output it
@@ -903,7 +903,11 @@ static bool taps_match(const int *dxyz, const float *w, int n)
 }
 
 // The patch shapes with a tiled kernel: radii as rx * 100 + ry * 10 + rz.
-#define INLM_TILED_SHAPES(X) X(1, 1, 1) X(2, 2, 2) X(3, 3, 3)
+// The isotropic ones, those the reference has kernels for
+// (iternlm_cpu_kernels.cpp), and the disks of a single slice.
+#define INLM_TILED_SHAPES(X)                                                             \
+    X(1, 1, 1) X(2, 2, 2) X(3, 3, 3) X(1, 1, 2) X(1, 1, 3) X(2, 2, 1) X(3, 3, 1) X(3, 3, 2) \
+    X(1, 1, 0) X(2, 2, 0) X(3, 3, 0)
 
 int tiled_shape(const int rp[3], const int *dxyz, const float *w, int n)
 {

@@ -70,6 +70,62 @@ def test_tiled_equals_pervoxel_on_ragged_shape(gpu_available, rp):
     assert np.array_equal(bits(outs[0]), bits(ref))
 
 
+@pytest.mark.parametrize("rp", [(1, 1, 2), (1, 1, 3), (2, 2, 1), (3, 3, 1), (3, 3, 2), (1, 1, 0), (2, 2, 0), (3, 3, 0)])
+@pytest.mark.parametrize("shape", [(33, 9, 9), (32, 64, 8), (31, 65, 3), (7, 5, 2), (65, 127, 1)])
+def test_tiled_shapes_at_tile_edges(gpu_available, rp, shape):
+    """The anisotropic patches and the disks around their tiles (32x8x8, and
+    32x64x1 for the disks): the per-voxel kernel's and the oracle's bits,
+    z anisotropy included; a search of 63 offsets or more crosses the lane
+    table's blocks of 62 steps."""
+    nx, ny, nz = shape
+    if nz == 1 and rp[2] > 0:
+        pytest.skip("one slice drops the z radius")
+    rng = np.random.default_rng(nx * ny)
+    raw = (rng.normal(size=(nz, ny, nx)) * 400 + 5000).astype(np.float32)
+    raw[:, ny // 2:] += 3000
+    sig = np.linspace(500, 900, nz).astype(np.float32)
+    for rs, aniso in (((3, 2, 1), 1.0), ((3, 3, 2), 2.5)):
+        rz = 0 if nz == 1 else rs[2]
+        outs = []
+        for kernel in (0, 1):
+            print(f"[gpu] shape {shape} rp={rp} rs={rs} kernel={kernel}", flush=True)
+            g, _ = make_gpu(shape, (rs[0], rs[1], rz), rp, kernel=kernel, z_anisotropy=aniso)
+            g.set_sigma(sig)
+            g.Run_GaussianNoise(1, raw)
+            g.Run_GaussianNoise(2)
+            outs.append(g.get_result())
+            g.free_device()
+        assert np.array_equal(bits(outs[0]), bits(outs[1]))
+        if aniso == 1.0:
+            p = O.Params(radius_searchspace=(rs[0], rs[1], rz), radius_patchspace=rp, blockwise=False)
+            ref = O.filter_iteration(raw, O.filter_iteration(raw, raw, sig, p), sig, p)
+            assert np.array_equal(bits(outs[0]), bits(ref))
+
+
+@pytest.mark.parametrize("rp", [(1, 1, 1), (3, 3, 3), (2, 2, 0)])
+def test_infinite_and_nan_values_reach_the_same_voxels(gpu_available, rp):
+    """A zero weight times an infinite value is a NaN in the sums, also where
+    a wavefront has no weight above the cutoff (skipped for large patches)."""
+    rng = np.random.default_rng(3)
+    raw = (rng.normal(size=(12, 30, 80)) * 400 + 5000).astype(np.float32)
+    raw[5, 7, 11] = np.inf
+    raw[6, 20, 60] = np.nan
+    raw[2, 3, 40] = -np.inf
+    sig = np.full(12, 60.0, np.float32)  # most weights are zero
+    outs = []
+    for kernel in (0, 1):
+        print(f"[gpu] special values rp={rp} kernel={kernel}", flush=True)
+        g, _ = make_gpu((80, 30, 12), (3, 3, 2), rp, kernel=kernel)
+        g.set_sigma(sig)
+        g.Run_GaussianNoise(1, raw)
+        outs.append(g.get_result())
+        g.free_device()
+    assert 0 < np.isnan(outs[1]).sum() < outs[1].size
+    assert np.array_equal(np.isnan(outs[0]), np.isnan(outs[1]))
+    ok = ~np.isnan(outs[1])
+    assert np.array_equal(bits(outs[0][ok]), bits(outs[1][ok]))
+
+
 def test_config1_parity_vs_oracle(gpu_available):
     """Config 1 (128x128x64 uint16 phantom, patch r=1, search r=5, 4
     iterations, fixed sigma lists) against the FP32 restatement: every voxel
