@@ -204,26 +204,6 @@ inlm_status hip_fail(inlm_handle *h, hipError_t e, const char *where)
         if (e_ != hipSuccess) return hip_fail(h, e_, #expr); \
     } while (0)
 
-// Highest element index a filter kernel may read in a padded volume.  The
-// kernels read whole tiles (32x8x8, or 32x64x1 for a flat patch; the block
-// kernel's buffer loads check their range), so for shapes that are not
-// multiples of the tile they read past the padded volume; those voxels feed
-// only discarded outputs, and the allocation covers them.
-size_t padded_alloc_elems(const inlm::Geometry &g, bool flat)
-{
-    const long sp = (long)g.nxp * g.nyp;
-    const long ntx = (g.nx + 31) / 32;
-    const long R = 3, pitch = 40;  // largest tile radius and its LDS pitch
-    const long xmax = (ntx - 1) * 32 + pitch - 1 + 2L * g.px;
-    auto highest = [&](long ty, long tz) {
-        const long nty = (g.ny + ty - 1) / ty, ntz = (g.nz + tz - 1) / tz;
-        return (ntz * tz - 1 + 2L * g.pz) * sp + (nty * ty - 1 + 2L * g.py) * g.nxp + xmax + 2 * R;
-    };
-    long need = std::max<long>(highest(8, 8) + 1, (long)g.voxels_p());
-    if (flat) need = std::max<long>(need, highest(64, 1) + 1);
-    return (size_t)need + 64;
-}
-
 long tile_count(const inlm::Geometry &g)
 {
     return (long)((g.nx + 31) / 32) * ((g.ny + 7) / 8) * ((g.nz + 7) / 8);
@@ -271,6 +251,26 @@ inlm_status ensure_samples(inlm_handle *h, int64_t n)
 }  // namespace
 
 namespace inlm {
+// Highest element index a filter kernel may read in a padded volume.  The
+// kernels read whole tiles (32x8x8, or 32x64x1 for a flat patch; the block
+// kernel's buffer loads check their range), so for shapes that are not
+// multiples of the tile they read past the padded volume; those voxels feed
+// only discarded outputs, and the allocation covers them.
+size_t padded_elems(const inlm::Geometry &g, bool flat)
+{
+    const long sp = (long)g.nxp * g.nyp;
+    const long ntx = (g.nx + 31) / 32;
+    const long R = 3, pitch = 40;  // largest tile radius and its LDS pitch
+    const long xmax = (ntx - 1) * 32 + pitch - 1 + 2L * g.px;
+    auto highest = [&](long ty, long tz) {
+        const long nty = (g.ny + ty - 1) / ty, ntz = (g.nz + tz - 1) / tz;
+        return (ntz * tz - 1 + 2L * g.pz) * sp + (nty * ty - 1 + 2L * g.py) * g.nxp + xmax + 2 * R;
+    };
+    long need = std::max<long>(highest(8, 8) + 1, (long)g.voxels_p());
+    if (flat) need = std::max<long>(need, highest(64, 1) + 1);
+    return (size_t)need + 64;
+}
+
 // Device bytes a handle of these parameters allocates for `shape` (the sums
 // of inlm_create's allocations, plus the sample buffers of one noise
 // estimate with n_samples samples).
@@ -285,7 +285,7 @@ size_t handle_bytes(const inlm_params &pin, const int32_t shape_in[3])
     Geometry g = make_geometry(shape, p.radius_searchspace, p.radius_patchspace, p.nslices);
     const size_t esz = form_elem_size(p.precision);
     if (esz == 2 && (g.nxp & 1) != 0) g.nxp += 1;
-    const size_t pad_elems = padded_alloc_elems(g, p.radius_patchspace[2] == 0);
+    const size_t pad_elems = inlm::padded_elems(g, p.radius_patchspace[2] == 0);
     const bool fast = p.precision != INLM_PREC_FP32;
     const size_t shifted = fast && esz == 2 ? (pad_elems + kGuard + 63) / 64 * 64 : 0;
     const size_t padb = (shifted > 0 ? kGuard + shifted + pad_elems : pad_elems + kGuard) * esz;
@@ -441,7 +441,7 @@ inlm_status inlm_create(const inlm_params *pin, const int32_t shape_in[3], int32
         return bail(hip_fail(nullptr, e, "hipStreamCreate"));
     if ((e = hipEventCreate(&h->ev0)) != hipSuccess || (e = hipEventCreate(&h->ev1)) != hipSuccess)
         return bail(hip_fail(nullptr, e, "hipEventCreate"));
-    h->pad_elems = padded_alloc_elems(g, p.radius_patchspace[2] == 0);
+    h->pad_elems = inlm::padded_elems(g, p.radius_patchspace[2] == 0);
     // kGuard elements in front of each padded volume: the matrix-core staging
     // reads chunks that start up to 3 elements before the volume.  The
     // 16-bit forms follow each volume with a copy shifted by one element

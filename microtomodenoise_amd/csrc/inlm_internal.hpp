@@ -28,6 +28,11 @@ size_t cluster_bytes(int nz);
 inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,
                             const double *std_dev, void *work, hipStream_t st, float *sig, std::string &err);
 
+// Elements of a padded volume's allocation behind its guard (flat: the patch
+// has no z radius).
+struct Geometry;
+size_t padded_elems(const Geometry &g, bool flat);
+
 // Device bytes a handle of these parameters allocates for `shape`.
 size_t handle_bytes(const inlm_params &p, const int32_t shape[3]);
 

@@ -46,10 +46,11 @@ hipError_t launch_filter(int form, int shape, int weight_fn, const float *R, con
                          const TapTable &taps, const FilterGeom &g, hipStream_t st, float *mass = nullptr);
 
 // Three-channel filter of the colour path (iternlm_cpu.cpp:932-1075) on
-// padded FP32 channels; mult[c] = -1 / (sigma_c^2 beta).
-hipError_t launch_filter_rgb(int weight_fn, const float *const R[3], const float *const P[3], float *const out[3],
-                             const float mult[3], int independent, const SearchEntry *search, int n_search,
-                             const TapTable &taps, const FilterGeom &g, hipStream_t st);
+// padded FP32 channels; mult[c] = -1 / (sigma_c^2 beta).  shape as in
+// launch_filter: disks (rz = 0) of one slice run tiled, others per pixel.
+hipError_t launch_filter_rgb(int shape, int weight_fn, const float *const R[3], const float *const P[3],
+                             float *const out[3], const float mult[3], int independent, const SearchEntry *search,
+                             int n_search, const TapTable &taps, const FilterGeom &g, hipStream_t st);
 
 // The shape (radii as rx * 100 + ry * 10 + rz) of the tiled kernel that sums
 // exactly the given taps in the given order (dx,dy,dz per tap, centre first),

@@ -112,14 +112,18 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
         ~StreamGuard() { (void)hipStreamDestroy(s); }
     } sg{st};
 
-    const size_t padn = (size_t)geo.voxels_p();
+    // a guard in front of each padded channel and room for whole tiles behind,
+    // as in the volumes' handles
+    constexpr size_t guard = 64;
+    const size_t padn = (guard + padded_elems(geo, true) + 63) / 64 * 64;
+    const int shape = tiled_shape(p.radius_patchspace, taps.dxyz, taps.w, taps.n);
     DevBuf bR, bP, bO, bU, bS, bSm, bSd, bC;
     RGB_HIP(hipMalloc(&bR.p, 3 * padn * sizeof(float)));
     RGB_HIP(hipMalloc(&bP.p, 3 * padn * sizeof(float)));
     RGB_HIP(hipMalloc(&bO.p, 3 * npix * sizeof(float)));
     RGB_HIP(hipMalloc(&bU.p, 3 * npix * sizeof(float)));
     RGB_HIP(hipMalloc(&bS.p, se.size() * sizeof(SearchEntry)));
-    float *Rd = static_cast<float *>(bR.p), *Pd = static_cast<float *>(bP.p), *Od = static_cast<float *>(bO.p);
+    float *Rd = static_cast<float *>(bR.p) + guard, *Pd = static_cast<float *>(bP.p) + guard, *Od = static_cast<float *>(bO.p);
     float *Ud = static_cast<float *>(bU.p);
     RGB_HIP(hipMemcpyAsync(bS.p, se.data(), se.size() * sizeof(SearchEntry), hipMemcpyHostToDevice, st));
 
@@ -200,7 +204,7 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
         float mult[3];
         for (int ch = 0; ch < 3; ch++) mult[ch] = -1.f / (s0[ch] * s0[ch] * p.beta);  // iternlm_cpu.cpp:384-386
         if (sigma_log) std::memcpy(sigma_log + 3 * (iter - 1), s0, sizeof(s0));
-        RGB_HIP(launch_filter_rgb(p.weight_fn, R3, P3, O3, mult, c->independent_channels, static_cast<SearchEntry *>(bS.p),
+        RGB_HIP(launch_filter_rgb(shape, p.weight_fn, R3, P3, O3, mult, c->independent_channels, static_cast<SearchEntry *>(bS.p),
                                   (int)se.size(), taps, g, st));
         if (on_iteration) {
             RGB_HIP(hipMemcpyAsync(res.data(), Od, 3 * npix * sizeof(float), hipMemcpyDeviceToHost, st));

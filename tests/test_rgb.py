@@ -246,6 +246,22 @@ def test_filter_bit_exact_vs_oracle(gpu_available, rs, rp, shape, independent):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rp", [1, 2, 3, 4])
+@pytest.mark.parametrize("shape", [(64, 32), (65, 33), (63, 31), (130, 65)])
+@pytest.mark.parametrize("independent", [False, True])
+def test_filter_at_tile_edges(gpu_available, rp, shape, independent):
+    """Images around the 32x64 tiles, two iterations; radius 4 runs per pixel."""
+    img = _image(*shape, seed=rp)
+    p = _rgb_params(5, rp, 2, sigma=(14.0, 9.0))
+    print(f"[gpu] rgb tiles rp={rp} shape={shape} independent={independent}", flush=True)
+    out, log = denoise_rgb(img, p, independent_channels=independent, stabilize_variance=False,
+                           average_channelsigma=False)
+    ref = O.filter_rgb(img, img, list(log[0]), _op(5, rp), independent)
+    ref = O.filter_rgb(img, ref, list(log[1]), _op(5, rp), independent)
+    assert np.array_equal(_bits(out), _bits(ref))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("continuous", [False, True])
 @pytest.mark.parametrize("independent", [False, True])
 def test_schedule_manual_sigma_bit_exact(gpu_available, continuous, independent):
