@@ -208,11 +208,15 @@ __device__ __forceinline__ float weight_of(float a)
 
 // Workgroup id -> tile, so that the tiles one XCD runs are contiguous (the
 // hardware deals workgroups to the 8 XCDs round-robin, and neighbouring tiles
-// share their halo in that XCD's L2).
+// share their halo in that XCD's L2), for any number of workgroups: the first
+// nwg % 8 XCDs take one more.  Where the count is no
+// multiple of 8, dealing tiles in order (as before) cost 8% at r = 2 on
+// 301x333x131 (37.6 against 34.8 ms) and 66% on a 1200x900 colour image (1.63
+// against 0.98 ms), whose tiles then came from the other XCDs' side of memory.
 __device__ __forceinline__ int xcd_swizzle(int wg, int nwg)
 {
-    if ((nwg & 7) != 0) return wg;
-    return (wg & 7) * (nwg >> 3) + (wg >> 3);
+    const int xcd = wg & 7, more = nwg & 7;
+    return xcd * (nwg >> 3) + (xcd < more ? xcd : more) + (wg >> 3);
 }
 
 // Chunks lo..hi of a row of half-width J: whole 16-byte reads (one
@@ -627,7 +631,9 @@ __device__ __forceinline__ float third(float x)
 // squares of the three channels are staged together, and every thread sums
 // three stencils of a 4-pixel run and shares one weight (or takes three).  The
 // kernel above gathers two values per tap, channel and offset from global
-// memory: 2.71 ms a pass on 1200x900 at r = 1 and 316 offsets, 1.63 ms here.
+// memory: 2.71 ms a pass on 1200x900 at r = 1 and 316 offsets, 0.98 ms here
+// (vector issue: three times the tap and staging work of the grey kernel per
+// weight; 1.1 rounds of workgroups at that size).
 template <class PT>
 struct RgbTile {
     using T = Tile<PT>;

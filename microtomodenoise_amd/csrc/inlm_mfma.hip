@@ -395,10 +395,11 @@ struct MTile {
     static_assert(UPR % 2 == 0, "8-column chunks must not straddle region rows");
 };
 
+// Workgroup id -> tile: contiguous tiles per XCD (see xcd_swizzle of the FP32 kernels)
 __device__ __forceinline__ int mxcd_swizzle(int wg, int nwg)
 {
-    if ((nwg & 7) != 0) return wg;
-    return (wg & 7) * (nwg >> 3) + (wg >> 3);
+    const int xcd = wg & 7, more = nwg & 7;
+    return xcd * (nwg >> 3) + (xcd < more ? xcd : more) + (wg >> 3);
 }
 
 // Weight of one distance, from the MFMA accumulator d and a per-lane scale.
