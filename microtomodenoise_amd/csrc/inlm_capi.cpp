@@ -85,24 +85,36 @@ inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64
     }
 }
 
-size_t cluster_bytes(int nz) { return (size_t)nz * 2 * (sizeof(int64_t) + sizeof(double)); }
+size_t cluster_bytes(int nz) { return kClusterWorkBytes + (size_t)nz * 2 * (sizeof(int64_t) + sizeof(double)); }
 
 inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,
                             const double *std_dev, void *work, hipStream_t st, float *sig, std::string &err)
 {
     const int nz = shape[2];
     const bool windows = p.noise_mode == INLM_NOISE_ZADAPTIVE;
-    const int nwin = windows ? nz : 1;
-    int64_t *bounds_dev = static_cast<int64_t *>(work);
-    double *out_dev = reinterpret_cast<double *>(bounds_dev + 2 * (size_t)nz);
+    // slices whose windows hold the same samples share one
     std::vector<int64_t> bounds;
+    std::vector<int> of((size_t)nz, 0);
+    int nwin = 1;
+    if (windows) {
+        std::vector<int64_t> all;
+        zwindow_bounds(samples, n, shape, p.zwindow, all);
+        bounds.assign(all.begin(), all.begin() + 2);
+        for (int z = 1; z < nz; z++) {
+            if (all[2 * (size_t)z] != bounds[bounds.size() - 2] || all[2 * (size_t)z + 1] != bounds.back())
+                bounds.insert(bounds.end(), all.begin() + 2 * (size_t)z, all.begin() + 2 * (size_t)z + 2);
+            of[(size_t)z] = (int)(bounds.size() / 2) - 1;
+        }
+        nwin = (int)(bounds.size() / 2);
+    }
+    const bool whole = !windows || (nwin == 1 && bounds[0] == 0 && bounds[1] == n - 1);
+    int64_t *bounds_dev = reinterpret_cast<int64_t *>(static_cast<char *>(work) + kClusterWorkBytes);
+    double *out_dev = reinterpret_cast<double *>(bounds_dev + 2 * (size_t)nz);
     std::vector<double> got(2 * (size_t)nwin);
     hipError_t e = hipSuccess;
-    if (windows) {
-        zwindow_bounds(samples, n, shape, p.zwindow, bounds);
+    if (!whole)
         e = hipMemcpyAsync(bounds_dev, bounds.data(), sizeof(int64_t) * bounds.size(), hipMemcpyHostToDevice, st);
-    }
-    if (e == hipSuccess) e = launch_clusters(std_dev, n, windows ? bounds_dev : nullptr, nwin, out_dev, st);
+    if (e == hipSuccess) e = launch_clusters(std_dev, n, whole ? nullptr : bounds_dev, nwin, out_dev, work, st);
     if (e == hipSuccess) e = hipMemcpyAsync(got.data(), out_dev, sizeof(double) * got.size(), hipMemcpyDeviceToHost, st);
     const hipError_t w = hipStreamSynchronize(st);  // also before the vectors go
     if (e == hipSuccess) e = w;
@@ -110,14 +122,14 @@ inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int6
         err = std::string("noise clustering: ") + hipGetErrorString(e);
         return INLM_HIP_ERROR;
     }
-    std::vector<double> mean((size_t)nwin), stdev((size_t)nwin);
-    for (int i = 0; i < nwin; i++) {
-        mean[i] = got[2 * (size_t)i];
-        stdev[i] = got[2 * (size_t)i + 1];
+    std::vector<double> mean((size_t)nz), stdev((size_t)nz);
+    for (int z = 0; z < nz; z++) {
+        mean[(size_t)z] = got[2 * (size_t)of[(size_t)z]];
+        stdev[(size_t)z] = got[2 * (size_t)of[(size_t)z] + 1];
     }
     if (windows) fill_empty_slices(mean, stdev);
     const double k = p.stds_from_mean;
-    for (int i = 0; i < nz; i++) sig[i] = (float)(mean[windows ? i : 0] + k * stdev[windows ? i : 0]);
+    for (int z = 0; z < nz; z++) sig[z] = (float)(mean[(size_t)z] + k * stdev[(size_t)z]);
     return INLM_OK;
 }
 }  // namespace inlm

@@ -19,6 +19,7 @@
 // result is bit-identical to the reference CPU path.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "inlm_kernels.hpp"
@@ -833,40 +834,70 @@ __global__ __launch_bounds__(NT) void patchstd_kernel(const float *__restrict__ 
 // ---------------------------------------------------------------------------
 // Two-cluster hard EM (Noise/noiselevel.cpp:366-528) in FP64, one workgroup
 // per window of the sample list: the steps of create2clusters, the sums in a
-// fixed order over 1024 threads.  A sweep over a window reads its values from
-// the L2; nothing else is kept per value: the assignments of a sweep follow
-// from the parameters they were made with, so the test for a change evaluates
-// the previous parameters again and the variances the current ones.
+// fixed order over 1024 threads.  An assignment is one sweep over the window
+// (values from the L2), the variances about the new means another; the
+// assignment is kept as one bit per value in LDS, for the second sweep and for
+// the next one's test for a change (a window beyond kClusterWords * 64 values
+// derives it again from the parameters it was made with).
 //
-// p2 > p1 is decided from the difference of the logarithms, without the two
-// exponentials and square roots, wherever the rounding of that difference
-// (bounded below) cannot reach its sign and at least one density is far from
-// underflow; the densities themselves decide the rest.  On the host one
-// thread took 35 ms for a window of 1e5 samples and 1.1 s for the 2 x 256
-// windows of a 256^3 volume with 2e4 samples; here that is 1.9 ms and
-// 2 x 0.4 ms.
+// p2 > p1 is decided from the difference of the logarithms, a quadratic in the
+// value, wherever rounding (bounded for the whole interval in which the wider
+// density is far from underflow) cannot reach its sign; the densities
+// themselves decide the rest.  FP64 issue on the window's one CU bounds it.  On
+// the host one thread took 35 ms for a window of 1e5 samples and 1.1 s for the
+// 2 x 256 windows of a 256^3 volume with 2e4 samples; here that is 1.4 ms (0.5
+// when spread, below) and 2 x 0.3 ms.
 // ---------------------------------------------------------------------------
 constexpr int NTC = 1024;
+constexpr int kClusterRun = 4;          // 64-value words of a wavefront in flight
+constexpr int kClusterWords = 1 << 14;  // at most this many words of bits (128 KB)
 
 struct ClusterParams {
-    double m1, m2;         // means
-    double h1, h2;         // 1 / (2 variance)
-    double k1, k2;         // logarithms of the densities' factors
-    double v1, v2;
-    bool first;            // the initial assignment: the nearer of m1, m2
-    bool plain;            // factors in a range where the logarithms decide
+    double m1, m2, v1, v2;  // means and variances
+    double a, b, c;         // log p2 - log p1 = (a x + b) x + c, x = v - m1
+    double lo, hi, margin;  // the quadratic's sign decides between lo and hi beyond the margin
+    bool first;             // the initial assignment: the nearer of m1, m2
 };
 
-// whether v belongs to the second cluster; ok: the cheap test decides it
-__device__ __forceinline__ bool second_cluster(const ClusterParams &c, double v, bool &ok)
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform(double v)
 {
-    if (c.first) return !(fabs(v - c.m1) < fabs(v - c.m2));
-    const double d1 = v - c.m1, d2 = v - c.m2;
-    const double e1 = d1 * d1 * c.h1, e2 = d2 * d2 * c.h2;
-    const double l = (c.k2 - e2) - (c.k1 - e1);
-    ok = ok && c.plain && fmin(e1, e2) < 600.0 && fabs(l) > 1e-9 + 1e-13 * (e1 + e2);
-    return l > 0.0;
+    const unsigned long b = __builtin_bit_cast(unsigned long, v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __builtin_bit_cast(double, (unsigned long)hi << 32 | lo);
 }
+__device__ __forceinline__ unsigned long uniform(unsigned long v)
+{
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (unsigned long)hi << 32 | lo;
+}
+
+__device__ __forceinline__ ClusterParams cluster_params(double m1, double m2, double v1, double v2)
+{
+    const double PI = 3.14159265358979323846;
+    const double h1 = 1.0 / (2 * v1), h2 = 1.0 / (2 * v2);
+    const double k1 = -0.5 * log(v1 * 2 * PI), k2 = -0.5 * log(v2 * 2 * PI), d = m2 - m1;
+    ClusterParams p;
+    p.m1 = m1;
+    p.m2 = m2;
+    p.v1 = v1;
+    p.v2 = v2;
+    p.first = false;
+    p.a = h1 - h2;
+    p.b = 2 * d * h2;
+    p.c = (k2 - k1) - d * d * h2;
+    // exponents up to 600 of the wider density; no interval where the factors
+    // leave the range in which a density of that exponent is a normal number
+    const double h = fmin(h1, h2), r = sqrt(600.0 / h), mid = h1 < h2 ? m1 : m2;
+    const bool plain = fabs(k1) < 50.0 && fabs(k2) < 50.0;
+    p.lo = plain ? mid - r : 1e308;
+    p.hi = plain ? mid + r : -1e308;
+    const double x = fmax(fabs(p.lo - m1), fabs(p.hi - m1));
+    p.margin = 1e-10 + 1e-12 * (fabs(p.a) * x * x + fabs(p.b) * x + fabs(p.c));
+    for (double *q : {&p.a, &p.b, &p.c, &p.lo, &p.hi, &p.margin}) *q = uniform(*q);
+    return p;
+}
+
 // not inlined: its divisions and exponentials would take the registers of the
 // sweeps around it
 __device__ __attribute__((noinline)) bool second_cluster_densities(double m1, double v1, double m2, double v2, double v)
@@ -876,34 +907,35 @@ __device__ __attribute__((noinline)) bool second_cluster_densities(double m1, do
     const double p2 = 1. / sqrt(v2 * 2 * PI) * exp(-((v - m2) * (v - m2) / (2 * v2)));
     return p2 > p1;
 }
-// the same for kClusterRun values: bit j for v[j]
-constexpr int kClusterRun = 4;
-__device__ __forceinline__ unsigned second_clusters(const ClusterParams &c, const double (&v)[kClusterRun])
+// whether each of kClusterRun values belongs to the second cluster
+__device__ __forceinline__ void second_cluster(const ClusterParams &c, const double (&v)[kClusterRun],
+                                               bool (&r)[kClusterRun])
 {
-    unsigned m = 0;
+    if (c.first) {
+#pragma unroll
+        for (int j = 0; j < kClusterRun; j++) r[j] = !(fabs(v[j] - c.m1) < fabs(v[j] - c.m2));
+        return;
+    }
     bool ok = true;
 #pragma unroll
-    for (int j = 0; j < kClusterRun; j++) m |= (second_cluster(c, v[j], ok) ? 1u : 0u) << j;
-    if (!ok) {  // rare
-        m = 0;
-#pragma unroll 1
-        for (int j = 0; j < kClusterRun; j++) {
-            const double x = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
-            m |= (second_cluster_densities(c.m1, c.v1, c.m2, c.v2, x) ? 1u : 0u) << j;
-        }
+    for (int j = 0; j < kClusterRun; j++) {
+        const double x = v[j] - c.m1;
+        const double l = __builtin_fma(__builtin_fma(c.a, x, c.b), x, c.c);
+        r[j] = l > 0.0;
+        ok = ok && (v[j] == 0.0 || (fabs(l) > c.margin && v[j] > c.lo && v[j] < c.hi));
     }
-    return m;
+    if (__builtin_amdgcn_ballot_w64(!ok) == 0) return;
+    unsigned m = 0;  // rare: one call in the code
+#pragma unroll 1
+    for (int j = 0; j < kClusterRun; j++) {
+        const double x = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
+        m |= (second_cluster_densities(c.m1, c.v1, c.m2, c.v2, x) ? 1u : 0u) << j;
+    }
+#pragma unroll
+    for (int j = 0; j < kClusterRun; j++) r[j] = (m >> j & 1) != 0;
 }
 
-// a value that is the same in every lane, in scalar registers
-__device__ __forceinline__ double uniform(double v)
-{
-    const unsigned long b = __builtin_bit_cast(unsigned long, v);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
-    return __builtin_bit_cast(double, (unsigned long)hi << 32 | lo);
-}
-
-// the sum of v over the block, the same value in every thread
+// op over the block, the same value in every thread
 template <class Op>
 __device__ __forceinline__ double block_total(double v, double *sh, Op op)
 {
@@ -917,12 +949,27 @@ __device__ __forceinline__ double block_total(double v, double *sh, Op op)
     return uniform(r);
 }
 
+// KEPT: the windows' bits fit LDS (n <= 64 kClusterWords)
+template <bool KEPT>
 __global__ __launch_bounds__(NTC) void cluster_kernel(const double *__restrict__ values, long n,
                                                       const int64_t *__restrict__ bounds, double *__restrict__ out)
 {
-    __shared__ double sh[5][NTC / 64];
+    extern __shared__ unsigned long bits[];  // the last assignment
+    __shared__ double sh[4][NTC / 64];
+    __shared__ unsigned long cnt[3][NTC / 64];
     const long fs = bounds ? bounds[2 * blockIdx.x] : 0, ls = bounds ? bounds[2 * blockIdx.x + 1] : n - 1;
+    const long nword = (ls - fs + 64) / 64;  // 64-value words of the window (ls >= fs - 1)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NW = NTC / 64;
     auto add = [](double a, double b) { return a + b; };
+    // this lane's value of a word; 0 (never counted) past the window
+    auto load = [&](long w, double (&v)[kClusterRun]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kClusterRun; j++) {
+            const long i = fs + (w + (long)j * NW) * 64 + lane;
+            v[j] = i <= ls ? values[i] : 0.0;
+        }
+    };
     double mn = 1e300, mx = -1e300;
     for (long i = fs + threadIdx.x; i <= ls; i += NTC) {
         const double v = values[i];
@@ -936,66 +983,83 @@ __global__ __launch_bounds__(NTC) void cluster_kernel(const double *__restrict__
     cur.m2 = uniform(mx - 0.25 * (mx - mn));
     cur.first = true;
     double m1 = cur.m1, m2 = cur.m2, v1 = 0.0, v2 = 0.0;
-    // this thread's next values; 0 (never counted) past the window
-    auto load = [&](long i, double (&v)[kClusterRun]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < kClusterRun; j++) v[j] = i + j * NTC <= ls ? values[i + j * NTC] : 0.0;
-    };
-    // one assignment: sums, means, then the variances about them
+    // one assignment: counts, sums and means, then the variances about them
     auto assign = [&](bool test) -> bool {
-        double c1 = 0, c2 = 0, s1 = 0, s2 = 0, diff = 0;
-        double v[kClusterRun];
-        for (long i = fs + threadIdx.x; i <= ls; i += kClusterRun * NTC) {
-            load(i, v);
-            const unsigned m = second_clusters(cur, v), was = test ? second_clusters(prev, v) : m;
+        double c1 = 0, c2 = 0;
+        unsigned long s1 = 0, s2 = 0, diff = 0;
+        for (long w = wave; w < nword; w += kClusterRun * NW) {
+            double v[kClusterRun];
+            bool r[kClusterRun], was[kClusterRun];
+            load(w, v);
+            second_cluster(cur, v, r);
+            if (!KEPT && test) second_cluster(prev, v, was);
 #pragma unroll
             for (int j = 0; j < kClusterRun; j++) {
-                const bool b = (m >> j & 1) != 0, in = v[j] != 0.0;
-                c1 += in && !b ? v[j] : 0.0;
-                s1 += in && !b ? 1.0 : 0.0;
-                c2 += in && b ? v[j] : 0.0;
-                s2 += in && b ? 1.0 : 0.0;
-                diff += in && ((m ^ was) >> j & 1) != 0 ? 1.0 : 0.0;
+                const long word = w + (long)j * NW;
+                const bool in = v[j] != 0.0, b = in && r[j], a = in && !r[j];
+                const unsigned long mb = __builtin_amdgcn_ballot_w64(b);
+                c1 += a ? v[j] : 0.0;
+                c2 += b ? v[j] : 0.0;
+                s1 += __builtin_popcountl(__builtin_amdgcn_ballot_w64(a));
+                s2 += __builtin_popcountl(mb);
+                if constexpr (KEPT) {
+                    if (word < nword) {
+                        if (test) diff |= uniform(bits[word]) ^ mb;
+                        if (lane == 0) bits[word] = mb;
+                    }
+                } else if (test) {
+                    diff |= __builtin_amdgcn_ballot_w64(in && r[j] != was[j]);
+                }
             }
         }
-        c1 = block_total(c1, sh[0], add);
-        s1 = block_total(s1, sh[1], add);
-        c2 = block_total(c2, sh[2], add);
-        s2 = block_total(s2, sh[3], add);
-        if (test) diff = block_total(diff, sh[4], add);
-        if (s1 > 0) m1 = uniform(c1 / s1);
-        if (s2 > 0) m2 = uniform(c2 / s2);
+        if (lane == 0) {
+            cnt[0][wave] = s1;
+            cnt[1][wave] = s2;
+            cnt[2][wave] = diff;
+        }
+        c1 = block_total(c1, sh[0], add);  // its barriers also publish cnt
+        c2 = block_total(c2, sh[1], add);
+        s1 = s2 = diff = 0;
+        for (int w = 0; w < NW; w++) {
+            s1 += cnt[0][w];
+            s2 += cnt[1][w];
+            diff |= cnt[2][w];
+        }
+        if (s1 > 0) m1 = uniform(c1 / (double)s1);
+        if (s2 > 0) m2 = uniform(c2 / (double)s2);
         double q1 = 0, q2 = 0;
-        for (long i = fs + threadIdx.x; i <= ls; i += kClusterRun * NTC) {
-            load(i, v);
-            const unsigned m = second_clusters(cur, v);
+        for (long w = wave; w < nword; w += kClusterRun * NW) {
+            double v[kClusterRun];
+            bool r[kClusterRun];
+            load(w, v);
+            if constexpr (KEPT) {
+#pragma unroll
+                for (int j = 0; j < kClusterRun; j++) {
+                    const long word = w + (long)j * NW;
+                    r[j] = word < nword && (bits[word] >> lane & 1) != 0;
+                }
+            } else {
+                second_cluster(cur, v, r);
+            }
 #pragma unroll
             for (int j = 0; j < kClusterRun; j++) {
-                const bool b = (m >> j & 1) != 0, in = v[j] != 0.0;
-                q1 += in && !b ? (v[j] - m1) * (v[j] - m1) : 0.0;
-                q2 += in && b ? (v[j] - m2) * (v[j] - m2) : 0.0;
+                const bool in = v[j] != 0.0;
+                const double d = v[j] - (r[j] ? m2 : m1);
+                const double d1 = in && !r[j] ? d : 0.0, d2 = in && r[j] ? d : 0.0;
+                q1 += d1 * d1;
+                q2 += d2 * d2;
             }
         }
-        v1 = uniform(block_total(q1, sh[0], add) / fmax(1.0, s1));
-        v2 = uniform(block_total(q2, sh[1], add) / fmax(1.0, s2));
-        return test ? diff > 0.0 : s1 > 0 || s2 > 0;
+        v1 = uniform(block_total(q1, sh[2], add) / fmax(1.0, (double)s1));
+        v2 = uniform(block_total(q2, sh[3], add) / fmax(1.0, (double)s2));
+        return test ? diff != 0 : s1 > 0 || s2 > 0;
     };
     double mean = 0.0, stdev = 0.0;
     if (assign(false)) {
         bool change = true;
         for (int iters = 1; change && v1 > 0 && v2 > 0; iters++) {
             prev = cur;
-            const double PI = 3.14159265358979323846;
-            cur.m1 = m1;
-            cur.m2 = m2;
-            cur.v1 = v1;
-            cur.v2 = v2;
-            cur.h1 = uniform(1.0 / (2 * v1));
-            cur.h2 = uniform(1.0 / (2 * v2));
-            cur.k1 = uniform(-0.5 * log(v1 * 2 * PI));
-            cur.k2 = uniform(-0.5 * log(v2 * 2 * PI));
-            cur.first = false;
-            cur.plain = fabs(cur.k1) < 50.0 && fabs(cur.k2) < 50.0;
+            cur = cluster_params(m1, m2, v1, v2);
             change = assign(true);
             if (iters == 1000) break;
         }
@@ -1007,6 +1071,180 @@ __global__ __launch_bounds__(NTC) void cluster_kernel(const double *__restrict__
         out[2 * blockIdx.x] = mean;
         out[2 * blockIdx.x + 1] = stdev;
     }
+}
+
+// One large window over many CUs: the same steps as two launches per
+// iteration, each block taking a share of the values and first adding the
+// partial sums that the launch before left (in block order, every block the
+// same), so nothing is exchanged within a launch.  Launches behind the last
+// iteration return at once.
+constexpr int kSpreadBlocks = 64;
+// From here on one window is spread.  One workgroup takes 0.13 ms for 4096
+// samples and 0.52 ms for 16384, in proportion; spread, 16384 take 0.66 ms,
+// 32768 take 0.51 ms and 1e5 0.53 ms (two launches an iteration, whatever the
+// samples), where one workgroup takes 1.4 ms.
+constexpr int64_t kSpreadSamples = 20480;
+constexpr int kSpreadBatch = 16;  // iterations between looks at the end (about 20 are common)
+constexpr int NTS = 256;
+struct ClusterWork {
+    ClusterParams params[2];          // of even and odd iterations
+    double mean[2];                   // after the last assignment
+    double minmax[kSpreadBlocks][2];
+    double sums[2][kSpreadBlocks][5]; // c1, c2, s1, s2, changed values; of even and odd iterations
+    double squares[kSpreadBlocks][2];
+    int done;
+};
+static_assert(sizeof(ClusterWork) <= kClusterWorkBytes, "the callers' workspace");
+
+// the sums of N columns of per-block partials
+template <int N>
+__device__ __forceinline__ void add_partials(const double (*p)[N], double (&t)[N])
+{
+#pragma unroll
+    for (int e = 0; e < N; e++) t[e] = 0.0;
+    for (int b = 0; b < kSpreadBlocks; b++)
+#pragma unroll
+        for (int e = 0; e < N; e++) t[e] += p[b][e];
+}
+// thread 0 gets the block's sums
+template <int N>
+__device__ __forceinline__ void block_sums(double (&v)[N])
+{
+    __shared__ double sh[N][NTS / 64];
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) v[e] += __shfl_xor(v[e], o, 64);
+        if ((threadIdx.x & 63) == 0) sh[e][threadIdx.x >> 6] = v[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < N; e++) v[e] = (sh[e][0] + sh[e][1]) + (sh[e][2] + sh[e][3]);
+}
+// this thread's next values of the block's share; 0 (never counted) past it
+__device__ __forceinline__ void load_share(const double *values, long i, long end, double (&v)[kClusterRun])
+{
+#pragma unroll
+    for (int j = 0; j < kClusterRun; j++) v[j] = i + j * NTS < end ? values[i + j * NTS] : 0.0;
+}
+
+__global__ __launch_bounds__(NTS) void spread_minmax_kernel(const double *__restrict__ values, long n, ClusterWork *w)
+{
+    __shared__ double sh[2][NTS / 64];
+    const long end = n * (blockIdx.x + 1) / kSpreadBlocks;
+    double mn = 1e300, mx = -1e300;
+    for (long i = n * blockIdx.x / kSpreadBlocks + threadIdx.x; i < end; i += NTS) {
+        const double v = values[i];
+        mn = v < mn ? v : mn;
+        mx = mx < v ? v : mx;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        const double a = __shfl_xor(mn, o, 64), b = __shfl_xor(mx, o, 64);
+        mn = a < mn ? a : mn;
+        mx = mx < b ? b : mx;
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = mn;
+        sh[1][threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < NTS / 64; k++) {
+        mn = sh[0][k] < mn ? sh[0][k] : mn;
+        mx = mx < sh[1][k] ? sh[1][k] : mx;
+    }
+    w->minmax[blockIdx.x][0] = mn;
+    w->minmax[blockIdx.x][1] = mx;
+    if (blockIdx.x == 0) w->done = 0;
+}
+
+__global__ __launch_bounds__(NTS) void spread_assign_kernel(const double *__restrict__ values, long n, ClusterWork *w,
+                                                            int it, double *__restrict__ out)
+{
+    if (w->done != 0) return;
+    ClusterParams cur{}, prev{};
+    if (it == 0) {
+        double mn = 1e300, mx = -1e300;
+        for (int b = 0; b < kSpreadBlocks; b++) {
+            mn = w->minmax[b][0] < mn ? w->minmax[b][0] : mn;
+            mx = mx < w->minmax[b][1] ? w->minmax[b][1] : mx;
+        }
+        cur.m1 = mn + 0.25 * (mx - mn);
+        cur.m2 = mx - 0.25 * (mx - mn);
+        cur.first = true;
+    } else {
+        double s[5], q[2];
+        add_partials(w->sums[(it - 1) & 1], s);
+        add_partials(w->squares, q);
+        const double m1 = w->mean[0], m2 = w->mean[1], v1 = q[0] / fmax(1.0, s[2]), v2 = q[1] / fmax(1.0, s[3]);
+        const bool any = it > 1 || s[2] > 0 || s[3] > 0, change = it == 1 || s[4] > 0;
+        if (!any || !change || !(v1 > 0) || !(v2 > 0) || it > 1000) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                const bool low = m1 <= m2 || v2 <= 0.0;
+                out[0] = any ? (low ? m1 : m2) : 0.0;
+                out[1] = any ? sqrt(low ? v1 : v2) : 0.0;
+                w->done = 1;
+            }
+            return;
+        }
+        prev = w->params[(it - 1) & 1];
+        cur = cluster_params(m1, m2, v1, v2);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) w->params[it & 1] = cur;
+    const long end = n * (blockIdx.x + 1) / kSpreadBlocks;
+    double s[5] = {0, 0, 0, 0, 0};
+    for (long i = n * blockIdx.x / kSpreadBlocks + threadIdx.x; i - (long)threadIdx.x < end; i += kClusterRun * NTS) {
+        double v[kClusterRun];
+        bool r[kClusterRun], was[kClusterRun];
+        load_share(values, i, end, v);
+        second_cluster(cur, v, r);
+        if (it > 0) second_cluster(prev, v, was);
+#pragma unroll
+        for (int j = 0; j < kClusterRun; j++) {
+            const bool in = v[j] != 0.0;
+            s[0] += in && !r[j] ? v[j] : 0.0;
+            s[1] += in && r[j] ? v[j] : 0.0;
+            s[2] += in && !r[j] ? 1.0 : 0.0;
+            s[3] += in && r[j] ? 1.0 : 0.0;
+            s[4] += it > 0 && in && r[j] != was[j] ? 1.0 : 0.0;
+        }
+    }
+    block_sums(s);
+    if (threadIdx.x == 0)
+        for (int e = 0; e < 5; e++) w->sums[it & 1][blockIdx.x][e] = s[e];
+}
+
+__global__ __launch_bounds__(NTS) void spread_squares_kernel(const double *__restrict__ values, long n, ClusterWork *w,
+                                                             int it)
+{
+    if (w->done != 0) return;
+    const ClusterParams cur = w->params[it & 1];
+    double s[5];
+    add_partials(w->sums[it & 1], s);
+    const double m1 = s[2] > 0 ? s[0] / s[2] : cur.m1, m2 = s[3] > 0 ? s[1] / s[3] : cur.m2;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        w->mean[0] = m1;
+        w->mean[1] = m2;
+    }
+    const long end = n * (blockIdx.x + 1) / kSpreadBlocks;
+    double q[2] = {0, 0};
+    for (long i = n * blockIdx.x / kSpreadBlocks + threadIdx.x; i - (long)threadIdx.x < end; i += kClusterRun * NTS) {
+        double v[kClusterRun];
+        bool r[kClusterRun];
+        load_share(values, i, end, v);
+        second_cluster(cur, v, r);
+#pragma unroll
+        for (int j = 0; j < kClusterRun; j++) {
+            const bool in = v[j] != 0.0;
+            const double d1 = in && !r[j] ? v[j] - m1 : 0.0, d2 = in && r[j] ? v[j] - m2 : 0.0;
+            q[0] += d1 * d1;
+            q[1] += d2 * d2;
+        }
+    }
+    block_sums(q);
+    if (threadIdx.x == 0)
+        for (int e = 0; e < 2; e++) w->squares[blockIdx.x][e] = q[e];
 }
 
 // Every negative float from -0 down to the cutoff, as bit patterns
@@ -1236,11 +1474,38 @@ hipError_t launch_patchstd(const float *origin, int64_t row_pitch, int64_t slice
     return hipGetLastError();
 }
 
-hipError_t launch_clusters(const double *values, int64_t n, const int64_t *bounds, int nwin, double *out,
+hipError_t launch_clusters(const double *values, int64_t n, const int64_t *bounds, int nwin, double *out, void *work,
                            hipStream_t st)
 {
     if (nwin < 1 || n < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(cluster_kernel, dim3((unsigned)nwin), dim3(NTC), 0, st, values, (long)n, bounds, out);
+    if (nwin == 1 && !bounds && work && n >= kSpreadSamples) {
+        ClusterWork *w = static_cast<ClusterWork *>(work);
+        hipLaunchKernelGGL(spread_minmax_kernel, dim3(kSpreadBlocks), dim3(NTS), 0, st, values, (long)n, w);
+        for (int it = 0, done = 0; done == 0 && it <= 1001;) {
+            // a batch of iterations, then a look whether the last has come
+            for (const int end = std::min(it + kSpreadBatch, 1002); it < end; it++) {
+                hipLaunchKernelGGL(spread_assign_kernel, dim3(kSpreadBlocks), dim3(NTS), 0, st, values, (long)n, w, it,
+                                   out);
+                hipLaunchKernelGGL(spread_squares_kernel, dim3(kSpreadBlocks), dim3(NTS), 0, st, values, (long)n, w, it);
+            }
+            hipError_t e = hipGetLastError();
+            if (e == hipSuccess) e = hipMemcpyAsync(&done, &w->done, sizeof(int), hipMemcpyDeviceToHost, st);
+            const hipError_t f = hipStreamSynchronize(st);  // also before `done` goes
+            if (e != hipSuccess || f != hipSuccess) return e != hipSuccess ? e : f;
+        }
+        return hipSuccess;
+    }
+    if (n > 64L * kClusterWords) {
+        hipLaunchKernelGGL(cluster_kernel<false>, dim3((unsigned)nwin), dim3(NTC), 0, st, values, (long)n, bounds, out);
+        return hipGetLastError();
+    }
+    // beyond 64 KB of LDS a kernel has to ask for it
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(cluster_kernel<true>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             kClusterWords * (int)sizeof(unsigned long));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(cluster_kernel<true>, dim3((unsigned)nwin), dim3(NTC),
+                       (size_t)((n + 63) / 64) * sizeof(unsigned long), st, values, (long)n, bounds, out);
     return hipGetLastError();
 }
 

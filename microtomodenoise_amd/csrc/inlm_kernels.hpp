@@ -73,8 +73,10 @@ hipError_t launch_patchstd(const float *origin, int64_t row_pitch, int64_t slice
 // Two-cluster hard EM (create2clusters) of values[bounds[2 i] .. bounds[2 i + 1]]
 // for each of nwin windows: out[2 i] the mean and out[2 i + 1] the standard
 // deviation of the lower cluster.  Device pointers; bounds may be null for one
-// window over all n values.
-hipError_t launch_clusters(const double *values, int64_t n, const int64_t *bounds, int nwin, double *out,
+// window over all n values, which then, with kClusterWorkBytes at work and
+// enough values, is spread over the chip (the call then waits for the stream).
+constexpr size_t kClusterWorkBytes = 16384;
+hipError_t launch_clusters(const double *values, int64_t n, const int64_t *bounds, int nwin, double *out, void *work,
                            hipStream_t st);
 
 // Matrix-core forms (FP32_FAST, FP16, BF16).  Rs/Ps are normalised padded

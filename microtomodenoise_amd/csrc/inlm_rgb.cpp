@@ -166,7 +166,7 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
         if (cluster) {
             int64_t *bounds_dev = static_cast<int64_t *>(bC.p);
             double *out_dev = reinterpret_cast<double *>(bounds_dev + 6), got[6];
-            RGB_HIP(launch_clusters(sd_dev, 3 * ns, bounds_dev, 3, out_dev, st));
+            RGB_HIP(launch_clusters(sd_dev, 3 * ns, bounds_dev, 3, out_dev, nullptr, st));
             RGB_HIP(hipMemcpyAsync(got, out_dev, sizeof(got), hipMemcpyDeviceToHost, st));
             RGB_HIP(hipStreamSynchronize(st));
             for (int ch = 0; ch < 3; ch++) sig[ch] = (float)(got[2 * ch] + (double)p.stds_from_mean * got[2 * ch + 1]);

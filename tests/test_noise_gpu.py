@@ -73,7 +73,7 @@ def _noise_volume(kind):
     return np.ascontiguousarray(v)
 
 
-@pytest.mark.parametrize("n", [1, 2, 1023, 1024, 1025, 4096, 4097, 20011])
+@pytest.mark.parametrize("n", [1, 2, 1023, 1024, 1025, 4097, 16384, 20479, 20480, 20737])
 @pytest.mark.parametrize("kind", ["plain", "flat", "half-flat", "two-level", "outlier", "tiny"])
 def test_clustering_on_the_gpu_equals_the_host(gpu_available, kind, n):
     """Both run the same steps in FP64 and differ by the order of at most
@@ -96,3 +96,24 @@ def test_clustering_on_the_gpu_equals_the_host(gpu_available, kind, n):
         g.free_device()
         want = _capi.sigma_from_patchstd(p.to_c(), [nx, ny, nz], samples, stds)
         assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
+
+
+def test_clustering_beyond_the_bits_in_lds(gpu_available):
+    """More samples than the 2^20 whose assignments LDS keeps; the sums of
+    1.1e6 terms differ by 1e-10 relative at most."""
+    raw = _noise_volume("two-level")
+    nz, ny, nx = raw.shape
+    n = 1_100_003
+    samples = _capi.draw_samples([nx, ny, nz], n, 15, 5)
+    p = DenoiseParameters(radius_searchspace=[2, 2, 2], radius_patchspace=[1, 1, 1])
+    p.noiselevel.mode = "global"
+    p.noiselevel.n_samples = n
+    print(f"[gpu] clustering n={n}", flush=True)
+    g = IterativeNLM_GPU()
+    assert g.configure_device([nx, ny, nz], p) == nz
+    g.load_raw(raw)
+    stds = g.patchstd(samples)
+    got = g.estimate_noise(samples)
+    g.free_device()
+    want = _capi.sigma_from_patchstd(p.to_c(), [nx, ny, nz], samples, stds)
+    assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
