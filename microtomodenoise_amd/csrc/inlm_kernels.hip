@@ -795,6 +795,20 @@ __global__ __launch_bounds__(NT) void pad_reflect_kernel(const float *__restrict
 }
 
 // ---------------------------------------------------------------------------
+// Anscombe transform of the colour path and its algebraic inverse
+// (Color/colorspace.h:87-123): the same float operations as anscombe() and
+// inverse_anscombe() on the host, which took 5 of the 15 ms of a 1200x900
+// image's call.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(NT) void anscombe_kernel(float *__restrict__ v, long n, int inverse)
+{
+    const long i = (long)blockIdx.x * NT + threadIdx.x;
+    if (i >= n) return;
+    const float x = v[i];
+    v[i] = inverse ? (x / 2.f) * (x / 2.f) - 3.f / 8.f : 2.f * sqrtf(x + 3.f / 8.f);
+}
+
+// ---------------------------------------------------------------------------
 // Noise: one wavefront per sample computes the population standard deviation
 // of its patchsize x patchsize in-slice patch (noiselevel.cpp:235-283) with
 // FP64 two-pass accumulation and a wavefront butterfly reduction.
@@ -1339,6 +1353,12 @@ hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, 
     const long n = (long)g.nxp * g.nyp * g.nzp;
     const unsigned blocks = (unsigned)((n + NT - 1) / NT);
     hipLaunchKernelGGL(pad_reflect_kernel, dim3(blocks), dim3(NT), 0, st, in, out, g);
+    return hipGetLastError();
+}
+
+hipError_t launch_anscombe(float *v, long n, bool inverse, hipStream_t st)
+{
+    hipLaunchKernelGGL(anscombe_kernel, dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, st, v, n, inverse ? 1 : 0);
     return hipGetLastError();
 }
 

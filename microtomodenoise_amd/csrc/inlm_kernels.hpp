@@ -35,6 +35,9 @@ struct TapTable {
 // (mirror without repeating the edge, iternlm_prepare.cpp:6-48).
 hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, hipStream_t st);
 
+// Anscombe transform in place, or its inverse.
+hipError_t launch_anscombe(float *v, long n, bool inverse, hipStream_t st);
+
 // One filter pass.  R/P are padded volumes; out is unpadded; sigma has nz
 // entries.  shape is the patch shape of a tiled kernel (tiled_shape), or 0 for
 // the per-voxel kernel, which runs any tap table.  With mass != nullptr the

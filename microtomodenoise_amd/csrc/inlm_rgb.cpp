@@ -127,10 +127,8 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
     float *Ud = static_cast<float *>(bU.p);
     RGB_HIP(hipMemcpyAsync(bS.p, se.data(), se.size() * sizeof(SearchEntry), hipMemcpyHostToDevice, st));
 
-    // the channels, Anscombe-transformed on the host as the reference does
-    std::vector<float> host(in, in + 3 * npix);
-    if (c->stabilize_variance) anscombe(host.data(), host.size());
-    RGB_HIP(hipMemcpyAsync(Ud, host.data(), 3 * npix * sizeof(float), hipMemcpyHostToDevice, st));
+    RGB_HIP(hipMemcpyAsync(Ud, in, 3 * npix * sizeof(float), hipMemcpyHostToDevice, st));
+    if (c->stabilize_variance) RGB_HIP(launch_anscombe(Ud, (long)(3 * npix), false, st));
     for (int ch = 0; ch < 3; ch++) RGB_HIP(launch_pad_reflect(Ud + ch * npix, Rd + ch * padn, g, st));
 
     // noise level per channel (noiselevel.cpp:96-184): one sample list for
@@ -188,7 +186,7 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
     float s0[3], s1[3];
     inlm_status s = estimate(Ud, 0, s0);
     if (s != INLM_OK) return s;
-    std::vector<float> res(3 * npix);
+    std::vector<float> res(on_iteration ? 3 * npix : 0);
     for (int iter = 1; iter <= p.maxiterations; iter++) {
         const float *R3[3] = {Rd, Rd + padn, Rd + 2 * padn};
         const float *P3[3];
@@ -220,10 +218,9 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
             for (int ch = 0; ch < 3; ch++) s0[ch] = p.alpha * s0[ch] + (1.f - p.alpha) * s1[ch];
         }
     }
-    RGB_HIP(hipMemcpyAsync(res.data(), Od, 3 * npix * sizeof(float), hipMemcpyDeviceToHost, st));
+    if (c->stabilize_variance) RGB_HIP(launch_anscombe(Od, (long)(3 * npix), true, st));
+    RGB_HIP(hipMemcpyAsync(out, Od, 3 * npix * sizeof(float), hipMemcpyDeviceToHost, st));
     RGB_HIP(hipStreamSynchronize(st));
-    if (c->stabilize_variance) inverse_anscombe(res.data(), res.size());
-    std::memcpy(out, res.data(), 3 * npix * sizeof(float));
     return INLM_OK;
 #undef RGB_HIP
 }
