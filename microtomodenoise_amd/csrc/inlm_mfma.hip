@@ -17,11 +17,11 @@
 // every weight unchanged once the per-slice multiplier is divided by scale^2.
 //
 // This row form (filter_mfma: every patch radius, the FP8-plane and FP32_FAST
-// forms, the pruned per-tile lists): a workgroup (8 wavefronts) owns a
+// forms, full search and per-tile lists): a workgroup (8 wavefronts) owns a
 // 32x8x8 output tile and stages D_s over the tile plus the patch halo in LDS
 // (double buffered, one barrier per offset); wavefront w computes the 16x16
-// block x-half (w & 1), z pair (w >> 1).  The full search at patch radius 2
-// in the 16-bit forms runs the block form (filter_mfma_b4, further below).
+// block x-half (w & 1), z pair (w >> 1).  At patch radius 2 the 16-bit forms
+// run the block form (filter_mfma_b4, further below).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1327,32 +1327,60 @@ void filter_mfma(MfmaArgs<TS> a)
 #ifndef INLM_B4_KD
 #define INLM_B4_KD 2
 #endif
-namespace b4 {
-constexpr int TX = 32, TY = 16, TZ = 8;
-constexpr int NH = TY / 8;  // 32x8 output halves per wavefront
-constexpr int RX = TX + 4, RY = TY + 4, RZ = TZ + 4;  // staged region
-constexpr int ROW = 64;                               // LDS row pitch, halves (8 windows)
-constexpr int SLICE = RY * ROW + 8;                   // LDS slice pitch, halves (97 16-byte units)
-constexpr int LDS = RZ * SLICE;                       // halves per buffer
-constexpr int NSLOT = (RY / 4) * (RZ / 4);
-static_assert(RX == 36 && RY % 4 == 0 && RZ % 4 == 0 && NSLOT > 8 && NSLOT <= 16, "staging slots");
-constexpr int NOPS = 7, NCLS = 5;
-// plane and row of the K group q of MFMA o; o = 4 holds rows 3, 4 of
-// plane +1 (q < 2) and of plane -1 (q >= 2)
-__host__ __device__ constexpr int op_dz(int o, int q)
+template <int TY_>
+struct B4 {
+    static constexpr int TX = 32, TY = TY_, TZ = 8;
+    static constexpr int NH = TY / 8;  // 32x8 output halves per wavefront
+    static constexpr int RX = TX + 4, RY = TY + 4, RZ = TZ + 4;  // staged region
+    static constexpr int ROW = 64;                               // LDS row pitch, halves (8 windows)
+    static constexpr int SLICE = RY * ROW + 8;                   // LDS slice pitch, halves (1 mod 16 16-byte units)
+    static constexpr int LDS = RZ * SLICE;                       // halves per buffer
+    static constexpr int NSLOT = (RY / 4) * (RZ / 4);
+    static_assert(RX == 36 && RY % 4 == 0 && RZ % 4 == 0 && NSLOT > 8 && NSLOT <= 16, "staging slots");
+    static_assert(SLICE / 8 % 16 == 1, "slices one 16-byte unit apart in the banks");
+    static constexpr int NOPS = 7, NCLS = 5;
+    // plane and row of the K group q of MFMA o; o = 4 holds rows 3, 4 of
+    // plane +1 (q < 2) and of plane -1 (q >= 2)
+    __host__ __device__ static constexpr int op_dz(int o, int q)
+    {
+        return o <= 1 ? 0 : o == 2 ? 1 : o == 3 ? -1 : o == 4 ? (q < 2 ? 1 : -1) : o == 5 ? 2 : -2;
+    }
+    __host__ __device__ static constexpr int op_row(int o, int q)
+    {
+        return o == 0 ? q - 2 : o == 1 ? q + 2 : o <= 3 ? q - 1 : o == 4 ? (q < 2 ? q + 3 : q + 1) : q;
+    }
+    // operations with equal weights share an A operand (the weights depend on |dz|)
+    static constexpr int kCls[NOPS] = {0, 1, 2, 2, 3, 4, 4};
+    static constexpr int kClsOp[NCLS] = {0, 1, 2, 4, 5};
+    // LDS offset of MFMA o relative to a lane's row of K group 0 (uniform except o = 4)
+    static constexpr int kOff[NOPS] = {-2 * ROW, 2 * ROW, SLICE - ROW, -SLICE - ROW, 0, 2 * SLICE, -2 * SLICE};
+};
+
+// The patch weights by (|dz|, |dy|, dx + 2) for the lists' form, whose tiles run
+// few steps: its lanes read them from LDS, where the argument block is read
+// through the vector cache, one wait per weight.  (In the full search's form
+// the table costs a register in the loop, 4% of the pass.)
+__device__ __forceinline__ void b4_weight_table(const float (&band)[kMfmaMaxPatterns][8], float *tab)
 {
-    return o <= 1 ? 0 : o == 2 ? 1 : o == 3 ? -1 : o == 4 ? (q < 2 ? 1 : -1) : o == 5 ? 2 : -2;
+    constexpr const MRows<2> &rows = MRowsOf<2>::value;
+    const int t = threadIdx.x;
+    if (t < 45) {
+        const int adz = t / 15, ady = t / 5 % 3, dx = t % 5 - 2;
+        int at = -1;
+#pragma unroll
+        for (int p = 0; p < rows.npat; p++)
+            if (rows.pdy[p] == ady && rows.pdz[p] == adz && dx >= -rows.pj[p] && dx <= rows.pj[p]) at = p * 8 + dx + 2;
+        const float w = (&band[0][0])[at >= 0 ? at : 0];
+        tab[t] = at >= 0 ? w : 0.f;
+    }
 }
-__host__ __device__ constexpr int op_row(int o, int q)
+__device__ __forceinline__ float b4_table_weight(const float *tab, int dx, int dy, int dz)
 {
-    return o == 0 ? q - 2 : o == 1 ? q + 2 : o <= 3 ? q - 1 : o == 4 ? (q < 2 ? q + 3 : q + 1) : q;
+    const int ady = dy < 0 ? -dy : dy, adz = dz < 0 ? -dz : dz;
+    const bool in = dx >= -2 && dx <= 2 && ady <= 2;
+    const float w = tab[in ? adz * 15 + ady * 5 + dx + 2 : 0];
+    return in ? w : 0.f;
 }
-// operations with equal weights share an A operand (the weights depend on |dz|)
-constexpr int kCls[NOPS] = {0, 1, 2, 2, 3, 4, 4};
-constexpr int kClsOp[NCLS] = {0, 1, 2, 4, 5};
-// LDS offset of MFMA o relative to a lane's row of K group 0 (uniform except o = 4)
-constexpr int kOff[NOPS] = {-2 * ROW, 2 * ROW, SLICE - ROW, -SLICE - ROW, 0, 2 * SLICE, -2 * SLICE};
-}  // namespace b4
 
 template <class TS>
 __device__ __forceinline__ float b4_weight(const MfmaArgs<TS> &a, int dx, int dy, int dz)
@@ -1366,15 +1394,20 @@ __device__ __forceinline__ float b4_weight(const MfmaArgs<TS> &a, int dx, int dy
     return w;
 }
 
-// Its loop holds up to 128 registers: two workgroups per CU (4 waves per SIMD)
-template <class TS>
-__global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) void filter_mfma_b4(MfmaArgs<TS> a)
+// The full search's loop holds up to 128 registers: two workgroups per CU (4
+// waves per SIMD); so does the lists' form (105 registers; at 6 waves per SIMD
+// it spills 17 to 30).
+template <class TS, bool PRUNED>
+__global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) void
+filter_mfma_b4(MfmaArgs<TS> a)
 {
+    using b4 = B4<PRUNED ? 8 : 16>;
     using ST8 = Stager<8, TS, _Float16>;
     using ST4 = Stager<4, TS, _Float16>;
     typedef typename ST8::chunk chunk8;
     typedef typename ST4::chunk chunk4;
     __shared__ __attribute__((aligned(16))) _Float16 lds[2][b4::LDS];
+    __shared__ float wtab[PRUNED ? 45 : 1];
 
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -1389,6 +1422,10 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const long sp = (long)g.nxp * g.nyp;
 
     for (int i = t; i < (int)(sizeof(lds) / 4); i += NTM) reinterpret_cast<unsigned *>(&lds[0][0])[i] = 0u;
+    if constexpr (PRUNED) {
+        b4_weight_table(a.band, wtab);
+        __syncthreads();
+    }
 
     // A operands: lane l holds row m = l % 16 (output bx = m & 3, by = m >> 2)
     // of K group q = l / 16
@@ -1401,7 +1438,10 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             const int o = b4::kClsOp[c];
             const int dz = b4::op_dz(o, q), row = b4::op_row(o, q);
 #pragma unroll
-            for (int i = 0; i < 8; i++) aop[c][i] = (_Float16)b4_weight(a, i - 2 - mx, row - my, dz);
+            for (int i = 0; i < 8; i++) {
+                if constexpr (PRUNED) aop[c][i] = (_Float16)b4_table_weight(wtab, i - 2 - mx, row - my, dz);
+                else aop[c][i] = (_Float16)b4_weight(a, i - 2 - mx, row - my, dz);
+            }
         }
     }
 
@@ -1505,7 +1545,7 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     // bytes past their 8-column chunk): columns 32-35, or 32-39 for slot A of
     // the FP16 form, which moves its chunks along runs of the search instead
     // of loading them at every offset (below)
-    constexpr bool kMove = std::is_same<TS, _Float16>::value;
+    constexpr bool kMove = std::is_same<TS, _Float16>::value && !PRUNED;
     chunk8 pnA, pnX;
     std::conditional_t<kMove, chunk8, chunk4> pqA = {};
     chunk4 pqX = {};
@@ -1626,11 +1666,29 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         }
     };
 
-    const int nS = a.n_search;
-    auto lin_at = [&](int k) __attribute__((always_inline)) { return a.search_full[k < nS ? k : nS - 1].lin; };
+    // offsets this tile visits: the whole search, or its list (32x8x8 tiles)
+    int nS = a.n_search;
+    const int *lst = nullptr;
+    if constexpr (PRUNED) {
+        const int c = a.counts[wg];
+        if (c >= 1 && c < nS) {
+            nS = c;
+            lst = a.lists + (long)wg * a.K;
+        }
+    }
+    auto lin_at = [&](int k) __attribute__((always_inline)) {
+        const int i = k < nS ? k : nS - 1;
+        if constexpr (PRUNED) {
+            if (lst) {
+                const unsigned e = (unsigned)lst[i];
+                return a.search[e < (unsigned)a.n_search ? e : 0u].lin;
+            }
+        }
+        return a.search_full[i].lin;
+    };
     // per offset of the full search, after the table: 0 to load slot A's
     // chunks, s > 0 to move those of the offset before it (kStageMovesMax)
-    const int *moves = reinterpret_cast<const int *>(a.search_full + nS);
+    const int *moves = reinterpret_cast<const int *>(a.search_full + a.n_search);
     auto loads_a = [&](int mv) __attribute__((always_inline)) { return !kMove || mv == 0; };
 
     // Software pipeline as in filter_mfma: step k runs the MFMA chain of
@@ -1640,7 +1698,7 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     __syncthreads();
     load_chunks(lin_at(0), true);
     stage(lds[0]);
-    load_chunks(lin_at(1), loads_a(nS > 1 ? moves[1] : 0));
+    load_chunks(lin_at(1), loads_a(kMove && nS > 1 ? moves[1] : 0));
     __syncthreads();
 
     DVals dA, dB;
@@ -2029,17 +2087,23 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
         if (iso) fp8_tables_plan<R, true>(codes, a);
         else fp8_tables_plan<R, false>(codes, a);
     }
-    // the block form: full search at patch radius 2, 16-bit storage, FP16
-    // planes, Pade weights; it packs lin * 4 + moves into one int, so |lin|
+    // the block form (lists of 128 offsets over 640x640x256: FP16 9.9 ms, BF16
+    // 10.8 ms; the row form 11.2 and 11.5): full search or lists at patch radius 2, 16-bit storage,
+    // FP16 planes, Pade weights; it packs lin * 4 + moves into one int, so |lin|
     // stays below 2^29 (the search space is symmetric: the largest lin is
     // -min_lin); beyond that the row form runs
     if constexpr (R == 2 && sizeof(TS) == 2 && std::is_same<TD, _Float16>::value && WFN == 0) {
-        if (!ol && !row_form && -(long)min_lin < (1L << 29)) {
-            a.ntx = (g.nx + b4::TX - 1) / b4::TX;
-            a.nty = (g.ny + b4::TY - 1) / b4::TY;
-            a.ntz = (g.nz + b4::TZ - 1) / b4::TZ;
+        if (!row_form && -(long)min_lin < (1L << 29)) {
+            if (ol) {  // one 32x8x8 tile, the lists' own, per workgroup
+                hipLaunchKernelGGL((filter_mfma_b4<TS, true>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
+                return hipGetLastError();
+            }
+            using B = B4<16>;
+            a.ntx = (g.nx + B::TX - 1) / B::TX;
+            a.nty = (g.ny + B::TY - 1) / B::TY;
+            a.ntz = (g.nz + B::TZ - 1) / B::TZ;
             const long nb = (long)a.ntx * a.nty * a.ntz;
-            hipLaunchKernelGGL((filter_mfma_b4<TS>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
+            hipLaunchKernelGGL((filter_mfma_b4<TS, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
             return hipGetLastError();
         }
     }

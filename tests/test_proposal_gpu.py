@@ -225,6 +225,42 @@ def test_pruned_lists_match_oracle_per_tile(gpu_available, form):
     assert sep > 10 * rms
 
 
+@pytest.mark.parametrize("form", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(33, 9, 9), (64, 24, 16), (95, 31, 7)])
+def test_lists_on_the_block_kernel_equal_the_row_kernel(gpu_available, form, shape):
+    """Patch radius 2: both kernels sum the same FP16 squares of the same
+    offsets, in another FP32 order (the budget of their full-search
+    comparison); tiles of one offset, odd and even counts, more than the 62
+    steps of a table block, and whole searches."""
+    nx, ny, nz = shape
+    spec = ph.PhantomSpec(shape, seed=nx, radii=(2, 7), noise_sigma=1500.0, blur_sigma=0.8)
+    raw = ph.make(spec)
+    sig = np.linspace(600.0, 900.0, nz).astype(np.float32)
+    rs = (4, 4, 3)
+    ns = len(O.search_offsets(rs))
+    K = 80
+    nt = ((nx + 31) // 32) * ((ny + 7) // 8) * ((nz + 7) // 8)
+    rng = np.random.default_rng(nx)
+    lists = np.stack([np.sort(rng.permutation(ns)[:K]) for _ in range(nt)]).astype(np.int32)
+    counts = np.resize(np.array([1, 2, 61, ns, 62, 63, 80], np.int32), nt)
+    outs = []
+    for ks in (0, 2):
+        print(f"[gpu] lists {form} {shape} kernel_select {ks}", flush=True)
+        p = DenoiseParameters(radius_searchspace=list(rs), radius_patchspace=[2, 2, 2], precision=form, kernel_select=ks)
+        g = IterativeNLM_GPU()
+        assert g.configure_device(list(shape), p) == nz
+        g.load_raw(raw)
+        g.set_sigma(sig)
+        g.set_offset_lists(lists, counts, K)
+        g.Run_GaussianNoise(1)
+        outs.append(g.get_result().astype(np.float64))
+        g.free_device()
+    err = np.abs(outs[0] - outs[1]) / spec.noise_sigma
+    mx, rms = float(err.max()), float(np.sqrt(np.mean(err ** 2)))
+    print(f"[gpu]   block vs row: max {mx:.3e} rms {rms:.3e}", flush=True)
+    assert mx < 0.02 and rms < 2e-4, (mx, rms)
+
+
 @pytest.mark.parametrize("form", ["fp16", "fp16_fp8"])
 def test_proposal_fallback_audit_and_topk(gpu_available, form):
     spec = ph.PhantomSpec((64, 32, 24), seed=81, radii=(2, 7), streaks=3, streak_len=(5, 15))
