@@ -1307,10 +1307,9 @@ void filter_mfma(MfmaArgs<TS> a)
 //
 // Staging: 15 slots of 64 lanes each cover a 4x4 block of region rows
 // (ry in 4 (s % 5) .. +3, rz in 4 (s / 5) .. +3); lane 4 j + c computes the D
-// values of columns 8c .. 8c+7 of row (ry0 + j / 4, rz0 + j % 4), and lanes
-// with c = 3 also of columns 32-35.  It writes window 2c (its own 8 columns)
-// and window 2c+1 (its upper four and the next lane's lower four, moved by
-// DPP; columns 32-35 for c = 3).  The two rows of 8 consecutive lanes
+// values of columns 8c .. 8c+11 of row (ry0 + j / 4, rz0 + j % 4).  It writes
+// window 2c (the first eight) and window 2c+1 (the last eight).  The two rows
+// of 8 consecutive lanes
 // (j = 2i, 2i+1) are one slice apart, an odd number of 16-byte units, so
 // their chunks interleave in the banks; an earlier mapping with the two rows
 // two slices apart wrote with 2-way conflicts (2% slower).  Wave w runs
@@ -1319,8 +1318,8 @@ void filter_mfma(MfmaArgs<TS> a)
 //
 // Run moves (FP16 form): slot w's chunks are loaded only at every third
 // offset of a run of the full search (one dz and dy, dx stepping by 2) and
-// moved one dword along the row in between (the cg = 3 lanes load columns
-// 32-39 for that), which skips about half of slot w's loads at search
+// moved one dword along the row in between (each lane loads 16 columns for
+// that), which skips about half of slot w's loads at search
 // radius 7: 3-4% faster.  Moving the second slot as well, or moving in the
 // BF16 form, puts a spill reload into the loop and was slower (3% and 7%).
 // ---------------------------------------------------------------------------
@@ -1542,10 +1541,14 @@ filter_mfma_b4(MfmaArgs<TS> a)
     auto soff_of = [&](int lin) __attribute__((always_inline)) {
         return (unsigned)((lin - min_lin) * (int)sizeof(TS));
     };
-    // per slot: 8 columns, and the row's tail on lanes with cg = 3 (at 16
-    // bytes past their 8-column chunk): columns 32-35, or 32-39 for slot A of
-    // the FP16 form, which moves its chunks along runs of the search instead
-    // of loading them at every offset (below)
+    // per slot: 8 columns and the tail behind them, the next four, or the next
+    // eight for slot A of the FP16 form, which moves its chunks along runs of
+    // the search instead of loading them at every offset (below).  Only the
+    // row's last lane (cg = 3) needs columns no other lane holds, but with a
+    // tail of its own in every lane neither the staging nor a move exchanges
+    // lanes or branches, in as many vector instructions (the masked ones took
+    // a slot too): lists of 128 offsets, BF16, 640x640x256: 12.1 -> 11.9 ms a
+    // call; the full search the same within 0.3%.
     constexpr bool kMove = std::is_same<TS, _Float16>::value && !PRUNED;
     chunk8 pnA, pnX;
     std::conditional_t<kMove, chunk8, chunk4> pqA = {};
@@ -1556,15 +1559,12 @@ filter_mfma_b4(MfmaArgs<TS> a)
         const unsigned oA = (unsigned)(coffA * (int)sizeof(TS)), oX = (unsigned)(coffX * (int)sizeof(TS));
         if (slot_a) {
             stg8.load(pnA, r, oA, so);
-            if constexpr (kMove) {
-                if (cg == 3) stg8.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
-            } else {
-                if (cg == 3) stg4.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
-            }
+            if constexpr (kMove) stg8.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
+            else stg4.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
         }
         if (two) {
             stg8.load(pnX, r, oX, so);
-            if (cg == 3) stg4.load(pqX, r, oX + 8 * (unsigned)sizeof(TS), so);
+            stg4.load(pqX, r, oX + 8 * (unsigned)sizeof(TS), so);
         }
     };
     // the chunks at the tile's own positions (the P(y) side of every
@@ -1585,24 +1585,17 @@ filter_mfma_b4(MfmaArgs<TS> a)
     auto st16 = [](_Float16 *dst, const half2v *v) __attribute__((always_inline)) {
         __builtin_memcpy(__builtin_assume_aligned(dst, 16), v, 16);
     };
-    // window 2 cg (own 8 columns) and window 2 cg + 1 (upper four, then the
-    // next lane's lower four by DPP row shift, or columns 32-35 for cg = 3)
+    // window 2 cg (own 8 columns) and window 2 cg + 1 (the upper four, then
+    // the tail's first four)
     auto store_slot = [&](_Float16 *buf, const chunk8 &pn, const chunk8 &p0, const chunk4 &pq, const chunk4 &q0,
                           int lrow) __attribute__((always_inline)) {
-        half2v d[4], e[4];
+        half2v d[4], e[4], d4[2];
         stg8.scaled(pn, p0, d);
+        stg4.scaled(pq, q0, d4);
         e[0] = d[2];
         e[1] = d[3];
-#pragma unroll
-        for (int h = 0; h < 2; h++)  // row_shl:1, lane i reads lane i + 1 of its 16-lane row
-            e[2 + h] = __builtin_bit_cast(half2v, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, d[h]), 0x101, 0xf, 0xf,
-                                                                            true));
-        if (cg == 3) {
-            half2v d4[2];
-            stg4.scaled(pq, q0, d4);
-            e[2] = d4[0];
-            e[3] = d4[1];
-        }
+        e[2] = d4[0];
+        e[3] = d4[1];
         st16(buf + lrow, d);
         st16(buf + lrow + 8, e);
     };
@@ -1614,19 +1607,18 @@ filter_mfma_b4(MfmaArgs<TS> a)
     };
     // Slot A's chunks of an offset from those of the offset before it when
     // the two differ by dx + 2 (same dz and dy): each region row moves by one
-    // dword, so dwords 1-3 move down and the last comes from the next lane of
-    // the row (DPP row shift) or, for cg = 3, from the tail, which holds
-    // columns 32-39 of the loaded offset and so serves two such moves.
+    // dword, so dwords 1-3 move down and the last comes from the tail, which
+    // holds the next eight columns of the loaded offset and so serves two
+    // such moves.
     auto move_a = [&]() __attribute__((always_inline)) {
         if constexpr (kMove) {
             unsigned w[4], tl[4];
             __builtin_memcpy(w, &pnA, 16);
             __builtin_memcpy(tl, &pqA, 16);
-            const unsigned from_next = (unsigned)__builtin_amdgcn_mov_dpp((int)w[0], 0x101, 0xf, 0xf, true);
             w[0] = w[1];
             w[1] = w[2];
             w[2] = w[3];
-            w[3] = cg == 3 ? tl[0] : from_next;
+            w[3] = tl[0];
             tl[0] = tl[1];
             tl[1] = tl[2];
             tl[2] = tl[3];
@@ -1752,6 +1744,14 @@ filter_mfma_b4(MfmaArgs<TS> a)
             if constexpr (r + KD < NR) ab[r % KD] = b_of(std::integral_constant<int, r + KD>{});
         });
         accumulate(din, rin);
+        // The sums are finished in the block that holds the MFMAs: left free,
+        // the compiler moves the weights behind the branches of the staging,
+        // where no MFMA runs beside them (FP16, 1326 offsets of 1024x1024x512:
+        // 425 -> 411 ms).
+#pragma unroll
+        for (int h = 0; h < b4::NH; h++)
+            asm volatile("" : "+v"(fv[h][0]), "+v"(fv[h][1]), "+v"(fv[h][2]), "+v"(fv[h][3]), "+v"(fw[h][0]),
+                         "+v"(fw[h][1]), "+v"(fw[h][2]), "+v"(fw[h][3]));
         if (!loads_a(m1)) move_a();
         stage(st);
         constexpr int NV = (2 * b4::NH * kWeightValuPacked + kStageValu<TS, _Float16> * 3 * 2 + NR - 2) / (NR - 1);
