@@ -117,7 +117,7 @@ constexpr int kMomentDoubles = 2 + 2 * kMomentBlocks;
 
 // The full-search order of the matrix-core forms is followed on the device by
 // n_search + kStageMovesPad ints, one per offset and zero past the last: 0
-// where the block kernel loads the staging chunks of a wavefront's own slot,
+// where the block kernel loads its staging chunks,
 // s = 1 .. kStageMovesMax where the offset is the one before it moved by
 // dx + 2 within one dz and dy (one dword per region row), s such moves after
 // the last load.

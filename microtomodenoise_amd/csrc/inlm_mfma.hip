@@ -597,14 +597,16 @@ struct Stager<W, _Float16, _Float16> {
 #pragma unroll
         for (int h = 0; h < W / 2; h++) b[h] = -(b[h] * f);
     }
-    __device__ __forceinline__ void scaled(const chunk &pn, const chunk &b, half2v (&out)[W / 2]) const
+    __device__ __forceinline__ half2v scaled_pair(half2v v, half2v b) const
     {
         const half2v zero = {(_Float16)0.f, (_Float16)0.f}, one = {(_Float16)1.f, (_Float16)1.f};
+        const half2v d = __builtin_elementwise_fma(v, f, b);
+        return __builtin_elementwise_min(__builtin_elementwise_max(d * d, zero), one);
+    }
+    __device__ __forceinline__ void scaled(const chunk &pn, const chunk &b, half2v (&out)[W / 2]) const
+    {
 #pragma unroll
-        for (int h = 0; h < W / 2; h++) {
-            const half2v d = __builtin_elementwise_fma(pn[h], f, b[h]);
-            out[h] = __builtin_elementwise_min(__builtin_elementwise_max(d * d, zero), one);
-        }
+        for (int h = 0; h < W / 2; h++) out[h] = scaled_pair(pn[h], b[h]);
     }
     __device__ __forceinline__ void store_scaled(const chunk &pn, const chunk &b, _Float16 *dst) const
     {
@@ -653,14 +655,16 @@ struct Stager<W, __bf16, _Float16> {
 #pragma unroll
         for (int h = 0; h < W / 2; h++) b[h] = __builtin_bit_cast(unsigned, -(widen(b[h]) * f));
     }
-    __device__ __forceinline__ void scaled(const chunk &pn, const chunk &b, half2v (&out)[W / 2]) const
+    __device__ __forceinline__ half2v scaled_pair(unsigned v, unsigned b) const
     {
         const half2v zero = {(_Float16)0.f, (_Float16)0.f}, one = {(_Float16)1.f, (_Float16)1.f};
+        const half2v d = __builtin_elementwise_fma(widen(v), f, __builtin_bit_cast(half2v, b));
+        return __builtin_elementwise_min(__builtin_elementwise_max(d * d, zero), one);
+    }
+    __device__ __forceinline__ void scaled(const chunk &pn, const chunk &b, half2v (&out)[W / 2]) const
+    {
 #pragma unroll
-        for (int h = 0; h < W / 2; h++) {
-            const half2v d = __builtin_elementwise_fma(widen(pn[h]), f, __builtin_bit_cast(half2v, b[h]));
-            out[h] = __builtin_elementwise_min(__builtin_elementwise_max(d * d, zero), one);
-        }
+        for (int h = 0; h < W / 2; h++) out[h] = scaled_pair(pn[h], b[h]);
     }
     __device__ __forceinline__ void store_scaled(const chunk &pn, const chunk &b, _Float16 *dst) const
     {
@@ -1316,12 +1320,15 @@ void filter_mfma(MfmaArgs<TS> a)
 // slot w and, unless w = (workgroup index + 7) mod 8, slot
 // 8 + (w - workgroup index) mod 8.
 //
-// Run moves (FP16 form): slot w's chunks are loaded only at every third
-// offset of a run of the full search (one dz and dy, dx stepping by 2) and
-// moved one dword along the row in between (each lane loads 16 columns for
-// that), which skips about half of slot w's loads at search
-// radius 7: 3-4% faster.  Moving the second slot as well, or moving in the
-// BF16 form, puts a spill reload into the loop and was slower (3% and 7%).
+// Run moves (FP16 form): a slot's chunks are loaded only at every third
+// offset of a run of the full search (one dz and dy, dx stepping by 2).  A
+// lane loads 16 columns, of which such an offset and the next two read 12
+// each, one dword further on each time; three copies of the staging name the
+// registers, so a move costs no instruction.  It skips about half of the
+// loads at search radius 7, whose data return (86% busy) is what the full
+// search comes nearest to: FP16, 1326 offsets of 1024x1024x512, 422 -> 407 ms
+// against moving only slot w's registers.  In the BF16 form the longer tails
+// spill in the loop: 463 -> 482 ms.
 // ---------------------------------------------------------------------------
 // operand reads in flight ahead of the MFMA that consumes them
 #ifndef INLM_B4_KD
@@ -1542,36 +1549,34 @@ filter_mfma_b4(MfmaArgs<TS> a)
         return (unsigned)((lin - min_lin) * (int)sizeof(TS));
     };
     // per slot: 8 columns and the tail behind them, the next four, or the next
-    // eight for slot A of the FP16 form, which moves its chunks along runs of
-    // the search instead of loading them at every offset (below).  Only the
+    // eight in the FP16 form, which reads its chunks moved along runs of the
+    // search instead of loading them at every offset (below).  Only the
     // row's last lane (cg = 3) needs columns no other lane holds, but with a
-    // tail of its own in every lane neither the staging nor a move exchanges
-    // lanes or branches, in as many vector instructions (the masked ones took
-    // a slot too): lists of 128 offsets, BF16, 640x640x256: 12.1 -> 11.9 ms a
-    // call; the full search the same within 0.3%.
-    constexpr bool kMove = std::is_same<TS, _Float16>::value && !PRUNED;
+    // tail of its own in every lane the staging exchanges no lanes, in as many
+    // vector instructions (the masked ones took a slot too): lists of 128
+    // offsets, BF16, 640x640x256: 12.1 -> 11.9 ms a call; the full search the
+    // same within 0.3%.
+        constexpr bool kMove = std::is_same<TS, _Float16>::value && !PRUNED;
     chunk8 pnA, pnX;
-    std::conditional_t<kMove, chunk8, chunk4> pqA = {};
-    chunk4 pqX = {};
-    auto load_chunks = [&](int lin, bool slot_a) __attribute__((always_inline)) {
+    typedef std::conditional_t<kMove, ST8, ST4> STT;
+    const STT stt{};
+    typename STT::chunk pqA = {}, pqX = {};
+    auto load_chunks = [&](int lin) __attribute__((always_inline)) {
         const rsrc_t r = rsrc_p(lin);
         const unsigned so = soff_of(lin);
         const unsigned oA = (unsigned)(coffA * (int)sizeof(TS)), oX = (unsigned)(coffX * (int)sizeof(TS));
-        if (slot_a) {
-            stg8.load(pnA, r, oA, so);
-            if constexpr (kMove) stg8.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
-            else stg4.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
-        }
+        stg8.load(pnA, r, oA, so);
+        stt.load(pqA, r, oA + 8 * (unsigned)sizeof(TS), so);
         if (two) {
             stg8.load(pnX, r, oX, so);
-            stg4.load(pqX, r, oX + 8 * (unsigned)sizeof(TS), so);
+            stt.load(pqX, r, oX + 8 * (unsigned)sizeof(TS), so);
         }
     };
     // the chunks at the tile's own positions (the P(y) side of every
     // difference, search offset 0), scaled by -f, in registers
     chunk8 p0A, p0X;
     chunk4 q0A, q0X;
-    load_chunks(0, true);
+    load_chunks(0);
     __builtin_memcpy(&p0A, &pnA, sizeof(p0A));
     __builtin_memcpy(&q0A, &pqA, sizeof(q0A));
     stg8.own_scaled(p0A);
@@ -1585,46 +1590,30 @@ filter_mfma_b4(MfmaArgs<TS> a)
     auto st16 = [](_Float16 *dst, const half2v *v) __attribute__((always_inline)) {
         __builtin_memcpy(__builtin_assume_aligned(dst, 16), v, 16);
     };
-    // window 2 cg (own 8 columns) and window 2 cg + 1 (the upper four, then
-    // the tail's first four)
-    auto store_slot = [&](_Float16 *buf, const chunk8 &pn, const chunk8 &p0, const chunk4 &pq, const chunk4 &q0,
-                          int lrow) __attribute__((always_inline)) {
-        half2v d[4], e[4], d4[2];
-        stg8.scaled(pn, p0, d);
-        stg4.scaled(pq, q0, d4);
-        e[0] = d[2];
-        e[1] = d[3];
-        e[2] = d4[0];
-        e[3] = d4[1];
+    // window 2 cg (columns 8 cg .. + 7) and window 2 cg + 1 (8 cg + 4 .. + 11)
+    // of the loaded columns moved by S dwords
+    auto store_slot = [&](auto sc, _Float16 *buf, const chunk8 &pn, const typename STT::chunk &pq, const chunk8 &p0,
+                          const chunk4 &q0, int lrow) __attribute__((always_inline)) {
+        constexpr int S = decltype(sc)::value;
+        half2v d[6];
+        mstatic_for<0, 6>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            d[i] = stg8.scaled_pair(i + S < 4 ? pn[(i + S) & 3] : pq[(i + S) & 3], i < 4 ? p0[i & 3] : q0[i & 1]);
+        });
         st16(buf + lrow, d);
-        st16(buf + lrow + 8, e);
+        st16(buf + lrow + 8, d + 2);
     };
-    auto stage = [&](_Float16 *buf) __attribute__((always_inline)) {
-        chunk4 pq;
-        __builtin_memcpy(&pq, &pqA, sizeof(pq));
-        store_slot(buf, pnA, p0A, pq, q0A, lrowA);
-        if (two) store_slot(buf, pnX, p0X, pqX, q0X, lrowX);
+    auto stage_at = [&](auto sc, _Float16 *buf) __attribute__((always_inline)) {
+        store_slot(sc, buf, pnA, pqA, p0A, q0A, lrowA);
+        if (two) store_slot(sc, buf, pnX, pqX, p0X, q0X, lrowX);
     };
-    // Slot A's chunks of an offset from those of the offset before it when
-    // the two differ by dx + 2 (same dz and dy): each region row moves by one
-    // dword, so dwords 1-3 move down and the last comes from the tail, which
-    // holds the next eight columns of the loaded offset and so serves two
-    // such moves.
-    auto move_a = [&]() __attribute__((always_inline)) {
-        if constexpr (kMove) {
-            unsigned w[4], tl[4];
-            __builtin_memcpy(w, &pnA, 16);
-            __builtin_memcpy(tl, &pqA, 16);
-            w[0] = w[1];
-            w[1] = w[2];
-            w[2] = w[3];
-            w[3] = tl[0];
-            tl[0] = tl[1];
-            tl[1] = tl[2];
-            tl[2] = tl[3];
-            __builtin_memcpy(&pnA, w, 16);
-            __builtin_memcpy(&pqA, tl, 16);
-        }
+    // An offset that differs from the loaded one by moves of dx + 2 (same dz
+    // and dy) reads each region row moves dwords further on, in the registers
+    // that are there.
+    auto stage = [&](_Float16 *buf, int moves) __attribute__((always_inline)) {
+        if (!kMove || moves == 0) stage_at(std::integral_constant<int, 0>{}, buf);
+        else if (moves == 1) stage_at(std::integral_constant<int, 1>{}, buf);
+        else stage_at(std::integral_constant<int, 2>{}, buf);
     };
     struct RVals {
         TS v[b4::NH][4];
@@ -1679,19 +1668,20 @@ filter_mfma_b4(MfmaArgs<TS> a)
         }
         return a.search_full[i].lin;
     };
-    // per offset of the full search, after the table: 0 to load slot A's
-    // chunks, s > 0 to move those of the offset before it (kStageMovesMax)
+    // per offset of the full search, after the table: 0 to load
+    // the chunks, s > 0 to read the loaded ones moved by s dwords
+    // (kStageMovesMax)
     const int *moves = reinterpret_cast<const int *>(a.search_full + a.n_search);
-    auto loads_a = [&](int mv) __attribute__((always_inline)) { return !kMove || mv == 0; };
+    auto loads = [&](int mv) __attribute__((always_inline)) { return !kMove || mv == 0; };
 
     // Software pipeline as in filter_mfma: step k runs the MFMA chain of
     // offset k right after the barrier, with the weights of offset k-1 and
     // the staging arithmetic of offset k+1 interleaved, writes that plane to
     // the idle buffer and loads the chunks of offset k+2.
     __syncthreads();
-    load_chunks(lin_at(0), true);
-    stage(lds[0]);
-    load_chunks(lin_at(1), loads_a(kMove && nS > 1 ? moves[1] : 0));
+    load_chunks(lin_at(0));
+    stage(lds[0], 0);
+    if (loads(kMove && nS > 1 ? moves[1] : 0)) load_chunks(lin_at(1));
     __syncthreads();
 
     DVals dA, dB;
@@ -1752,8 +1742,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
         for (int h = 0; h < b4::NH; h++)
             asm volatile("" : "+v"(fv[h][0]), "+v"(fv[h][1]), "+v"(fv[h][2]), "+v"(fv[h][3]), "+v"(fw[h][0]),
                          "+v"(fw[h][1]), "+v"(fw[h][2]), "+v"(fw[h][3]));
-        if (!loads_a(m1)) move_a();
-        stage(st);
+        stage(st, m1);
         constexpr int NV = (2 * b4::NH * kWeightValuPacked + kStageValu<TS, _Float16> * 3 * 2 + NR - 2) / (NR - 1);
         __builtin_amdgcn_sched_group_barrier(0x0020, b4::NH, 0);
         __builtin_amdgcn_sched_group_barrier(0x0100, KD, 0);
@@ -1763,7 +1752,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
             if constexpr (decltype(ri)::value >= 1) __builtin_amdgcn_sched_group_barrier(0x0002, NV, 0);
         });
         __builtin_amdgcn_sched_barrier(0);
-        load_chunks(l2, loads_a(m2));
+        if (loads(m2)) load_chunks(l2);
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < b4::NH; h++) dout[h] = acc[h];
