@@ -1615,36 +1615,68 @@ filter_mfma_b4(MfmaArgs<TS> a)
         else if (moves == 1) stage_at(std::integral_constant<int, 1>{}, buf);
         else stage_at(std::integral_constant<int, 2>{}, buf);
     };
+    // the R values of a lane's outputs: in the full search eight columns of the
+    // loaded offset, of which it and the next two along its run read four
+    // each, named by three copies of the sums (FP16, 1326 offsets of
+    // 1024x1024x512: 391 -> 385 ms against a load at every offset)
+    constexpr bool kMoveR = !PRUNED;
     struct RVals {
-        TS v[b4::NH][4];
+        unsigned v[b4::NH][kMoveR ? 4 : 2];
     };
     auto load_r = [&](RVals &rv, int lin) __attribute__((always_inline)) {
         const rsrc_t r = rsrc_r(lin);
         const unsigned so = soff_of(lin);
 #pragma unroll
         for (int h = 0; h < b4::NH; h++) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, rbyte + h * rhalf, so, 0);
-            __builtin_memcpy(rv.v[h], &v, 8);
+            if constexpr (kMoveR) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, rbyte + h * rhalf, so, 0);
+                __builtin_memcpy(rv.v[h], &v, 16);
+            } else {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, rbyte + h * rhalf, so, 0);
+                __builtin_memcpy(rv.v[h], &v, 8);
+            }
         }
     };
     typedef floatx4 DVals[b4::NH];
-    auto accumulate = [&](const DVals &dd, const RVals &rv) __attribute__((always_inline)) {
+    typedef half2w WVals[b4::NH][2];
+    auto weights = [&](const DVals &dd, WVals &w) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < b4::NH; h++) {
             const floatx4 &d = dd[h];
-            half2w w[2];
             packed_weights(__builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[0], d[1])),
-                           __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2], d[3])), msu, w[0], w[1]);
+                           __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2], d[3])), msu, w[h][0], w[h][1]);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float wi = (float)w[i >> 1][i & 1];
-                fv[h][i] = __builtin_fmaf(wi, (float)rv.v[h][i], fv[h][i]);
+            for (int i = 0; i < 4; i++)
                 // times a runtime 1.0, so the sum stays one mixed-precision FMA
-                fw[h][i] = __builtin_fmaf(wi, one, fw[h][i]);
-            }
+                fw[h][i] = __builtin_fmaf((float)w[h][i >> 1][i & 1], one, fw[h][i]);
 #pragma unroll
             for (int j = 0; j < 2; j++)
-                wmax2[h][j] = __builtin_elementwise_max(wmax2[h][j], __builtin_bit_cast(ushort2w, w[j]));
+                wmax2[h][j] = __builtin_elementwise_max(wmax2[h][j], __builtin_bit_cast(ushort2w, w[h][j]));
+        }
+    };
+    auto sums_at = [&](auto sc, const WVals &w, const RVals &rv) __attribute__((always_inline)) {
+        constexpr int S = decltype(sc)::value;
+#pragma unroll
+        for (int h = 0; h < b4::NH; h++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+            {
+                typedef TS pair __attribute__((ext_vector_type(2)));
+                const pair r = __builtin_bit_cast(pair, rv.v[h][(i >> 1) + S]);
+                fv[h][i] = __builtin_fmaf((float)w[h][i >> 1][i & 1], (float)r[i & 1], fv[h][i]);
+            }
+        // keeps the copies apart: merged into one, they would index R in memory
+#pragma unroll
+        for (int h = 0; h < b4::NH; h++)
+            asm volatile("; moved %4" : "+v"(fv[h][0]), "+v"(fv[h][1]), "+v"(fv[h][2]), "+v"(fv[h][3]) : "n"(S));
+    };
+    auto sums = [&](const WVals &w, const RVals &rv, int moves) __attribute__((always_inline)) {
+        if constexpr (kMoveR) {
+            if (moves == 0) sums_at(std::integral_constant<int, 0>{}, w, rv);
+            else if (moves == 1) sums_at(std::integral_constant<int, 1>{}, w, rv);
+            else sums_at(std::integral_constant<int, 2>{}, w, rv);
+        } else {
+            sums_at(std::integral_constant<int, 0>{}, w, rv);
         }
     };
 
@@ -1691,16 +1723,16 @@ filter_mfma_b4(MfmaArgs<TS> a)
         dA[h] = floatx4{0.f, 0.f, 0.f, 0.f};
         dB[h] = floatx4{__builtin_inff(), __builtin_inff(), __builtin_inff(), __builtin_inff()};
 #pragma unroll
-        for (int i = 0; i < 4; i++) rA.v[h][i] = rB.v[h][i] = TS(0.f);
+        for (int i = 0; i < (kMoveR ? 4 : 2); i++) rA.v[h][i] = rB.v[h][i] = 0u;
     }
     constexpr int kBlock = 62;
     // per lane of a 62-step block: offset kb + lane packed as lin * 4 + moves;
     // a step reads the entry of offset k+2 and carries those of k and k+1
     int pkv = 0, kb = 0;
     auto packed_at = [&](int k) __attribute__((always_inline)) {
-        return lin_at(k) * 4 + (kMove && k < nS ? moves[k] : 0);
+        return lin_at(k) * 4 + (kMoveR && k < nS ? moves[k] : 0);
     };
-    int pc0 = packed_at(0), pc1 = packed_at(1);
+    int pc0 = packed_at(0), pc1 = packed_at(1), mp = 0;
     auto step = [&](int k, const _Float16 *rd, _Float16 *st, DVals &dout, RVals &rout, const DVals &din,
                     const RVals &rin) __attribute__((always_inline)) {
         const int p2 = __builtin_amdgcn_readlane(pkv, k + 2 - kb);
@@ -1708,9 +1740,10 @@ filter_mfma_b4(MfmaArgs<TS> a)
         const int l2 = p2 >> 2;
         const int m1 = pc1 & 3;
         const int m2 = p2 & 3;
+        const int m0 = pc0 & 3;
         pc0 = pc1;
         pc1 = p2;
-        load_r(rout, l0);
+        if constexpr (!kMoveR) load_r(rout, l0);
         DVals acc;
 #pragma unroll
         for (int h = 0; h < b4::NH; h++) acc[h] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1733,15 +1766,18 @@ filter_mfma_b4(MfmaArgs<TS> a)
             acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop[b4::kCls[o]], ab[r % KD], acc[h], 0, 0, 0);
             if constexpr (r + KD < NR) ab[r % KD] = b_of(std::integral_constant<int, r + KD>{});
         });
-        accumulate(din, rin);
+        WVals w;
+        weights(din, w);
         // The sums are finished in the block that holds the MFMAs: left free,
         // the compiler moves the weights behind the branches of the staging,
         // where no MFMA runs beside them (FP16, 1326 offsets of 1024x1024x512:
         // 425 -> 411 ms).
 #pragma unroll
         for (int h = 0; h < b4::NH; h++)
-            asm volatile("" : "+v"(fv[h][0]), "+v"(fv[h][1]), "+v"(fv[h][2]), "+v"(fv[h][3]), "+v"(fw[h][0]),
-                         "+v"(fw[h][1]), "+v"(fw[h][2]), "+v"(fw[h][3]));
+            asm volatile("" : "+v"(fw[h][0]), "+v"(fw[h][1]), "+v"(fw[h][2]), "+v"(fw[h][3]), "+v"(wmax2[h][0]),
+                         "+v"(wmax2[h][1]), "+v"(w[h][0]), "+v"(w[h][1]));
+        sums(w, rin, mp);
+        mp = m0;
         stage(st, m1);
         constexpr int NV = (2 * b4::NH * kWeightValuPacked + kStageValu<TS, _Float16> * 3 * 2 + NR - 2) / (NR - 1);
         __builtin_amdgcn_sched_group_barrier(0x0020, b4::NH, 0);
@@ -1752,6 +1788,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
             if constexpr (decltype(ri)::value >= 1) __builtin_amdgcn_sched_group_barrier(0x0002, NV, 0);
         });
         __builtin_amdgcn_sched_barrier(0);
+        if (kMoveR && m0 == 0) load_r(rout, l0);
         if (loads(m2)) load_chunks(l2);
         __syncthreads();
 #pragma unroll
@@ -1766,13 +1803,17 @@ filter_mfma_b4(MfmaArgs<TS> a)
         pkv = packed_at(kb + ln);
         const int ke = kb + kBlock < nS ? kb + kBlock : nS;
         for (int k = kb; k < ke; k += 2) {
-            step(k, lds[0], lds[1], dA, rA, dB, rB);
-            step(k + 1, lds[1], lds[0], dB, rB, dA, rA);
+            step(k, lds[0], lds[1], dA, rA, dB, kMoveR ? rA : rB);
+            step(k + 1, lds[1], lds[0], dB, kMoveR ? rA : rB, dA, rA);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-    if ((nS & 1) == 0) accumulate(dB, rB);
+    if ((nS & 1) == 0) {
+        WVals w;
+        weights(dB, w);
+        sums(w, kMoveR ? rA : rB, mp);
+    }
 
 #pragma unroll
     for (int h = 0; h < b4::NH; h++) {
