@@ -1015,7 +1015,16 @@ void filter_mfma(MfmaArgs<TS> a)
     auto soff_of = [&](int lin) __attribute__((always_inline)) {
         return (unsigned)((lin - min_lin) * (int)sizeof(TS));
     };
-    chunk8 pn8[S8 > 0 ? S8 : 1];
+    // Along a run of the full search (one dz and dy, dx stepping by 2) every
+    // row moves by one dword.  Where a thread stages one chunk (16-bit storage,
+    // r = 1) it is loaded at every third offset only, with the eight columns
+    // behind it, and the next two offsets read the same registers one and two
+    // dwords further on, named by three copies of the code; R likewise.  The
+    // texture addresser and data return were busy all the time (two loads a
+    // step for 33 vector instructions): FP16, 3102 offsets of 411x377x203,
+    // 51.1 -> 44.8 ms.
+    constexpr bool kMove = !PRUNED && sizeof(TS) == 2 && S8 == 1 && S4 == 0;
+    chunk8 pn8[S8 > 0 ? S8 : 1], pt8[1];
     chunk4 pn4[S4 > 0 ? S4 : 1];
     auto load_chunks = [&](int lin) __attribute__((always_inline)) {
         const rsrc_t r = rsrc_p(lin);
@@ -1024,6 +1033,7 @@ void filter_mfma(MfmaArgs<TS> a)
         for (int c = 0; c < S8; c++) stg8.load(pn8[c], r, (unsigned)(coff8[c] * (int)sizeof(TS)), so);
 #pragma unroll
         for (int c = 0; c < S4; c++) stg4.load(pn4[c], r, (unsigned)(coff4[c] * (int)sizeof(TS)), so);
+        if constexpr (kMove) stg8.load(pt8[0], r, (unsigned)(coff8[0] * (int)sizeof(TS)) + 16u, so);
     };
     auto stage = [&](TD *buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -1041,10 +1051,36 @@ void filter_mfma(MfmaArgs<TS> a)
                 stg4.store(pn4[c], kP0Reg ? p0r4[c] : p0s4[t + c * NTM], buf + loff4[c]);
         }
     };
+    // stages the loaded columns moved by `moves` dwords
+    auto stage_moved = [&](TD *buf, int moves) __attribute__((always_inline)) {
+        auto at = [&](auto sc) __attribute__((always_inline)) {
+            constexpr int S = decltype(sc)::value;
+            chunk8 c;
+            mstatic_for<0, 4>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value + S;
+                c[decltype(ic)::value] = i < 4 ? pn8[0][i & 3] : pt8[0][i & 3];
+            });
+            if constexpr (kSC)
+                stg8.store_scaled(c, kP0Reg ? p0r8[0] : p0s8[t], buf + loff8[0]);
+            else
+                stg8.store(c, kP0Reg ? p0r8[0] : p0s8[t], buf + loff8[0]);
+            // keeps the copies apart: merged into one, they would index the
+            // columns in memory
+            asm volatile("; moved %0" ::"n"(S));
+        };
+        if (moves == 0) at(std::integral_constant<int, 0>{});
+        else if (moves == 1) at(std::integral_constant<int, 1>{});
+        else at(std::integral_constant<int, 2>{});
+    };
     // R at this lane's four outputs shifted by one search offset, in the
-    // stored type
+    // stored type; with moves the eight columns of the loaded offset
     struct RVals {
         TS v[4];
+    };
+    unsigned rm[4] = {0u, 0u, 0u, 0u};
+    auto load_rm = [&](int lin) __attribute__((always_inline)) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_r(lin), rbyte, soff_of(lin), 0);
+        __builtin_memcpy(rm, &v, 16);
     };
     auto load_r = [&](RVals &rv, int lin) __attribute__((always_inline)) {
         const rsrc_t rR = rsrc_r(lin);
@@ -1085,6 +1121,43 @@ void filter_mfma(MfmaArgs<TS> a)
         }
     };
 
+    // the same with R moved: weights and their sums, then sum w R
+    auto accumulate_moved = [&](const floatx4 &d, int moves) __attribute__((always_inline)) {
+        float w[4];
+        half2w wp[2];
+        if constexpr (kPacked) {
+            packed_weights(__builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[0], d[1])),
+                           __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2], d[3])), msu, wp[0], wp[1]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) fw[i] = __builtin_fmaf((float)wp[i >> 1][i & 1], one, fw[i]);
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                wmax2[j] = __builtin_elementwise_max(wmax2[j], __builtin_bit_cast(ushort2w, wp[j]));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                w[i] = fast_weight<WFN>(d[i], ms);
+                fw[i] = fw[i] + w[i];
+                wmax_bits[i] = __builtin_elementwise_max(wmax_bits[i], __builtin_bit_cast(unsigned, w[i]));
+            }
+        }
+        auto at = [&](auto sc) __attribute__((always_inline)) {
+            constexpr int S = decltype(sc)::value;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                TS r[2];
+                __builtin_memcpy(r, &rm[(i >> 1) + S], sizeof(unsigned));
+                if constexpr (kPacked) fv[i] = __builtin_fmaf((float)wp[i >> 1][i & 1], (float)r[i & 1], fv[i]);
+                else fv[i] = __builtin_fmaf(w[i], (float)r[i & 1], fv[i]);
+            }
+            // keeps the copies apart: merged into one, they would index R in memory
+            asm volatile("; moved %4" : "+v"(fv[0]), "+v"(fv[1]), "+v"(fv[2]), "+v"(fv[3]) : "n"(S));
+        };
+        if (moves == 0) at(std::integral_constant<int, 0>{});
+        else if (moves == 1) at(std::integral_constant<int, 1>{});
+        else at(std::integral_constant<int, 2>{});
+    };
+
     // offsets this tile visits: the whole search, or its list
     int nS = a.n_search;
     const int *lst = nullptr;
@@ -1119,9 +1192,13 @@ void filter_mfma(MfmaArgs<TS> a)
     // repeats offset nS-1 and its distances are dropped.
     __syncthreads();  // zeroed LDS visible before the first staging
     auto lin_at = [&](int k) __attribute__((always_inline)) { return lin_of(k < nS ? k : nS - 1); };
+    // kMove: per offset of the full search, after the table, 0 to load or the
+    // dwords the loaded columns are moved by (kStageMovesMax)
+    const int *moves = reinterpret_cast<const int *>(a.search_full + a.n_search);
+    int movv = 0, mp = 0, m0 = 0, m1 = kMove && nS > 1 ? moves[1] : 0;
     load_chunks(lin_at(0));
     stage(lds[0]);
-    load_chunks(lin_at(1));
+    if (m1 == 0) load_chunks(lin_at(1));
     __syncthreads();
 
     // no offset before the first: an infinite distance has weight zero
@@ -1139,7 +1216,16 @@ void filter_mfma(MfmaArgs<TS> a)
                     const RVals &rin) __attribute__((always_inline)) {
         const int l0 = __builtin_amdgcn_readlane(linv, k - kb);
         const int l2 = __builtin_amdgcn_readlane(linv, k + 2 - kb);
-        load_r(rout, l0);
+        const int m2 = kMove ? __builtin_amdgcn_readlane(movv, k + 2 - kb) : 0;
+        if constexpr (!kMove) load_r(rout, l0);
+        auto weigh = [&]() __attribute__((always_inline)) {
+            if constexpr (kMove) accumulate_moved(din, mp);
+            else accumulate(din, rin);
+        };
+        auto put = [&]() __attribute__((always_inline)) {
+            if constexpr (kMove) stage_moved(st, m1);
+            else stage(st);
+        };
         const TD *L = rd + aoff;
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
         if constexpr (!kF8) {
@@ -1164,8 +1250,8 @@ void filter_mfma(MfmaArgs<TS> a)
                 acc = DP::mfma(bop[b], ab[r % KD], acc);
                 if constexpr (r + KD < NR) ab[r % KD] = a_of(std::integral_constant<int, r + KD>{});
             });
-            accumulate(din, rin);
-            stage(st);
+            weigh();
+            put();
             // order: the R load, KD reads, then per MFMA the next A read and
             // a share of the vector work (none right after the first MFMA);
             // the staging writes and the next loads follow the chain
@@ -1197,14 +1283,14 @@ void filter_mfma(MfmaArgs<TS> a)
             };
             vec8 ab[KD];
             mstatic_for<0, KD>([&](auto ri) __attribute__((always_inline)) { ab[decltype(ri)::value] = d_of(ri); });
-            if constexpr (kP0Reg) stage(st);
-            accumulate(din, rin);
+            if constexpr (kP0Reg) put();
+            weigh();
             mstatic_for<0, NM8>([&](auto ri) __attribute__((always_inline)) {
                 constexpr int r = decltype(ri)::value;
                 acc = DP::mfma(bop[F8PlanOf<R, ISO>::value.sig[r]], ab[r % KD], acc);
                 if constexpr (r + KD < NM8) ab[r % KD] = d_of(std::integral_constant<int, r + KD>{});
             });
-            if constexpr (!kP0Reg) stage(st);
+            if constexpr (!kP0Reg) put();
             // order: the first KD operand reads; while they land, the staging
             // of the next plane when its inputs are all in registers (its two
             // LDS writes then overlap the MFMA chain instead of preceding the
@@ -1223,12 +1309,19 @@ void filter_mfma(MfmaArgs<TS> a)
         }
         // the loads below overwrite the chunks the staging has just read
         __builtin_amdgcn_sched_barrier(0);
-        load_chunks(l2);
+        if constexpr (kMove) {
+            if (m0 == 0) load_rm(l0);
+            mp = m0;
+            m0 = m1;
+            m1 = m2;
+        }
+        if (m2 == 0) load_chunks(l2);
         __syncthreads();
         dout = acc;
     };
     for (kb = 0; kb < nS; kb += kBlock) {
         linv = lin_at(kb + lane);
+        if constexpr (kMove) movv = kb + lane < nS ? moves[kb + lane] : 0;
         const int ke = kb + kBlock < nS ? kb + kBlock : nS;
         for (int k = kb; k < ke; k += 2) {
             step(k, lds[0], lds[1], dA, rA, dB, rB);
@@ -1239,7 +1332,10 @@ void filter_mfma(MfmaArgs<TS> a)
     // (the compiler counts them across the loop exit too; these make sure)
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-    if ((nS & 1) == 0) accumulate(dB, rB);
+    if ((nS & 1) == 0) {
+        if constexpr (kMove) accumulate_moved(dB, mp);
+        else accumulate(dB, rB);
+    }
 
     float wmax[4];
 #pragma unroll

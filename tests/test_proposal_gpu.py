@@ -262,6 +262,38 @@ def test_lists_on_the_block_kernels_equal_the_row_kernel(gpu_available, form, rp
     assert mx < 0.02 and rms < 2e-4, (mx, rms)
 
 
+@pytest.mark.parametrize("weight_fn", ["pade", "exp"])
+@pytest.mark.parametrize("form", ["fp16", "bf16", "fp16_fp8"])
+@pytest.mark.parametrize("shape,rs,aniso", [((33, 9, 9), (10, 2, 1), 1.0), ((64, 24, 16), (4, 4, 3), 2.0),
+                                            ((31, 8, 7), (1, 1, 1), 1.0), ((70, 17, 8), (7, 1, 2), 0.5)])
+def test_radius1_runs_equal_a_load_per_offset(gpu_available, form, weight_fn, shape, rs, aniso):
+    """Patch radius 1: the full search reads its columns and R along runs of
+    the search (of every length from 1 to 11 here); a tile whose list is the
+    whole search loads them at every offset, in the same order, so the results
+    are equal to the bit."""
+    nx, ny, nz = shape
+    spec = ph.PhantomSpec(shape, seed=nx, radii=(2, 7), noise_sigma=1500.0, blur_sigma=0.8)
+    raw = ph.make(spec)
+    sig = np.linspace(600.0, 900.0, nz).astype(np.float32)
+    ns = len(O.search_offsets(rs))
+    nt = ((nx + 31) // 32) * ((ny + 7) // 8) * ((nz + 7) // 8)
+    outs = []
+    for whole in (False, True):
+        print(f"[gpu] r=1 {form} wf={weight_fn} {shape} rs={rs} aniso={aniso} lists={whole}", flush=True)
+        p = DenoiseParameters(radius_searchspace=list(rs), radius_patchspace=[1] * 3, precision=form,
+                              weight_fn=weight_fn, z_anisotropy=aniso)
+        g = IterativeNLM_GPU()
+        assert g.configure_device(list(shape), p) == nz
+        g.load_raw(raw)
+        g.set_sigma(sig)
+        if whole:
+            g.set_offset_lists(np.zeros((nt, 1), np.int32), np.full(nt, ns, np.int32), 1)
+        g.Run_GaussianNoise(1)
+        outs.append(g.get_result())
+        g.free_device()
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("form", ["fp16", "fp16_fp8"])
 def test_proposal_fallback_audit_and_topk(gpu_available, form):
     spec = ph.PhantomSpec((64, 32, 24), seed=81, radii=(2, 7), streaks=3, streak_len=(5, 15))
