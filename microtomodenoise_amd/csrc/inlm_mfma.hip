@@ -468,57 +468,6 @@ __device__ __forceinline__ void packed_weights(half2w d0, half2w d1, half2w ms, 
     w1 = __builtin_elementwise_fma(p1, u1, s1);
 }
 
-// One offset's weights (divided by c0) and sums for a run of four outputs, two
-// to an instruction, as N pieces of two to four instructions that a step puts
-// between its MFMAs (the two polynomial chains in lockstep, as in
-// packed_weights).
-template <class TS>
-struct WeightStep {
-    static constexpr int N = 11;
-    half2w u[2], p[2], s[2];
-    template <int S>
-    __device__ __forceinline__ void piece(const floatx4 &d, const TS (&r)[4], half2w ms, float unit, float (&fv)[4],
-                                          float (&fw)[4], ushort2w (&wmax2)[2])
-    {
-        constexpr const _Float16 *Q = kPadePolyQ5;
-        const half2w zero = {(_Float16)0.f, (_Float16)0.f}, one = {(_Float16)1.f, (_Float16)1.f};
-        const half2w big = {(_Float16)16384.f, (_Float16)16384.f};
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if constexpr (S == 0) {
-                u[j] = __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2 * j], d[2 * j + 1]));
-            } else if constexpr (S == 1) {
-                u[j] = __builtin_elementwise_fma(u[j], ms, one);
-                u[j] = __builtin_elementwise_min(__builtin_elementwise_max(u[j], zero), one);
-                p[j] = half2w{Q[4], Q[4]};
-            } else if constexpr (S <= 5) {
-                p[j] = __builtin_elementwise_fma(p[j], u[j], half2w{Q[5 - S], Q[5 - S]});
-            } else if constexpr (S == 6) {
-                s[j] = u[j] * big;
-                s[j] = __builtin_elementwise_min(__builtin_elementwise_max(s[j], zero), one);
-            } else if constexpr (S == 7) {
-                p[j] = __builtin_elementwise_fma(p[j], u[j], s[j]);
-            } else if constexpr (S <= 9) {
-                constexpr int k = S - 8;
-                const float w = (float)p[k][j];
-                fv[2 * k + j] = __builtin_fmaf(w, (float)r[2 * k + j], fv[2 * k + j]);
-                // times a runtime 1.0, so the sum stays one mixed-precision FMA
-                fw[2 * k + j] = __builtin_fmaf(w, unit, fw[2 * k + j]);
-            } else {
-                // weights are non-negative: their FP16 bit patterns order like them
-                wmax2[j] = __builtin_elementwise_max(wmax2[j], __builtin_bit_cast(ushort2w, p[j]));
-            }
-        }
-    }
-    __device__ __forceinline__ void all(const floatx4 &d, const TS (&r)[4], half2w ms, float unit, float (&fv)[4],
-                                        float (&fw)[4], ushort2w (&wmax2)[2])
-    {
-        mstatic_for<0, N>([&](auto i) __attribute__((always_inline)) {
-            piece<decltype(i)::value>(d, r, ms, unit, fv, fw, wmax2);
-        });
-    }
-};
-
 template <int WFN>
 __host__ __device__ constexpr float weight_scale_factor()
 {
@@ -2163,7 +2112,18 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         __builtin_memcpy(rv.v, &v, 8);
     };
     auto accumulate = [&](const floatx4 &d, const RVals &rv) __attribute__((always_inline)) {
-        WeightStep<TS>{}.all(d, rv.v, msu, one, fv, fw, wmax2);
+        half2w w[2];
+        packed_weights(__builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[0], d[1])),
+                       __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2], d[3])), msu, w[0], w[1]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float wi = (float)w[i >> 1][i & 1];
+            fv[i] = __builtin_fmaf(wi, (float)rv.v[i], fv[i]);
+            // times a runtime 1.0, so the sum stays one mixed-precision FMA
+            fw[i] = __builtin_fmaf(wi, one, fw[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) wmax2[i] = __builtin_elementwise_max(wmax2[i], __builtin_bit_cast(ushort2w, w[i]));
     };
 
     // offsets this tile visits: the whole search, or its list
@@ -2214,30 +2174,20 @@ __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         };
         half8 ab[KD];
         mstatic_for<0, KD>([&](auto ri) __attribute__((always_inline)) { ab[decltype(ri)::value] = b_of(ri); });
-        __builtin_amdgcn_sched_barrier(0);
-        // Each MFMA with the read KD ahead and a share of the weights of
-        // offset k-1 and of the staging of offset k+1, in this order: left to
-        // itself the compiler interleaved one of the two unrolled steps and
-        // ran the other's reads, MFMAs and vector work one after the other
-        // (BF16, 1326 offsets of 512x512x128: 49.3 -> 48.0 ms).
-        WeightStep<TS> ws;
-        half2v dn[b82::NSLOT][4];
-        constexpr int NP = WeightStep<TS>::N + 5 * b82::NSLOT;
         mstatic_for<0, NR>([&](auto ri) __attribute__((always_inline)) {
             constexpr int r = decltype(ri)::value;
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop[b82::kCls[r]], ab[r % KD], acc, 0, 0, 0);
             if constexpr (r + KD < NR) ab[r % KD] = b_of(std::integral_constant<int, r + KD>{});
-            mstatic_for<NP * r / NR, NP *(r + 1) / NR>([&](auto pi) __attribute__((always_inline)) {
-                constexpr int i = decltype(pi)::value;
-                if constexpr (i < WeightStep<TS>::N) {
-                    ws.template piece<i>(din, rin.v, msu, one, fv, fw, wmax2);
-                } else {
-                    constexpr int c = (i - WeightStep<TS>::N) / 5, e = (i - WeightStep<TS>::N) % 5;
-                    if constexpr (e < 4) dn[c][e] = stg.scaled_pair(pn[c][e], p0[c][e]);
-                    else __builtin_memcpy(__builtin_assume_aligned(st + 8 * (t + c * NTM), 16), dn[c], 16);
-                }
-            });
-            __builtin_amdgcn_sched_barrier(0);
+        });
+        accumulate(din, rin);
+        stage(st);
+        constexpr int NV = (2 * kWeightValuPacked + kStageValu<TS, _Float16> * 2 * b82::NSLOT + NR - 2) / (NR - 1);
+        __builtin_amdgcn_sched_group_barrier(0x0020, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x0100, KD, 0);
+        mstatic_for<0, NR>([&](auto ri) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
+            if constexpr (decltype(ri)::value + KD < NR) __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);
+            if constexpr (decltype(ri)::value >= 1) __builtin_amdgcn_sched_group_barrier(0x0002, NV, 0);
         });
         // the loads below overwrite the chunks the staging has just read
         __builtin_amdgcn_sched_barrier(0);
