@@ -21,8 +21,7 @@
 // 32x8x8 output tile and stages D_s over the tile plus the patch halo in LDS
 // (double buffered, one barrier per offset); wavefront w computes the 16x16
 // block x-half (w & 1), z pair (w >> 1).  At patch radius 2 the 16-bit forms
-// run a block form (filter_mfma_b4, further below), at radius 3 another
-// (filter_mfma_b82).
+// run the block form (filter_mfma_b4, further below).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1938,297 +1937,6 @@ filter_mfma_b4(MfmaArgs<TS> a)
 }
 
 // ---------------------------------------------------------------------------
-// Block form for patch radius 3 (FP16 and BF16 storage, FP16 D planes; full
-// search and per-tile lists).
-//
-// A block is 8x2 outputs in (x, y) at one z.  Its patch rows lie in 14 of 16
-// columns from x0 - 4, so one v_mfma_f32_16x16x32_f16 takes two such rows of
-// 16 blocks (A: the weights of output m = (bx, by) at row q / 2, columns
-// 8 (q % 2) ..; B: the D rows of block n).  Plane dz = 0 needs rows -3..4 (four
-// products), dz = +-1 and +-2 rows -2..3 (three each), dz = +-3 rows 0, 1 (one
-// each): 18 products and 18 LDS reads per 256 outputs, where the row form's
-// 16-wide rows take 27 and 29 (and are bound by those reads).  The weights
-// depend on |dz|: 11 A operands in 44 registers, which leave two workgroups
-// per CU.
-//
-// A workgroup of 8 wavefronts owns a 32x8x8 tile, wave w slice Z0 + w; D over
-// the tile and its halo is staged as 8-column chunks in rows of 40 columns
-// (x from X0 - 4), chunk c at 16 c bytes.  With 80-byte rows and the block of
-// lane n at x-block (n2, n0), y-block (n1, n3) (bits of n), the 16 lanes of
-// every service group of a ds_read_b128 hit 16 distinct 16-byte bank groups.
-// The pipeline is filter_mfma's.  BF16, 1326 offsets of 512x512x128: 49.2 ms
-// a pass against the row form's 75.0.
-// ---------------------------------------------------------------------------
-namespace b82 {
-constexpr int TX = 32, TY = 8, TZ = 8;
-constexpr int RY = TY + 6, RZ = TZ + 6, CPR = 5;  // region rows, slices, chunks per row
-constexpr int ROW = 8 * CPR, SLICE = RY * ROW;     // halves
-constexpr int NCHUNK = RZ * RY * CPR;
-constexpr int NSLOT = (NCHUNK + NTM - 1) / NTM;
-constexpr int LDS = NSLOT * NTM * 8;  // halves per buffer; slots past the region write behind it
-constexpr int NOPS = 18, NCLS = 11;
-// plane, first row and A operand of each product
-constexpr int kDz[NOPS] = {0, 0, 0, 0, 1, 1, 1, -1, -1, -1, 2, 2, 2, -2, -2, -2, 3, -3};
-constexpr int kRow[NOPS] = {-3, -1, 1, 3, -2, 0, 2, -2, 0, 2, -2, 0, 2, -2, 0, 2, 0, 0};
-constexpr int kCls[NOPS] = {0, 1, 2, 3, 4, 5, 6, 4, 5, 6, 7, 8, 9, 7, 8, 9, 10, 10};
-constexpr int kClsOp[NCLS] = {0, 1, 2, 3, 4, 5, 6, 10, 11, 12, 16};
-}  // namespace b82
-
-template <class TS, bool PRUNED>
-__global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) void filter_mfma_b82(MfmaArgs<TS> a)
-{
-    using ST = Stager<8, TS, _Float16>;
-    typedef typename ST::chunk chunk;
-    constexpr const MRows<3> &rows = MRowsOf<3>::value;
-    __shared__ __attribute__((aligned(16))) _Float16 lds[2][b82::LDS];
-    __shared__ float wtab[4 * 4 * 7];  // patch weights by (|dz|, |dy|, dx + 3)
-
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wg = mxcd_swizzle(blockIdx.x, gridDim.x);
-    const int bxi = wg % a.ntx;
-    const int rem = wg / a.ntx;
-    const int byi = rem % a.nty;
-    const int bzi = rem / a.nty;
-    const int X0 = bxi * b82::TX, Y0 = byi * b82::TY, Z0 = bzi * b82::TZ;
-    const FilterGeom g = a.g;
-    const long sp = (long)g.nxp * g.nyp;
-
-    if (t < 112) {
-        const int adz = t / 28, ady = t / 7 % 4, dx = t % 7 - 3;
-        int at = -1;
-#pragma unroll
-        for (int p = 0; p < rows.npat; p++)
-            if (rows.pdy[p] == ady && rows.pdz[p] == adz && dx >= -rows.pj[p] && dx <= rows.pj[p]) at = p * 8 + dx + 3;
-        const float w = (&a.band[0][0])[at >= 0 ? at : 0];
-        wtab[t] = at >= 0 ? w : 0.f;
-    }
-    __syncthreads();
-    const int q = lane >> 4, n = lane & 15;
-    half8 aop[b82::NCLS];
-#pragma unroll
-    for (int c = 0; c < b82::NCLS; c++) {
-        constexpr int kMaxD = 3;
-        const int dz = b82::kDz[b82::kClsOp[c]], dy = b82::kRow[b82::kClsOp[c]] + (q >> 1) - (n >> 3);
-        const int ady = dy < 0 ? -dy : dy;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int dx = 8 * (q & 1) + i - 4 - (n & 7);
-            const bool in = dx >= -kMaxD && dx <= kMaxD && ady <= kMaxD;
-            const float w = wtab[in ? dz * 28 + ady * 7 + dx + 3 : 0];
-            aop[c][i] = (_Float16)(in ? w : 0.f);
-        }
-    }
-
-    // Scaled FP16 planes, as in filter_mfma: D * f^2 clamped to [0, 1] with a
-    // clamped tap four times beyond the tile's largest cutoff distance.
-    float pf;
-    {
-        float smax = 0.f;
-#pragma unroll
-        for (int zz = 0; zz < b82::TZ; zz++) smax = __builtin_fmaxf(smax, a.sigma[Z0 + zz < g.nz ? Z0 + zz : g.nz - 1]);
-        const float x = __builtin_fabsf((-1.f / (smax * smax * a.beta)) * a.mscale) * a.wmin * (1.f / (4.f * 3.56648f));
-        int e = (int)((__builtin_bit_cast(unsigned, x) >> 23) & 0xffu) - 127;
-        e = e < -24 ? -24 : e > 16 ? 16 : e;
-        const int mexp = e >> 1;
-        pf = __builtin_bit_cast(float, (unsigned)(127 + mexp) << 23);
-    }
-
-    // Staging: region row (ry, rz) = slice Z0-3+rz, row Y0-3+ry, column c = x X0-4+c
-    const TS *Pt = a.P + ((long)(Z0 - 3 + g.pz) * sp + (long)(Y0 - 3 + g.py) * g.nxp + (X0 - 4 + g.px));
-    ST stg;
-    const _Float16 fh = (_Float16)pf;
-    stg.f = half2v{fh, fh};
-    int coff[b82::NSLOT];
-    chunk p0[b82::NSLOT];
-#pragma unroll
-    for (int c = 0; c < b82::NSLOT; c++) {
-        const int ci = t + c * NTM < b82::NCHUNK ? t + c * NTM : 0;  // slots past the region repeat chunk 0
-        const int row = ci / b82::CPR;
-        coff[c] = (int)((row / b82::RY) * sp + (long)(row % b82::RY) * g.nxp + 8 * (ci % b82::CPR));
-        stg.load(p0[c], Pt + coff[c]);
-        stg.own_scaled(p0[c]);
-    }
-
-    // this lane's block and outputs
-    const int xb = (n >> 2 & 1) | (n & 1) << 1, yb = (n >> 1 & 1) | (n >> 3) << 1;
-    const int x0 = X0 + 8 * xb + 4 * (q & 1);
-    const int y = Y0 + 2 * yb + (q >> 1);
-    const int z = Z0 + wave;
-    const TS *Rt = a.R + ((long)(Z0 + g.pz) * sp + (long)(Y0 + g.py) * g.nxp + (X0 + g.px));
-    const unsigned rbyte = (unsigned)(((long)(z - Z0) * sp + (long)(y - Y0) * g.nxp + (x0 - X0)) * sizeof(TS));
-    const TS *Rv = reinterpret_cast<const TS *>(reinterpret_cast<const char *>(Rt) + rbyte);
-    const int zc = z < g.nz ? z : g.nz - 1;
-    const float sig = a.sigma[zc];
-    const float mm = (-1.f / (sig * sig * a.beta)) * a.mscale;
-    const int bbase = (wave + 3) * b82::SLICE + (2 * yb + 3 + (q >> 1)) * b82::ROW + 8 * (xb + (q & 1));
-
-    float fv[4] = {0.f, 0.f, 0.f, 0.f}, fw[4] = {0.f, 0.f, 0.f, 0.f};
-    ushort2w wmax2[2] = {{0, 0}, {0, 0}};
-    const _Float16 msu1 = (_Float16)(mm * (1.f / 3.56648f) * (1.f / (pf * pf)));
-    const half2w msu = {msu1, msu1};
-
-    // buffer resources from the smallest search offset; an odd (px + lin)
-    // reads the copy shifted by one element, so every load is 4-byte aligned
-    const TS *Pb = Pt + a.min_lin;
-    const TS *Rb = Rt + a.min_lin;
-    const TS *Pb1 = Pb + (a.shifted - 1);
-    const TS *Rb1 = Rb + (a.shifted - 1);
-    auto records = [](long bytes) __attribute__((always_inline)) {
-        const unsigned long b = (unsigned long)bytes;
-        return (b >> 31) != 0 ? 0x7fffffff : (int)b;
-    };
-    const int nP = records((long)(a.P_end - Pb) * (long)sizeof(TS));
-    const int nR = records((long)(a.R_end - Rb) * (long)sizeof(TS));
-    auto odd_of = [&](int lin) __attribute__((always_inline)) { return ((lin + g.px) & 1) != 0; };
-    const int min_lin = a.min_lin;
-    const float one = a.one;
-    asm volatile("" ::"s"(min_lin), "s"(one));
-    auto soff_of = [&](int lin) __attribute__((always_inline)) {
-        return (unsigned)((lin - min_lin) * (int)sizeof(TS));
-    };
-    chunk pn[b82::NSLOT];
-    auto load_chunks = [&](int lin) __attribute__((always_inline)) {
-        const rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<TS *>(odd_of(lin) ? Pb1 : Pb), (short)0, nP, kRsrcWord3);
-        const unsigned so = soff_of(lin);
-#pragma unroll
-        for (int c = 0; c < b82::NSLOT; c++) stg.load(pn[c], r, (unsigned)(coff[c] * (int)sizeof(TS)), so);
-    };
-    auto stage = [&](_Float16 *buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int c = 0; c < b82::NSLOT; c++) {
-            half2v d[4];
-            stg.scaled(pn[c], p0[c], d);
-            __builtin_memcpy(__builtin_assume_aligned(buf + 8 * (t + c * NTM), 16), d, 16);
-        }
-    };
-    struct RVals {
-        TS v[4];
-    };
-    auto load_r = [&](RVals &rv, int lin) __attribute__((always_inline)) {
-        const rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<TS *>(odd_of(lin) ? Rb1 : Rb), (short)0, nR, kRsrcWord3);
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, rbyte, soff_of(lin), 0);
-        __builtin_memcpy(rv.v, &v, 8);
-    };
-    auto accumulate = [&](const floatx4 &d, const RVals &rv) __attribute__((always_inline)) {
-        half2w w[2];
-        packed_weights(__builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[0], d[1])),
-                       __builtin_bit_cast(half2w, __builtin_amdgcn_cvt_pkrtz(d[2], d[3])), msu, w[0], w[1]);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float wi = (float)w[i >> 1][i & 1];
-            fv[i] = __builtin_fmaf(wi, (float)rv.v[i], fv[i]);
-            // times a runtime 1.0, so the sum stays one mixed-precision FMA
-            fw[i] = __builtin_fmaf(wi, one, fw[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; i++) wmax2[i] = __builtin_elementwise_max(wmax2[i], __builtin_bit_cast(ushort2w, w[i]));
-    };
-
-    // offsets this tile visits: the whole search, or its list
-    int nS = a.n_search;
-    const int *lst = nullptr;
-    if constexpr (PRUNED) {
-        const int c = a.counts[wg];
-        if (c >= 1 && c < nS) {
-            nS = c;
-            lst = a.lists + (long)wg * a.K;
-        }
-    }
-    auto lin_at = [&](int k) __attribute__((always_inline)) {
-        const int i = k < nS ? k : nS - 1;
-        if constexpr (PRUNED) {
-            if (lst) {
-                const unsigned e = (unsigned)lst[i];
-                return a.search[e < (unsigned)a.n_search ? e : 0u].lin;
-            }
-        }
-        return a.search_full[i].lin;
-    };
-
-    load_chunks(lin_at(0));
-    stage(lds[0]);
-    load_chunks(lin_at(1));
-    __syncthreads();
-
-    // no offset before the first: an infinite distance has weight zero
-    floatx4 dA = {0.f, 0.f, 0.f, 0.f};
-    floatx4 dB = {__builtin_inff(), __builtin_inff(), __builtin_inff(), __builtin_inff()};
-    RVals rA, rB;
-#pragma unroll
-    for (int i = 0; i < 4; i++) rA.v[i] = rB.v[i] = TS(0.f);
-    constexpr int kBlock = 62;  // a step looks two offsets ahead in the 64 of linv
-    int linv = 0, kb = 0;
-    auto step = [&](int k, const _Float16 *rd, _Float16 *st, floatx4 &dout, RVals &rout, const floatx4 &din,
-                    const RVals &rin) __attribute__((always_inline)) {
-        load_r(rout, __builtin_amdgcn_readlane(linv, k - kb));
-        const int l2 = __builtin_amdgcn_readlane(linv, k + 2 - kb);
-        const _Float16 *L = rd + bbase;
-        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        constexpr int NR = b82::NOPS, KD = 2;
-        auto b_of = [&](auto oi) __attribute__((always_inline)) {
-            constexpr int o = decltype(oi)::value;
-            return *reinterpret_cast<const half8 *>(
-                __builtin_assume_aligned(L + b82::kDz[o] * b82::SLICE + b82::kRow[o] * b82::ROW, 16));
-        };
-        half8 ab[KD];
-        mstatic_for<0, KD>([&](auto ri) __attribute__((always_inline)) { ab[decltype(ri)::value] = b_of(ri); });
-        mstatic_for<0, NR>([&](auto ri) __attribute__((always_inline)) {
-            constexpr int r = decltype(ri)::value;
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop[b82::kCls[r]], ab[r % KD], acc, 0, 0, 0);
-            if constexpr (r + KD < NR) ab[r % KD] = b_of(std::integral_constant<int, r + KD>{});
-        });
-        accumulate(din, rin);
-        stage(st);
-        constexpr int NV = (2 * kWeightValuPacked + kStageValu<TS, _Float16> * 2 * b82::NSLOT + NR - 2) / (NR - 1);
-        __builtin_amdgcn_sched_group_barrier(0x0020, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x0100, KD, 0);
-        mstatic_for<0, NR>([&](auto ri) __attribute__((always_inline)) {
-            __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
-            if constexpr (decltype(ri)::value + KD < NR) __builtin_amdgcn_sched_group_barrier(0x0100, 1, 0);
-            if constexpr (decltype(ri)::value >= 1) __builtin_amdgcn_sched_group_barrier(0x0002, NV, 0);
-        });
-        // the loads below overwrite the chunks the staging has just read
-        __builtin_amdgcn_sched_barrier(0);
-        load_chunks(l2);
-        __syncthreads();
-        dout = acc;
-    };
-    for (kb = 0; kb < nS; kb += kBlock) {
-        linv = lin_at(kb + lane);
-        // waited for here, not with the loads of the steps
-        asm volatile("" : "+v"(linv));
-        const int ke = kb + kBlock < nS ? kb + kBlock : nS;
-        for (int k = kb; k < ke; k += 2) {
-            step(k, lds[0], lds[1], dA, rA, dB, rB);
-            step(k + 1, lds[1], lds[0], dB, rB, dA, rA);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-    if ((nS & 1) == 0) accumulate(dB, rB);
-
-    if (y < g.ny && z < g.nz) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int x = x0 + i;
-            if (x < g.nx) {
-                const float wmax = (float)__builtin_bit_cast(half2w, wmax2[i >> 1])[i & 1];
-                const long o = ((long)z * g.ny + y) * g.nx + x;
-                float res = a.raw[o];
-                if (wmax > 0.f) {
-                    const double r0 = (double)(float)Rv[i];
-                    const double v = ((double)fv[i] + (double)wmax * r0) / ((double)fw[i] + (double)wmax);
-                    res = (float)(a.shift + v * a.inv_scale);
-                }
-                a.out[o] = res;
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Normalising reflect-pad: padded v_s = (v - shift) * scale in the storage
 // type, mirror without repeating the edge (iternlm_prepare.cpp:6-48).
 // ---------------------------------------------------------------------------
@@ -2522,14 +2230,6 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
             a.ntz = (g.nz + B::TZ - 1) / B::TZ;
             const long nb = (long)a.ntx * a.nty * a.ntz;
             hipLaunchKernelGGL((filter_mfma_b4<TS, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
-            return hipGetLastError();
-        }
-    }
-    // and at patch radius 3, on the same tiles as the row form
-    if constexpr (R == 3 && sizeof(TS) == 2 && std::is_same<TD, _Float16>::value && WFN == 0) {
-        if (!row_form) {
-            if (ol) hipLaunchKernelGGL((filter_mfma_b82<TS, true>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
-            else hipLaunchKernelGGL((filter_mfma_b82<TS, false>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
             return hipGetLastError();
         }
     }

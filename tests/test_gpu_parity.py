@@ -354,34 +354,6 @@ def test_block_kernel_equals_row_kernel(gpu_available, form, shape, rs):
     assert mx < 0.02 and rms < 2e-4, (mx, rms)
 
 
-@pytest.mark.parametrize("form", ["fp16", "bf16"])
-@pytest.mark.parametrize("aniso", [1.0, 2.0])
-@pytest.mark.parametrize("shape", [(32, 8, 8), (33, 9, 9), (31, 7, 23), (70, 40, 2)])
-def test_radius3_block_kernel_equals_row_kernel(gpu_available, form, aniso, shape):
-    """Patch radius 3 in the 16-bit forms: blocks of 8x2 outputs (18 matrix
-    operations) against the row kernel (27), which sum the same FP16 squares
-    in another FP32 order; around the 32x8x8 tiles, odd row pitches, weights
-    with z anisotropy.  The budget of the radius-2 comparison."""
-    nx, ny, nz = shape
-    spec = ph.PhantomSpec(shape, seed=nx, radii=(2, 7), noise_sigma=1500.0, blur_sigma=0.8)
-    raw = ph.make(spec)
-    sig = np.linspace(600.0, 900.0, nz).astype(np.float32)
-    outs = []
-    for ks in (0, 2):
-        print(f"[gpu] r=3 {form} shape {shape} aniso {aniso} kernel_select {ks}", flush=True)
-        g, _ = make_gpu(shape, (4, 3, 2), (3, 3, 3), precision=form, kernel=ks, z_anisotropy=aniso)
-        g.set_sigma(sig)
-        g.Run_GaussianNoise(1, raw)
-        g.set_sigma(sig * np.float32(0.9))
-        g.Run_GaussianNoise(2)
-        outs.append(g.get_result().astype(np.float64))
-        g.free_device()
-    err = np.abs(outs[0] - outs[1]) / spec.noise_sigma
-    mx, rms = float(err.max()), float(np.sqrt(np.mean(err ** 2)))
-    print(f"[gpu]   block vs row: max {mx:.3e} rms {rms:.3e} (noise-sigma units)", flush=True)
-    assert mx < 0.02 and rms < 2e-4, (mx, rms)
-
-
 @pytest.mark.parametrize("form", ["fp16", "bf16", "fp16_fp8"])
 def test_fast_forms_repeat_bit_for_bit(gpu_available, form):
     # the 16-bit forms normalise by the volume's FP64 moments; their
