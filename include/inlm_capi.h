@@ -109,7 +109,8 @@ typedef struct inlm_params {
     /* FP32 form: 0 the tiled kernel where one covers the patch, 1 the
      * per-voxel kernel.  Matrix-core forms: 0 the fastest kernel for the
      * case (at patch radius 2 with 16-bit storage and FP16 planes, the
-     * 4x4-block kernel), 2 the row kernel. */
+     * 4x4-block kernel, for the full search and per-tile lists), 2 the row
+     * kernel. */
     int32_t kernel_select;
     /* NoiseLevel.circular_mask_diameter (denoise_parameters.h:33): when > 0
      * noise samples are drawn only inside that circle around the slice
@@ -200,12 +201,12 @@ INLM_API inlm_status inlm_patchstd_noalloc(const float *vol, const int32_t shape
                                            const int64_t *samples, int64_t n, double *out, int32_t device);
 
 /* Noise level per slice (NoiseLevel::get_noiselevel, noiselevel.cpp:9-95):
- * patch std on the GPU, two-cluster EM in FP64 on the host, global or
+ * patch std and two-cluster EM (FP64) on the GPU, global or
  * z-adaptive, sigma = mean + stds_from_mean * std.  Writes nz floats. */
 INLM_API inlm_status inlm_estimate_noise(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n,
                                          float *sigma_out);
 
-/* The host half of get_noiselevel (noiselevel.cpp:9-95) on per-sample patch
+/* get_noiselevel (noiselevel.cpp:9-95) on the host from per-sample patch
  * standard deviations `stds` (n values for the sorted sample list): FP64
  * two-cluster EM, global or z-adaptive (with the reference's window and its
  * extrapolation into slices without valid samples, noiselevel.cpp:529-606),

@@ -9,10 +9,11 @@
 // which restates Denoiser/iternlm_cpu.cpp:758-843 and the specialised
 // Denoiser/iternlm_cpu_kernels.cpp:7-1108 of the reference.
 //
-// The tiled kernels are offset-major: a workgroup owns a 32x8x8 output tile;
+// The tiled kernels are offset-major: a workgroup owns a 32x8x8 output tile
+// (32x64x1 for flat patches);
 // for each search offset s it stages D_s(y) = (P(y+s) - P(y))^2 over the tile
 // plus the patch halo in LDS (double buffered, one barrier per offset) and
-// every thread sums the stencil for a run of 8 voxels along x from LDS
+// every thread sums the stencil for a run of 4 voxels along x from LDS
 // windows.  D_s(x+p) is the very float the reference computes as tmp*tmp for
 // tap p, and every voxel adds its taps in the reference order with separate
 // multiply and add (this file is compiled with -ffp-contract=off), so the
@@ -299,7 +300,8 @@ constexpr int waves_per_eu() { return Tile<PT>::CPT <= 2 && PT::RX <= 2 && !MASS
 // step waited for three loads one after the other.  Before (with the longer
 // division, a multiply per tap at r = 1 and two reads per row there) and now:
 // r = 1, 3102 offsets of 256^3: 54 and 43 ms; r = 2, 1326 offsets of
-// 301x333x131: 41.6 and 37.6 ms; r = 3, 256x256x96: 40.2 and 39.3 ms.
+// 301x333x131: 41.6 and 34.8 ms (37.6 before xcd_swizzle took any number of
+// workgroups); r = 3, 256x256x96: 40.2 and 38.1 ms.
 template <class PT, int WFN, bool MASS>
 __global__ __launch_bounds__(NTF) __attribute__((amdgpu_waves_per_eu(waves_per_eu<PT, MASS>(), waves_per_eu<PT, MASS>()))) void
 filter_tiled_fp32(TiledArgs a)
@@ -467,8 +469,7 @@ filter_tiled_fp32(TiledArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Per-voxel kernel for any tap table (non-isotropic patches, anisotropic
-// weights): one thread per voxel, gathers straight from global memory, the
+// Per-voxel kernel for any tap table without a tiled kernel: one thread per voxel, gathers straight from global memory, the
 // same operation sequence as the tiled kernel.
 // ---------------------------------------------------------------------------
 struct VoxelArgs {
