@@ -102,6 +102,10 @@ struct Patch {
     static constexpr bool kUniform = RX == 1 && RY == 1 && RZ <= 1;
     // large patches leave whole wavefronts without a weight above the cutoff
     static constexpr bool kSkip = rows.ntaps > 50;
+    // A NaN weight (an exp weight of a NaN distance): isotropic patches take it
+    // for the largest, and the voxel keeps its value; the others pass it over
+    // in the maximum and it reaches the sums, as in the per-voxel kernel.
+    static constexpr bool kNanIsLargest = RX == RY && RX == RZ;
 };
 
 // Compiler fence that also pins the running sums: the row's arithmetic must
@@ -400,7 +404,10 @@ filter_tiled_fp32(TiledArgs a)
                 const float wt = weight_of<WFN>(d[v] * m);
                 fv[v] = fv[v] + wt * rs[v];
                 fw[v] = fw[v] + wt;
-                wmax_bits[v] = __builtin_elementwise_max(wmax_bits[v], __builtin_bit_cast(unsigned, wt));
+                if constexpr (PT::kNanIsLargest)
+                    wmax_bits[v] = __builtin_elementwise_max(wmax_bits[v], __builtin_bit_cast(unsigned, wt));
+                else  // the other operand of a NaN; the builtin would first quiet wmax, an instruction more
+                    asm("v_max_f32 %0, %0, %1" : "+v"(wmax_bits[v]) : "v"(wt));
                 if constexpr (MASS) sw += (valid && x0 + v < g.nx) ? wt : 0.f;
             }
         } else {

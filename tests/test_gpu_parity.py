@@ -126,6 +126,31 @@ def test_infinite_and_nan_values_reach_the_same_voxels(gpu_available, rp):
     assert np.array_equal(bits(outs[0][ok]), bits(outs[1][ok]))
 
 
+@pytest.mark.parametrize("rp", [(1, 1, 2), (1, 1, 3), (2, 2, 1), (3, 3, 1), (3, 3, 2), (2, 2, 0), (3, 3, 0)])
+def test_nan_weights_on_the_tiled_shapes(gpu_available, rp):
+    """An exp weight of a NaN distance is NaN: it reaches the sums and is
+    passed over in the largest weight, as in the per-voxel kernel (both call
+    the same expf, so every bit is equal)."""
+    rng = np.random.default_rng(4)
+    raw = (rng.normal(size=(9, 30, 80)) * 400 + 5000).astype(np.float32)
+    raw[4, 7, 11] = np.nan
+    raw[5, 20, 60] = np.inf
+    raw[5, 21, 61] = np.inf
+    sig = np.full(9, 600.0, np.float32)
+    outs = []
+    for kernel in (0, 1):
+        print(f"[gpu] NaN weights rp={rp} kernel={kernel}", flush=True)
+        g, _ = make_gpu((80, 30, 9), (3, 3, 2), rp, kernel=kernel, weight_fn="exp")
+        g.set_sigma(sig)
+        g.Run_GaussianNoise(1, raw)
+        outs.append(g.get_result())
+        g.free_device()
+    nan = np.isnan(outs[1])
+    assert 0 < nan.sum() < nan.size
+    assert np.array_equal(np.isnan(outs[0]), nan)
+    assert np.array_equal(bits(outs[0][~nan]), bits(outs[1][~nan]))
+
+
 def test_config1_parity_vs_oracle(gpu_available):
     """Config 1 (128x128x64 uint16 phantom, patch r=1, search r=5, 4
     iterations, fixed sigma lists) against the FP32 restatement: every voxel
