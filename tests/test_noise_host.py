@@ -5,10 +5,13 @@ FP64 clustering (inlm_sigma_from_patchstd) against the oracle.  Each oracle
 function is pinned here by brute force or by values derived by hand from the
 reference's loop, not by retyping its formula."""
 import math
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from microtomodenoise_amd import _capi as capi
 from oracle import oracle as O
 
@@ -197,3 +200,25 @@ def test_manual_mode_first_and_later():
     p = params("manual", sigma=(11.0, 22.0))
     assert np.all(capi.sigma_from_patchstd(p, (20, 20, 3), np.zeros(0, np.int64), np.zeros(0), which=0) == 11.0)
     assert np.all(capi.sigma_from_patchstd(p, (20, 20, 3), np.zeros(0, np.int64), np.zeros(0), which=1) == 22.0)
+
+
+def test_samples_are_drawn_without_memory_for_a_second_list():
+    """The sample list is the caller's; with no room for another of its size
+    (6e6 samples, 48 MB, 16 MB of address space left) the call still returns
+    the same samples, and no exception leaves the C entry."""
+    code = """
+import ctypes as C, resource
+import numpy as np
+from microtomodenoise_amd import _capi
+n, sh = 6_000_000, np.array([400, 300, 200], np.int32)
+want = _capi.draw_samples(sh, n, 15, 3)
+got = np.full(n, -1, np.int64)
+size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (16 << 20), -1))
+st = _capi.lib().inlm_draw_samples(_capi.ptr(sh, C.c_int32), n, 15, 3, _capi.ptr(got, C.c_int64))
+resource.setrlimit(resource.RLIMIT_AS, (-1, -1))
+assert st == 0 and np.array_equal(got, want) and np.all(got[1:] >= got[:-1])
+print("same samples")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=ROOT)
+    assert r.returncode == 0 and "same samples" in r.stdout, (r.returncode, r.stderr[-2000:])
