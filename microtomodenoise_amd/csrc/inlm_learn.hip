@@ -103,9 +103,13 @@ __global__ __launch_bounds__(256, 2) void conv16_mfma(const __bf16 *__restrict__
                                                       __bf16 *__restrict__ out, ActGeom g)
 {
     constexpr int XCH = CRX * CRY * CRZ * 2, XPT = (XCH + 255) / 256;  // 16-byte chunks
-    __shared__ __attribute__((aligned(16))) __bf16 xs[CRZ * CRY * CRX * C];
+    __shared__ __attribute__((aligned(16))) __bf16 xs[CRZ * CRY * CRX * C + 8];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int m = lane & 15, q = lane >> 4, k0 = 8 * (q & 1);
+    // the tap past the last: zero weights on a zero input (on a voxel of the
+    // tile they would make a NaN of an infinite activation)
+    __bf16 *const none = xs + CRZ * CRY * CRX * C;
+    if (t < 8) none[t] = (__bf16)0.f;
     const int ntx = (g.nx + CTX - 1) / CTX, nty = (g.ny + CTY - 1) / CTY, ntz = (g.nz + CTZ - 1) / CTZ;
     const long tiles = (long)ntx * nty * ntz;
     const long t0 = tiles * blockIdx.x / gridDim.x, t1 = tiles * (blockIdx.x + 1) / gridDim.x;
@@ -120,7 +124,7 @@ __global__ __launch_bounds__(256, 2) void conv16_mfma(const __bf16 *__restrict__
         else
 #pragma unroll
             for (int e = 0; e < 8; e++) w[c][e] = (__bf16)0.f;
-        const int tp = tap < NTAP ? tap : NTAP - 1;  // the tap past the last has weight zero
+        const int tp = tap < NTAP ? tap : NTAP - 1;
         xoff[c] = ((tp / 9) * CRY * CRX + (tp / 3 % 3) * CRX + tp % 3 + m) * C + k0;
     }
     float bs[4] = {0.f, 0.f, 0.f, 0.f};
@@ -173,7 +177,9 @@ __global__ __launch_bounds__(256, 2) void conv16_mfma(const __bf16 *__restrict__
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     bf16x8 b;
-                    __builtin_memcpy(&b, __builtin_assume_aligned(xrow + xoff[c] + h * 16 * C, 16), 16);
+                    const __bf16 *p = xrow + xoff[c] + h * 16 * C;
+                    if (c == 13 && q >= 2) p = none;
+                    __builtin_memcpy(&b, __builtin_assume_aligned(p, 16), 16);
                     acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c], b, acc[h], 0, 0, 0);
                 }
             if (!row) continue;

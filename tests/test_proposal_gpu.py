@@ -130,6 +130,38 @@ def test_gradients_at_tile_edges(gpu_available, shape):
         assert err <= 2e-2, name
 
 
+@pytest.mark.parametrize("shape", [(16, 8, 8), (40, 17, 9)])
+def test_infinite_activations_pass_the_last_tap(gpu_available, shape):
+    """One voxel's first activation overflows to infinity; in each following
+    layer only the last tap of channel 0 has a weight, so exactly the voxel
+    one step before it stays infinite (every other neighbour is zero times
+    infinity, which the ReLU takes to zero).  The infinite pooled feature
+    makes its tile's probabilities NaN and no other's."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(5)
+    vol = rng.normal(size=(nz, ny, nx)).astype(np.float32)
+    at = (5, 6, 9)  # z, y, x: three steps back stays inside the first tile
+    vol[at] = 1000.0
+    x = float((vol[at] - vol.mean()) / vol.std())
+    w1 = np.zeros((27, 16), np.float32)
+    w1[13, 0] = 3e37
+    assert x * 3e37 > 6e38 and abs(np.delete(vol.ravel(), np.ravel_multi_index(at, vol.shape))).max() < 6
+    w = np.zeros((27, 16, 16), np.float32)
+    w[26, 0, 0] = 1e-3  # the finite activations (up to 3e37) stay far from overflow in the tiles' sums
+    ns = 11
+    wh, bh = np.full((16, ns), 0.5, np.float32), np.zeros(ns, np.float32)
+    zero = np.zeros(16, np.float32)
+    net = PR.OffsetProposal(ns)
+    net.set_params(np.concatenate([w1.ravel(), zero] + [w.ravel(), zero] * 3 + [wh.ravel(), bh]))
+    d = torch.from_numpy(vol).cuda()
+    torch.cuda.synchronize()
+    print(f"[gpu] infinite activation {shape}", flush=True)
+    probs = net.predict(d.data_ptr(), [nx, ny, nz])
+    net.close()
+    assert np.isnan(probs[0]).all()
+    assert np.isfinite(probs[1:]).all()
+
+
 def test_adam_update(gpu_available):
     ns, shape, vol, mass = _net_case(2)
     nz, ny, nx = shape
