@@ -164,6 +164,7 @@ struct inlm_handle {
     // search (the lists of the pruned forms index search_dev)
     inlm::SearchEntry *search_fast_dev = nullptr;
     int min_lin = 0;  // smallest linear search offset
+    int run_loads = 0;  // offsets of the full-search order that begin a run load
     int64_t *samples_dev = nullptr;
     double *std_dev = nullptr;
     int64_t samples_cap = 0;
@@ -510,6 +511,7 @@ inlm_status inlm_create(const inlm_params *pin, const int32_t shape_in[3], int32
             if (c.dz == b.dz && c.dy == b.dy && c.dx == b.dx + 2 && moves[k - 1] < inlm::kStageMovesMax)
                 moves[k] = moves[k - 1] + 1;
         }
+        h->run_loads = (int)std::count(moves.begin(), moves.begin() + (long)ns, 0);
         const size_t tb = sizeof(inlm::SearchEntry) * ns, mb = sizeof(int) * moves.size();
         h->search_fast_blob.resize(tb + mb);
         std::memcpy(h->search_fast_blob.data(), h->search_fast.data(), tb);
@@ -647,7 +649,7 @@ inlm_status run_iteration_impl(inlm_handle *h, int32_t iter, const float *raw, f
         HIP_TRY(h, inlm::launch_filter_mfma(h->p.precision, h->rp_tiled, h->p.weight_fn, h->Rs, P, h->pad_elems, h->shifted,
                                             h->raw, h->result, h->sigma, h->p.beta,
                                             (float)(1.0 / (h->scale * h->scale)), h->shift, 1.0 / h->scale,
-                                            h->search_dev, h->search_fast_dev, ns, h->min_lin, h->taps,
+                                            h->search_dev, h->search_fast_dev, ns, h->run_loads, h->min_lin, h->taps,
                                             h->fg, h->stream, pruned ? &ol : nullptr, h->p.kernel_select == 2));
     } else {
         HIP_TRY(h, inlm::launch_filter(h->p.precision, h->tiled, h->p.weight_fn, h->R_pad,

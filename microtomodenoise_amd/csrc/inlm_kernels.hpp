@@ -91,7 +91,8 @@ bool mfma_taps_supported(int rp, const int *dxyz, const float *w, int n);
 // from each volume to its copy shifted by one element (copy[j] =
 // volume[j + 1], written by launch_pad_normalise); those forms need an even
 // row pitch g.nxp.  0 for FP32_FAST.
-// min_lin: the smallest linear offset of the search table (<= 0).
+// min_lin: the smallest linear offset of the search table (<= 0).  loads: the
+// offsets of search_full with move count 0.
 // Per-tile offset lists for the matrix-core filter (32x8x8 tiles, x fastest):
 // tile t visits the search entries lists[t*K .. t*K + counts[t]) when
 // counts[t] < n_search, else the whole search.  Device pointers.
@@ -104,8 +105,8 @@ struct OffsetLists {
 hipError_t launch_filter_mfma(int form, int rp, int weight_fn, const void *Rs, const void *Ps, size_t elems,
                               long shifted, const float *raw, float *out, const float *sigma, float beta, float mscale,
                               double shift, double inv_scale, const SearchEntry *search,
-                              const SearchEntry *search_full, int n_search, int min_lin, const TapTable &taps,
-                              const FilterGeom &g, hipStream_t st, const OffsetLists *ol = nullptr,
+                              const SearchEntry *search_full, int n_search, int loads, int min_lin,
+                              const TapTable &taps, const FilterGeom &g, hipStream_t st, const OffsetLists *ol = nullptr,
                               bool row_form = false);
 hipError_t launch_pad_normalise(int form, const float *in, void *out, long shifted, const FilterGeom &g, float shift,
                                 float scale, hipStream_t st);

@@ -725,7 +725,7 @@ struct Stager<W, _Float16, f8_t> {
 template <int R, class TS>
 constexpr int mfma_waves_per_eu() { return R <= 2 && sizeof(TS) == 2 ? 6 : 4; }
 
-template <int R, class TS, class TD, int WFN, bool PRUNED, bool ISO>
+template <int R, class TS, class TD, int WFN, bool PRUNED, bool ISO, bool RUNS = false>
 __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu<R, TS>(), mfma_waves_per_eu<R, TS>())))
 void filter_mfma(MfmaArgs<TS> a)
 {
@@ -1014,15 +1014,16 @@ void filter_mfma(MfmaArgs<TS> a)
     auto soff_of = [&](int lin) __attribute__((always_inline)) {
         return (unsigned)((lin - min_lin) * (int)sizeof(TS));
     };
-    // Along a run of the full search (one dz and dy, dx stepping by 2) every
-    // row moves by one dword.  Where a thread stages one chunk (16-bit storage,
-    // r = 1) it is loaded at every third offset only, with the eight columns
-    // behind it, and the next two offsets read the same registers one and two
-    // dwords further on, named by three copies of the code; R likewise.  The
-    // texture addresser and data return were busy all the time (two loads a
-    // step for 33 vector instructions): FP16, 3102 offsets of 411x377x203,
-    // 51.1 -> 44.8 ms.
-    constexpr bool kMove = !PRUNED && sizeof(TS) == 2 && S8 == 1 && S4 == 0;
+    // RUNS (runs_pay): along a run of the full search (one dz and dy, dx
+    // stepping by 2) every row moves by one dword.  The one chunk a thread
+    // stages (16-bit storage, r = 1) is loaded at every third offset only,
+    // with the eight columns behind it, and the next two offsets read the same
+    // registers one and two dwords further on, named by three copies of the
+    // code; R likewise.  The texture addresser and data return were busy all
+    // the time (two loads a step for 33 vector instructions): FP16, 3102
+    // offsets of 411x377x203, 51.1 -> 44.8 ms.
+    constexpr bool kMove = RUNS;
+    static_assert(!RUNS || (!PRUNED && sizeof(TS) == 2 && S8 == 1 && S4 == 0), "one 16-bit chunk per thread");
     chunk8 pn8[S8 > 0 ? S8 : 1], pt8[1];
     chunk4 pn4[S4 > 0 ? S4 : 1];
     auto load_chunks = [&](int lin) __attribute__((always_inline)) {
@@ -2150,10 +2151,30 @@ void fp8_tables_plan(const unsigned char (*codes)[8], A &a)
         }
 }
 
+// Whether the row kernel at r = 1 loads along runs of the search: `loads` of
+// its n offsets begin one.  The moves' branches lengthen each step, so there
+// must be loads to save and enough workgroups to hide them (768 run at once).
+// A load per offset against runs, in us:
+//   FP16, 2046 offsets: 64x64x32 626 / 983, 160x128x128 2595 / 2616,
+//     192x192x96 (1728 tiles) 3720 / 3574, 300x300x203 20857 / 18001;
+//   FP16, 300x300x160: radii 2 (32 offsets, 0.72 loads) 312 / 349, 1,10,10
+//     (0.99) 1743 / 1837, 3 (114, 0.49) 933 / 883, 10,1,1 (24, 0.5) 262 / 275;
+//   BF16 stages with more vector work, and gains late: 2046 offsets of
+//     192x192x96 3911 / 4050, 256x192x128 (3072 tiles) 6614 / 6576,
+//     300x300x203 21342 / 20686; 514 offsets of 300x300x160 4035 / 4074.
+// FP8 planes lose at every size (2046 offsets of 300x300x203: 21.2 / 22.8 ms).
+template <class TS, class TD>
+bool runs_pay(long tiles, int n, int loads)
+{
+    if (sizeof(TS) != 2 || !std::is_same<TD, _Float16>::value) return false;
+    const bool bf16 = std::is_same<TS, __bf16>::value;
+    return 2L * loads <= n && n >= (bf16 ? 1000 : 64) && tiles >= (bf16 ? 4096 : 1536);
+}
+
 template <int R, class TS, class TD, int WFN>
 hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shifted, const float *raw, float *out,
                          const float *sigma, float beta, float mscale, double shift, double inv_scale,
-                         const SearchEntry *search, const SearchEntry *search_full, int n_search, int min_lin,
+                         const SearchEntry *search, const SearchEntry *search_full, int n_search, int loads, int min_lin,
                          const TapTable &taps, const FilterGeom &g, const OffsetLists *ol, bool row_form,
                          hipStream_t st)
 {
@@ -2234,6 +2255,13 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
         }
     }
     const dim3 grid((unsigned)nwg), block(NTM);
+    if constexpr (R == 1 && sizeof(TS) == 2 && std::is_same<TD, _Float16>::value) {
+        if (!ol && runs_pay<TS, TD>(nwg, n_search, loads)) {
+            if (iso) hipLaunchKernelGGL((filter_mfma<R, TS, TD, WFN, false, true, true>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((filter_mfma<R, TS, TD, WFN, false, false, true>), grid, block, 0, st, a);
+            return hipGetLastError();
+        }
+    }
     if (ol && iso) hipLaunchKernelGGL((filter_mfma<R, TS, TD, WFN, true, true>), grid, block, 0, st, a);
     else if (ol) hipLaunchKernelGGL((filter_mfma<R, TS, TD, WFN, true, false>), grid, block, 0, st, a);
     else if (iso) hipLaunchKernelGGL((filter_mfma<R, TS, TD, WFN, false, true>), grid, block, 0, st, a);
@@ -2245,23 +2273,23 @@ template <int R, int WFN>
 hipError_t launch_mfma_form(int form, const void *Rs, const void *Ps, size_t elems, long shifted, const float *raw,
                             float *out,
                             const float *sigma, float beta, float mscale, double shift, double inv_scale,
-                            const SearchEntry *search, const SearchEntry *search_full, int n_search, int min_lin,
+                            const SearchEntry *search, const SearchEntry *search_full, int n_search, int loads, int min_lin,
                             const TapTable &taps, const FilterGeom &g, const OffsetLists *ol, bool row_form,
                             hipStream_t st)
 {
     switch (form) {
     case FORM_FP32_FAST:
         return launch_mfma_t<R, float, _Float16, WFN>(Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift,
-                                                      inv_scale, search, search_full, n_search, min_lin, taps, g, ol, row_form, st);
+                                                      inv_scale, search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st);
     case FORM_FP16:
         return launch_mfma_t<R, _Float16, _Float16, WFN>(Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift,
-                                                         inv_scale, search, search_full, n_search, min_lin, taps, g, ol, row_form, st);
+                                                         inv_scale, search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st);
     case FORM_FP16_FP8:
         return launch_mfma_t<R, _Float16, f8_t, WFN>(Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift,
-                                                     inv_scale, search, search_full, n_search, min_lin, taps, g, ol, row_form, st);
+                                                     inv_scale, search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st);
     case FORM_BF16:
         return launch_mfma_t<R, __bf16, _Float16, WFN>(Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift,
-                                                     inv_scale, search, search_full, n_search, min_lin, taps, g, ol, row_form, st);
+                                                     inv_scale, search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -2282,15 +2310,15 @@ bool mfma_taps_supported(int rp, const int *dxyz, const float *w, int n)
 hipError_t launch_filter_mfma(int form, int rp, int weight_fn, const void *Rs, const void *Ps, size_t elems,
                               long shifted, const float *raw, float *out, const float *sigma, float beta, float mscale,
                               double shift, double inv_scale, const SearchEntry *search,
-                              const SearchEntry *search_full, int n_search, int min_lin, const TapTable &taps,
+                              const SearchEntry *search_full, int n_search, int loads, int min_lin, const TapTable &taps,
                               const FilterGeom &g, hipStream_t st, const OffsetLists *ol, bool row_form)
 {
     if (min_lin > 0) return hipErrorInvalidValue;
 #define INLM_MF(RR)                                                                                               \
     return weight_fn == 0 ? launch_mfma_form<RR, 0>(form, Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift, inv_scale, \
-                                                    search, search_full, n_search, min_lin, taps, g, ol, row_form, st)                       \
+                                                    search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st)                       \
                           : launch_mfma_form<RR, 1>(form, Rs, Ps, elems, shifted, raw, out, sigma, beta, mscale, shift, inv_scale, \
-                                                    search, search_full, n_search, min_lin, taps, g, ol, row_form, st)
+                                                    search, search_full, n_search, loads, min_lin, taps, g, ol, row_form, st)
     switch (rp) {
     case 1: INLM_MF(1);
     case 2: INLM_MF(2);

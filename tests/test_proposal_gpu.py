@@ -325,6 +325,63 @@ def test_radius1_runs_equal_a_load_per_offset(gpu_available, form, weight_fn, sh
     assert np.array_equal(outs[0], outs[1])
 
 
+def _whole_search(shape, rs, form, weight_fn, lists, repeats=1):
+    """One iteration at patch radius 1 over the whole search, by the
+    full-search kernel or by per-tile lists that hold all of it (a load per
+    offset, in the same order): the result and the best time in ms."""
+    nx, ny, nz = shape
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(nx)
+    vol = 20000.0 + 1500.0 * torch.randn((nz, ny, nx), generator=gen, device="cuda")
+    vol[:, ny // 2:] += 8000.0
+    torch.cuda.synchronize()
+    p = DenoiseParameters(radius_searchspace=list(rs), radius_patchspace=[1] * 3, precision=form, weight_fn=weight_fn)
+    g = IterativeNLM_GPU()
+    assert g.configure_device(list(shape), p) == nz
+    g.load_raw_device(vol.data_ptr())
+    g.set_sigma(np.linspace(600.0, 900.0, nz).astype(np.float32))
+    if lists:
+        ns, nt = g.table_sizes()[0], g.tile_count()
+        g.set_offset_lists(np.zeros((nt, 1), np.int32), np.full(nt, ns, np.int32), 1)
+    ms = []
+    for _ in range(repeats):
+        g.Run_GaussianNoise(1)
+        ms.append(g.last_filter_ms())
+    out = torch.empty_like(vol)
+    g.get_result_device(out.data_ptr())
+    g.free_device()
+    return out, min(ms)
+
+
+@pytest.mark.parametrize("form,shape,rs", [("fp16", (321, 130, 137), (5, 4, 3)), ("fp16", (330, 131, 140), (4, 3, 1)),
+                                           ("bf16", (501, 300, 90), (7, 7, 5)), ("bf16", (640, 296, 96), (9, 7, 5))])
+@pytest.mark.parametrize("weight_fn", ["pade", "exp"])
+def test_radius1_runs_on_large_volumes_equal_a_load_per_offset(gpu_available, form, shape, rs, weight_fn):
+    """Volumes and searches large enough for the runs to pay (FP16 from 1536
+    tiles and 64 offsets, BF16 from 4096 and 1000): the same order of sums."""
+    print(f"[gpu] r=1 runs {form} {weight_fn} {shape} rs={rs}", flush=True)
+    runs, _ = _whole_search(shape, rs, form, weight_fn, False)
+    ref, _ = _whole_search(shape, rs, form, weight_fn, True)
+    assert torch.equal(runs, ref)
+
+
+@pytest.mark.parametrize("form,shape,rs", [("fp16", (64, 64, 32), (7, 7, 5)), ("bf16", (64, 64, 32), (7, 7, 5)),
+                                           ("fp16_fp8", (64, 64, 32), (7, 7, 5)), ("fp16", (200, 192, 96), (1, 10, 10)),
+                                           ("bf16", (200, 192, 96), (1, 10, 10))])
+def test_radius1_small_or_without_runs_costs_a_load_per_offset(gpu_available, form, shape, rs):
+    """Where the runs do not pay, the full search is no slower than the lists
+    of the whole search: equal but for the lists' look-ups (run moves took 1.3
+    to 1.6 times as long here; the bound is 1.15)."""
+    ratio = 9.0
+    for _ in range(3):  # the two in turn, the best of three
+        a, t = _whole_search(shape, rs, form, "pade", False, 8)
+        b, u = _whole_search(shape, rs, form, "pade", True, 8)
+        print(f"[gpu] r=1 {form} {shape} rs={rs}: full {t:.4f} ms, lists {u:.4f} ms", flush=True)
+        ratio = min(ratio, t / u)
+        assert torch.equal(a, b)
+    assert ratio < 1.15, ratio
+
+
 @pytest.mark.parametrize("form", ["fp16", "fp16_fp8"])
 def test_proposal_fallback_audit_and_topk(gpu_available, form):
     spec = ph.PhantomSpec((64, 32, 24), seed=81, radii=(2, 7), streaks=3, streak_len=(5, 15))
