@@ -1500,7 +1500,7 @@ __device__ __forceinline__ float b4_weight(const MfmaArgs<TS> &a, int dx, int dy
 // The full search's loop holds up to 128 registers: two workgroups per CU (4
 // waves per SIMD); so does the lists' form (105 registers; at 6 waves per SIMD
 // it spills 17 to 30).
-template <class TS, bool PRUNED>
+template <class TS, bool PRUNED, bool RUNS>
 __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 filter_mfma_b4(MfmaArgs<TS> a)
 {
@@ -1652,7 +1652,8 @@ filter_mfma_b4(MfmaArgs<TS> a)
     // vector instructions (the masked ones took a slot too): lists of 128
     // offsets, BF16, 640x640x256: 12.1 -> 11.9 ms a call; the full search the
     // same within 0.3%.
-        constexpr bool kMove = std::is_same<TS, _Float16>::value && !PRUNED;
+    static_assert(!PRUNED || !RUNS, "lists are no runs");
+    constexpr bool kMove = std::is_same<TS, _Float16>::value && RUNS;
     chunk8 pnA, pnX;
     typedef std::conditional_t<kMove, ST8, ST4> STT;
     const STT stt{};
@@ -1715,7 +1716,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
     // loaded offset, of which it and the next two along its run read four
     // each, named by three copies of the sums (FP16, 1326 offsets of
     // 1024x1024x512: 391 -> 385 ms against a load at every offset)
-    constexpr bool kMoveR = !PRUNED;
+    constexpr bool kMoveR = RUNS;
     struct RVals {
         unsigned v[b4::NH][kMoveR ? 4 : 2];
     };
@@ -2242,7 +2243,7 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
     if constexpr (R == 2 && sizeof(TS) == 2 && std::is_same<TD, _Float16>::value && WFN == 0) {
         if (!row_form && -(long)min_lin < (1L << 29)) {
             if (ol) {  // one 32x8x8 tile, the lists' own, per workgroup
-                hipLaunchKernelGGL((filter_mfma_b4<TS, true>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
+                hipLaunchKernelGGL((filter_mfma_b4<TS, true, false>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
                 return hipGetLastError();
             }
             using B = B4<16>;
@@ -2250,7 +2251,17 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
             a.nty = (g.ny + B::TY - 1) / B::TY;
             a.ntz = (g.nz + B::TZ - 1) / B::TZ;
             const long nb = (long)a.ntx * a.nty * a.ntz;
-            hipLaunchKernelGGL((filter_mfma_b4<TS, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
+            // Loads along runs, where the search has some and the chip is full
+            // (two workgroups per CU): the moves' branches lengthen a step. A
+            // load per offset against runs, us: FP16, 300x300x160, radii
+            // 1,10,10 (0.99 of the offsets load) 2012 / 2159, 2 (0.72) 377 /
+            // 369, 7,7,5 (0.4) 9.6 / 9.0 ms; 1022 offsets of 128x128x64 (256
+            // workgroups) 679 / 827, 160x128x100 (520) 1986 / 1941; BF16 the
+            // same way (788 / 865, 2223 / 2133).
+            if (4L * loads <= 3L * n_search && nb >= 512)
+                hipLaunchKernelGGL((filter_mfma_b4<TS, false, true>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
+            else
+                hipLaunchKernelGGL((filter_mfma_b4<TS, false, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
             return hipGetLastError();
         }
     }
