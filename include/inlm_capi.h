@@ -109,8 +109,7 @@ typedef struct inlm_params {
     /* FP32 form: 0 the tiled kernel where one covers the patch, 1 the
      * per-voxel kernel.  Matrix-core forms: 0 the fastest kernel for the
      * case (at patch radius 2 with 16-bit storage and FP16 planes, the
-     * 4x4-block kernel, for the full search and per-tile lists), 2 the row
-     * kernel. */
+     * 4x4-block kernel for the full search), 2 the row kernel. */
     int32_t kernel_select;
     /* NoiseLevel.circular_mask_diameter (denoise_parameters.h:33): when > 0
      * noise samples are drawn only inside that circle around the slice

@@ -20,8 +20,8 @@
 // forms, full search and per-tile lists): a workgroup (8 wavefronts) owns a
 // 32x8x8 output tile and stages D_s over the tile plus the patch halo in LDS
 // (double buffered, one barrier per offset); wavefront w computes the 16x16
-// block x-half (w & 1), z pair (w >> 1).  At patch radius 2 the 16-bit forms
-// run the block form (filter_mfma_b4, further below).
+// block x-half (w & 1), z pair (w >> 1).  The full search at patch radius 2
+// in the 16-bit forms runs the block form (filter_mfma_b4, further below).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1430,9 +1430,8 @@ void filter_mfma(MfmaArgs<TS> a)
 #ifndef INLM_B4_KD
 #define INLM_B4_KD 2
 #endif
-template <int TY_>
 struct B4 {
-    static constexpr int TX = 32, TY = TY_, TZ = 8;
+    static constexpr int TX = 32, TY = 16, TZ = 8;
     static constexpr int NH = TY / 8;  // 32x8 output halves per wavefront
     static constexpr int RX = TX + 4, RY = TY + 4, RZ = TZ + 4;  // staged region
     static constexpr int ROW = 64;                               // LDS row pitch, halves (8 windows)
@@ -1459,32 +1458,6 @@ struct B4 {
     static constexpr int kOff[NOPS] = {-2 * ROW, 2 * ROW, SLICE - ROW, -SLICE - ROW, 0, 2 * SLICE, -2 * SLICE};
 };
 
-// The patch weights by (|dz|, |dy|, dx + 2) for the lists' form, whose tiles run
-// few steps: its lanes read them from LDS, where the argument block is read
-// through the vector cache, one wait per weight.  (In the full search's form
-// the table costs a register in the loop, 4% of the pass.)
-__device__ __forceinline__ void b4_weight_table(const float (&band)[kMfmaMaxPatterns][8], float *tab)
-{
-    constexpr const MRows<2> &rows = MRowsOf<2>::value;
-    const int t = threadIdx.x;
-    if (t < 45) {
-        const int adz = t / 15, ady = t / 5 % 3, dx = t % 5 - 2;
-        int at = -1;
-#pragma unroll
-        for (int p = 0; p < rows.npat; p++)
-            if (rows.pdy[p] == ady && rows.pdz[p] == adz && dx >= -rows.pj[p] && dx <= rows.pj[p]) at = p * 8 + dx + 2;
-        const float w = (&band[0][0])[at >= 0 ? at : 0];
-        tab[t] = at >= 0 ? w : 0.f;
-    }
-}
-__device__ __forceinline__ float b4_table_weight(const float *tab, int dx, int dy, int dz)
-{
-    const int ady = dy < 0 ? -dy : dy, adz = dz < 0 ? -dz : dz;
-    const bool in = dx >= -2 && dx <= 2 && ady <= 2;
-    const float w = tab[in ? adz * 15 + ady * 5 + dx + 2 : 0];
-    return in ? w : 0.f;
-}
-
 template <class TS>
 __device__ __forceinline__ float b4_weight(const MfmaArgs<TS> &a, int dx, int dy, int dz)
 {
@@ -1497,20 +1470,21 @@ __device__ __forceinline__ float b4_weight(const MfmaArgs<TS> &a, int dx, int dy
     return w;
 }
 
-// The full search's loop holds up to 128 registers: two workgroups per CU (4
-// waves per SIMD); so does the lists' form (105 registers; at 6 waves per SIMD
-// it spills 17 to 30).
-template <class TS, bool PRUNED, bool RUNS>
+// Its loop holds up to 128 registers: two workgroups per CU (4 waves per SIMD).
+// Per-tile lists stay with the row kernel: on 32x8x8 tiles this kernel took 5 to
+// 11% less for them, but its sums run in another FP32 order, and a distance
+// moved over an FP16 rounding limit changed single voxels by up to 1.1 noise
+// levels (FP16, 256 offsets, 640x640x256).
+template <class TS, bool RUNS>
 __global__ __launch_bounds__(NTM) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 filter_mfma_b4(MfmaArgs<TS> a)
 {
-    using b4 = B4<PRUNED ? 8 : 16>;
+    using b4 = B4;
     using ST8 = Stager<8, TS, _Float16>;
     using ST4 = Stager<4, TS, _Float16>;
     typedef typename ST8::chunk chunk8;
     typedef typename ST4::chunk chunk4;
     __shared__ __attribute__((aligned(16))) _Float16 lds[2][b4::LDS];
-    __shared__ float wtab[PRUNED ? 45 : 1];
 
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -1525,10 +1499,6 @@ filter_mfma_b4(MfmaArgs<TS> a)
     const long sp = (long)g.nxp * g.nyp;
 
     for (int i = t; i < (int)(sizeof(lds) / 4); i += NTM) reinterpret_cast<unsigned *>(&lds[0][0])[i] = 0u;
-    if constexpr (PRUNED) {
-        b4_weight_table(a.band, wtab);
-        __syncthreads();
-    }
 
     // A operands: lane l holds row m = l % 16 (output bx = m & 3, by = m >> 2)
     // of K group q = l / 16
@@ -1541,10 +1511,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
             const int o = b4::kClsOp[c];
             const int dz = b4::op_dz(o, q), row = b4::op_row(o, q);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                if constexpr (PRUNED) aop[c][i] = (_Float16)b4_table_weight(wtab, i - 2 - mx, row - my, dz);
-                else aop[c][i] = (_Float16)b4_weight(a, i - 2 - mx, row - my, dz);
-            }
+            for (int i = 0; i < 8; i++) aop[c][i] = (_Float16)b4_weight(a, i - 2 - mx, row - my, dz);
         }
     }
 
@@ -1649,10 +1616,8 @@ filter_mfma_b4(MfmaArgs<TS> a)
     // search instead of loading them at every offset (below).  Only the
     // row's last lane (cg = 3) needs columns no other lane holds, but with a
     // tail of its own in every lane the staging exchanges no lanes, in as many
-    // vector instructions (the masked ones took a slot too): lists of 128
-    // offsets, BF16, 640x640x256: 12.1 -> 11.9 ms a call; the full search the
-    // same within 0.3%.
-    static_assert(!PRUNED || !RUNS, "lists are no runs");
+    // vector instructions (the masked ones took a slot too): the same time
+    // within 0.3%.
     constexpr bool kMove = std::is_same<TS, _Float16>::value && RUNS;
     chunk8 pnA, pnX;
     typedef std::conditional_t<kMove, ST8, ST4> STT;
@@ -1756,8 +1721,7 @@ filter_mfma_b4(MfmaArgs<TS> a)
 #pragma unroll
         for (int h = 0; h < b4::NH; h++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-            {
+            for (int i = 0; i < 4; i++) {
                 typedef TS pair __attribute__((ext_vector_type(2)));
                 const pair r = __builtin_bit_cast(pair, rv.v[h][(i >> 1) + S]);
                 fv[h][i] = __builtin_fmaf((float)w[h][i >> 1][i & 1], (float)r[i & 1], fv[h][i]);
@@ -1777,30 +1741,11 @@ filter_mfma_b4(MfmaArgs<TS> a)
         }
     };
 
-    // offsets this tile visits: the whole search, or its list (32x8x8 tiles)
-    int nS = a.n_search;
-    const int *lst = nullptr;
-    if constexpr (PRUNED) {
-        const int c = a.counts[wg];
-        if (c >= 1 && c < nS) {
-            nS = c;
-            lst = a.lists + (long)wg * a.K;
-        }
-    }
-    auto lin_at = [&](int k) __attribute__((always_inline)) {
-        const int i = k < nS ? k : nS - 1;
-        if constexpr (PRUNED) {
-            if (lst) {
-                const unsigned e = (unsigned)lst[i];
-                return a.search[e < (unsigned)a.n_search ? e : 0u].lin;
-            }
-        }
-        return a.search_full[i].lin;
-    };
-    // per offset of the full search, after the table: 0 to load
-    // the chunks, s > 0 to read the loaded ones moved by s dwords
-    // (kStageMovesMax)
-    const int *moves = reinterpret_cast<const int *>(a.search_full + a.n_search);
+    const int nS = a.n_search;
+    auto lin_at = [&](int k) __attribute__((always_inline)) { return a.search_full[k < nS ? k : nS - 1].lin; };
+    // per offset of the full search, after the table: 0 to load the chunks,
+    // s > 0 to read the loaded ones moved by s dwords (kStageMovesMax)
+    const int *moves = reinterpret_cast<const int *>(a.search_full + nS);
     auto loads = [&](int mv) __attribute__((always_inline)) { return !kMove || mv == 0; };
 
     // Software pipeline as in filter_mfma: step k runs the MFMA chain of
@@ -2235,18 +2180,13 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
         if (iso) fp8_tables_plan<R, true>(codes, a);
         else fp8_tables_plan<R, false>(codes, a);
     }
-    // the block form (lists of 128 offsets over 640x640x256: FP16 9.9 ms, BF16
-    // 10.8 ms; the row form 11.2 and 11.5): full search or lists at patch radius 2, 16-bit storage,
-    // FP16 planes, Pade weights; it packs lin * 4 + moves into one int, so |lin|
+    // the block form: full search at patch radius 2, 16-bit storage, FP16
+    // planes, Pade weights; it packs lin * 4 + moves into one int, so |lin|
     // stays below 2^29 (the search space is symmetric: the largest lin is
     // -min_lin); beyond that the row form runs
     if constexpr (R == 2 && sizeof(TS) == 2 && std::is_same<TD, _Float16>::value && WFN == 0) {
-        if (!row_form && -(long)min_lin < (1L << 29)) {
-            if (ol) {  // one 32x8x8 tile, the lists' own, per workgroup
-                hipLaunchKernelGGL((filter_mfma_b4<TS, true, false>), dim3((unsigned)nwg), dim3(NTM), 0, st, a);
-                return hipGetLastError();
-            }
-            using B = B4<16>;
+        if (!ol && !row_form && -(long)min_lin < (1L << 29)) {
+            using B = B4;
             a.ntx = (g.nx + B::TX - 1) / B::TX;
             a.nty = (g.ny + B::TY - 1) / B::TY;
             a.ntz = (g.nz + B::TZ - 1) / B::TZ;
@@ -2259,9 +2199,9 @@ hipError_t launch_mfma_t(const void *Rs, const void *Ps, size_t elems, long shif
             // workgroups) 679 / 827, 160x128x100 (520) 1986 / 1941; BF16 the
             // same way (788 / 865, 2223 / 2133).
             if (4L * loads <= 3L * n_search && nb >= 512)
-                hipLaunchKernelGGL((filter_mfma_b4<TS, false, true>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
+                hipLaunchKernelGGL((filter_mfma_b4<TS, true>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
             else
-                hipLaunchKernelGGL((filter_mfma_b4<TS, false, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
+                hipLaunchKernelGGL((filter_mfma_b4<TS, false>), dim3((unsigned)nb), dim3(NTM), 0, st, a);
             return hipGetLastError();
         }
     }

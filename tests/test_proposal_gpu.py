@@ -325,6 +325,44 @@ def test_radius1_runs_equal_a_load_per_offset(gpu_available, form, weight_fn, sh
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("form", ["fp16", "bf16"])
+@pytest.mark.parametrize("K", [40, 128])
+def test_lists_at_patch_radius_2_run_the_row_kernel(gpu_available, form, K):
+    """Lists keep the row kernel's order of FP32 sums at every patch radius:
+    attenuation-like values around a zero background, with and without
+    kernel_select 2, are equal to the bit.  (The block kernel's order moves
+    distances over FP16 rounding limits: one voxel in a thousand differed,
+    some by a whole noise level.)"""
+    nx, ny, nz = shape = (200, 160, 60)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K)
+    f = torch.nn.functional.interpolate(torch.rand((1, 1, 6, 14, 16), generator=gen, device="cuda"), size=(nz, ny, nx),
+                                        mode="trilinear", align_corners=True)[0, 0]
+    vol = 0.4 * (f > 0.55).float() + 0.05 * f + 0.02 * torch.randn((nz, ny, nx), generator=gen, device="cuda")
+    torch.cuda.synchronize()
+    rng = np.random.default_rng(K)
+    outs = []
+    lists = None
+    for ks in (0, 2):
+        print(f"[gpu] lists {form} K={K} kernel_select {ks}", flush=True)
+        p = DenoiseParameters(radius_searchspace=[5, 5, 4], radius_patchspace=[2, 2, 2], precision=form, kernel_select=ks)
+        g = IterativeNLM_GPU()
+        assert g.configure_device(list(shape), p) == nz
+        nt, ns = g.tile_count(), g.table_sizes()[0]
+        if lists is None:
+            lists = np.stack([np.sort(rng.permutation(ns)[:K]) for _ in range(nt)]).astype(np.int32)
+            counts = np.resize(np.array([K, ns, 1, K - 1], np.int32), nt)
+        g.load_raw_device(vol.data_ptr())
+        g.set_sigma(np.full(nz, 0.02, np.float32))
+        g.set_offset_lists(lists, counts, K)
+        g.Run_GaussianNoise(1)
+        out = torch.empty_like(vol)
+        g.get_result_device(out.data_ptr())
+        outs.append(out)
+        g.free_device()
+    assert torch.equal(outs[0], outs[1])
+
+
 def _whole_search(shape, rs, form, weight_fn, lists, repeats=1):
     """One iteration at patch radius 1 over the whole search, by the
     full-search kernel or by per-tile lists that hold all of it (a load per
