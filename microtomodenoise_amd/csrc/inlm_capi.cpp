@@ -440,8 +440,10 @@ inlm_status inlm_create(const inlm_params *pin, const int32_t shape_in[3], int32
             return fail(nullptr, INLM_BAD_ARG, "the matrix-core forms need an isotropic patch of radius 1, 2 or 3");
         }
         h->rp_tiled = rp[0];
-    } else if (p.kernel_select == 0)
-        h->tiled = inlm::tiled_shape(rp, h->tap_dxyz.data(), h->taps.w, h->taps.n);
+    } else if (p.kernel_select == 0) {
+        const int s = inlm::tiled_shape(rp, h->tap_dxyz.data(), h->taps.w, h->taps.n);
+        if (s != 0 && inlm::tiled_pays(s, shape[0], shape[1], shape[2])) h->tiled = s;
+    }
 
     inlm_status st = INLM_OK;
     auto bail = [&](inlm_status s) {

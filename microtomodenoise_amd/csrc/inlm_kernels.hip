@@ -1356,6 +1356,28 @@ int tiled_shape(const int rp[3], const int *dxyz, const float *w, int n)
     return 0;
 }
 
+// Tiles compute whole, so a volume thinner than its tiles pays for the rest;
+// the per-voxel kernel does not.  Per-voxel against tiled, us:
+//   221 of 1024x1024x2 (a quarter of each tile) 2109 / 2028, 332 of it 11032 /
+//   5295; 220 of 256 slices of 1024x16 3501 / 3442, of 1024x8 (an eighth) 1835
+//   / 3420; 330 of 1024x8 3757 / 5228.  Up to 512 tiles the waste costs
+//   nothing, they run at once: 220 of 64 slices of 256x8 280 / 254.  Narrow
+//   rows cost the per-voxel kernel as much: 220 of 64 slices of 2x4096 4734 /
+//   1666.
+//   The five taps of 110 leave the tiles less to share: 1024x16 1589 / 2413,
+//   1024x32 3047 / 2420, 512 slices of 8x64 136 / 186, of 16x64 206 / 186, one
+//   slice of 300x300 52.4 / 54.4, of 512x512 60.0 / 54.2.
+bool tiled_pays(int shape, int nx, int ny, int nz)
+{
+    const int rx = shape / 100, ry = shape / 10 % 10, rz = shape % 10;
+    if (rx == ry && rx == rz) return true;  // 32x8x8 tiles at every size
+    const int tz = rz == 0 ? 1 : 8, ty = rz == 0 ? 64 : 8;
+    auto tiles = [](long n, long t) { return (n + t - 1) / t; };
+    auto fill = [&](long n, long t) { return (double)n / (double)(tiles(n, t) * t); };
+    if (shape == 110) return (long)nx * ny * nz >= (1L << 17) && fill(nx, TX) >= 0.4 && fill(ny, ty) >= 0.4;
+    return tiles(nx, TX) * tiles(ny, ty) * tiles(nz, tz) <= 512 || fill(ny, ty) * fill(nz, tz) >= 0.2;
+}
+
 hipError_t launch_pad_reflect(const float *in, float *out, const FilterGeom &g, hipStream_t st)
 {
     const long n = (long)g.nxp * g.nyp * g.nzp;

@@ -60,6 +60,10 @@ hipError_t launch_filter_rgb(int shape, int weight_fn, const float *const R[3], 
 // with one weight per class of taps; 0 when there is none.
 int tiled_shape(const int rp[3], const int *dxyz, const float *w, int n);
 
+// Whether a shape's tiled kernel is at least as quick as the per-voxel one on
+// a volume of this size.
+bool tiled_pays(int shape, int nx, int ny, int nz);
+
 // Exhaustive check of the parity kernel's division: counts weights that
 // differ from IEEE division over the float bit patterns 0x80000000+[first,
 // first+count).

@@ -102,6 +102,53 @@ def test_tiled_shapes_at_tile_edges(gpu_available, rp, shape):
             assert np.array_equal(bits(outs[0]), bits(ref))
 
 
+@pytest.mark.parametrize("rp,shape", [((1, 1, 0), (641, 257, 1)), ((1, 1, 0), (95, 700, 2)), ((2, 2, 0), (130, 40, 210)),
+                                      ((3, 3, 0), (130, 15, 210)), ((2, 2, 1), (331, 300, 2))])
+def test_tiled_shapes_beyond_512_tiles(gpu_available, rp, shape):
+    """Either side of the rule by which thin volumes keep the per-voxel
+    kernel; 110 runs tiled from 2^17 voxels on."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx + ny)
+    raw = (rng.normal(size=(nz, ny, nx)) * 400 + 5000).astype(np.float32)
+    raw[:, ny // 2:] += 3000
+    sig = np.linspace(500, 900, nz).astype(np.float32)
+    outs = []
+    for kernel in (0, 1):
+        print(f"[gpu] shape {shape} rp={rp} kernel={kernel}", flush=True)
+        g, _ = make_gpu(shape, (3, 2, min(1, nz - 1)), rp, kernel=kernel)
+        g.set_sigma(sig)
+        g.Run_GaussianNoise(1, raw)
+        g.Run_GaussianNoise(2)
+        outs.append(g.get_result())
+        g.free_device()
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
+
+
+@pytest.mark.parametrize("rp,shape", [((1, 1, 0), (512, 8, 256)), ((1, 1, 0), (256, 16, 64)), ((1, 1, 0), (8, 64, 512)),
+                                      ((2, 2, 0), (1024, 8, 256)), ((3, 3, 0), (1024, 8, 256))])
+def test_thin_volumes_cost_no_more_than_the_per_voxel_kernel(gpu_available, rp, shape):
+    """Flat patches on volumes that fill a small part of their 32x64 tiles
+    (tiled, these took 1.3 to 2.8 times the per-voxel kernel's time)."""
+    nx, ny, nz = shape
+    raw = (np.random.default_rng(nx).normal(size=(nz, ny, nx)) * 400 + 5000).astype(np.float32)
+    ratio = 9.0
+    for _ in range(3):  # the two in turn, the best of three
+        ms = {}
+        for kernel in (0, 1):
+            g, _ = make_gpu(shape, (5, 5, 2), rp, kernel=kernel)
+            g.load_raw(raw)
+            g.set_sigma(np.full(nz, 400.0, np.float32))
+            t = []
+            for _ in range(8):
+                g.Run_GaussianNoise(1)
+                t.append(g.last_filter_ms())
+            ms[kernel] = min(t)
+            g.free_device()
+        print(f"[gpu] {rp} {shape}: {ms[0]:.4f} ms, per voxel {ms[1]:.4f} ms", flush=True)
+        ratio = min(ratio, ms[0] / ms[1])
+    assert ratio < 1.15, ratio
+
+
 @pytest.mark.parametrize("rp", [(1, 1, 1), (3, 3, 3), (2, 2, 0)])
 def test_infinite_and_nan_values_reach_the_same_voxels(gpu_available, rp):
     """A zero weight times an infinite value is a NaN in the sums, also where
