@@ -87,6 +87,18 @@ inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64
 
 size_t cluster_bytes(int nz) { return kClusterWorkBytes + (size_t)nz * 2 * (sizeof(int64_t) + sizeof(double)); }
 
+bool clusters_on_host(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n)
+{
+    if (p.noise_mode != INLM_NOISE_GLOBAL && p.noise_mode != INLM_NOISE_ZADAPTIVE) return true;
+    if (n > kHostClusterSamples) return false;  // every sample lies in a window
+    if (p.noise_mode == INLM_NOISE_GLOBAL || n <= 0) return true;
+    std::vector<int64_t> bounds;
+    zwindow_bounds(samples, n, shape, p.zwindow, bounds);
+    int64_t total = 0;
+    for (size_t i = 0; i < bounds.size(); i += 2) total += bounds[i + 1] - bounds[i] + 1;
+    return total <= kHostClusterSamples;
+}
+
 inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,
                             const double *std_dev, void *work, hipStream_t st, float *sig, std::string &err)
 {
@@ -802,9 +814,8 @@ inlm_status inlm_estimate_noise(inlm_handle *h, int32_t which, const int64_t *sa
     if (!h || !sigma_out) return fail(h, INLM_BAD_ARG, "null argument");
     int shape[3] = {h->geo.nx, h->geo.ny, h->geo.nz};
     std::string err;
-    if (n > 0 && (h->p.noise_mode == INLM_NOISE_GLOBAL || h->p.noise_mode == INLM_NOISE_ZADAPTIVE)) {
-        // the sample statistics stay on the GPU
-        if (!samples) return fail(h, INLM_BAD_ARG, "null argument");
+    if (!samples && n > 0 && h->p.noise_mode != INLM_NOISE_MANUAL) return fail(h, INLM_BAD_ARG, "null argument");
+    if (!inlm::clusters_on_host(h->p, shape, samples, n)) {  // the sample statistics stay on the GPU
         inlm_status s = patchstd_on_device(h, which, samples, n);
         if (s != INLM_OK) return s;
         if (!h->clusters_dev) HIP_TRY(h, hipMalloc(&h->clusters_dev, inlm::cluster_bytes(h->geo.nz)));

@@ -21,6 +21,15 @@ void set_global_error(const std::string &msg);
 inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64_t *samples, const double *sd,
                            int64_t n, int which, int64_t &semi_ref, float *sig, std::string &err);
 
+// Whether sigma_from_std is the quicker one: no clustering, or one whose
+// windows hold at most kHostClusterSamples in all (a sample of several windows
+// counts in each).  The GPU takes about 25 us more than the host for a few
+// samples, the host 35 us for 1000: an estimate of 300 samples in one window
+// takes 38 us by the host and 54 by the GPU, of 1000 57 to 70 and 60 to 68, of
+// 300 in the 16 windows of 5 slices of 64x64x16 (1500 in all) 65 and 62.
+constexpr int64_t kHostClusterSamples = 1024;
+bool clusters_on_host(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n);
+
 // The same in the global and z-adaptive modes from standard deviations on the
 // device (n >= 1), clustered there; work: cluster_bytes(nz) of device memory.
 // Returns when sig is written.

@@ -241,7 +241,7 @@ extern "C" inlm_status inlm_denoise_slabs(const inlm_params *p, const int32_t sh
         }
         const int sh[3] = {nx, ny, nz};
         std::string err;
-        if (ns > 0 && (p->noise_mode == INLM_NOISE_GLOBAL || p->noise_mode == INLM_NOISE_ZADAPTIVE)) {
+        if (!inlm::clusters_on_host(*p, sh, samples.data(), ns)) {
             DevBuf stds, work;
             hipError_t e = hipSetDevice(device);
             if (e == hipSuccess) e = hipMalloc(&stds.p, sizeof(double) * (size_t)ns);

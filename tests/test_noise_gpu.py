@@ -2,6 +2,8 @@
 semimanual mode (Noise/noiselevel.cpp:56-79) and the circular sampling mask
 (:204-224), against the oracle's FP64 estimator on the same sample list and
 the oracle's FP32 filter on the sigma lists the library used."""
+import time
+
 import numpy as np
 import pytest
 
@@ -117,3 +119,38 @@ def test_clustering_beyond_the_bits_in_lds(gpu_available):
     g.free_device()
     want = _capi.sigma_from_patchstd(p.to_c(), [nx, ny, nz], samples, stds)
     assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
+
+
+@pytest.mark.parametrize("mode,window,n", [("global", 0, 20), ("global", 0, 200), ("z-adaptive", 4, 50)])
+def test_few_samples_cost_no_more_than_the_host_clustering(gpu_available, mode, window, n):
+    """An estimate of a few samples takes the time of their patch statistics
+    and the host's clustering (1.3 to 1.8 times that when clustered on the
+    GPU), and gives its very result."""
+    raw = _noise_volume("plain")
+    nz, ny, nx = raw.shape
+    samples = _capi.draw_samples([nx, ny, nz], n, 15, 5)
+    p = DenoiseParameters(radius_searchspace=[2, 2, 2], radius_patchspace=[1, 1, 1])
+    p.noiselevel.mode = mode
+    p.noiselevel.zwindow = window
+    p.noiselevel.n_samples = n
+    g = IterativeNLM_GPU()
+    assert g.configure_device([nx, ny, nz], p) == nz
+    g.load_raw(raw)
+    c = p.to_c()
+
+    def whole():
+        return g.estimate_noise(samples)
+
+    def parts():
+        return _capi.sigma_from_patchstd(c, [nx, ny, nz], samples, g.patchstd(samples))
+
+    best = {whole: 1e9, parts: 1e9}
+    assert np.array_equal(whole(), parts())
+    for _ in range(300):
+        for f in best:
+            t = time.perf_counter()
+            f()
+            best[f] = min(best[f], time.perf_counter() - t)
+    g.free_device()
+    print(f"[gpu] {mode} n={n}: estimate {best[whole] * 1e6:.1f} us, parts {best[parts] * 1e6:.1f} us", flush=True)
+    assert best[whole] < 1.15 * best[parts], best
