@@ -1478,7 +1478,16 @@ hipError_t launch_filter_rgb(int shape, int weight_fn, const float *const R[3], 
     a.independent = independent;
     a.g = g;
     a.taps = taps;
-    if (g.nz == 1) {
+    // Few tiles leave each step's latency to show, which the three weights of
+    // independent channels lengthen: a call of four iterations and 316 offsets
+    // without noise estimate, us per pixel against tiled, joint (independent):
+    //   110: 64x64 1376 / 1709 (1429 / 2280), 256x200 1608 / 1813 (1660 / 2385),
+    //     4096x20 2010 / 1848 (2066 / 2400)
+    //   220: 64x64 2704 / 2453 (2785 / 3140), 256x200 3261 / 2600 (3265 / 3268)
+    //   330: 64x64 5.3 / 4.0 ms (5445 / 5683), 160x160 5.9 / 4.1 ms (5986 / 5710)
+    const long pixels = (long)g.nx * g.ny;
+    const long few = shape == 110 ? (independent ? 98304 : 65536) : !independent ? 0 : shape == 220 ? 32768 : 20480;
+    if (g.nz == 1 && pixels >= few) {
         switch (shape) {
         case 110: return launch_rgb_tiled<Patch<1, 1, 0>>(weight_fn, a, taps, st);
         case 220: return launch_rgb_tiled<Patch<2, 2, 0>>(weight_fn, a, taps, st);

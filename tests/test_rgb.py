@@ -11,6 +11,7 @@ volume filter at sigma * sqrt(3).  The GPU tests compare the HIP path with
 the oracle bit for bit (FP32) and the schedule with a restatement built on
 the oracle's filter."""
 import os
+import time
 
 import numpy as np
 import pytest
@@ -259,6 +260,38 @@ def test_filter_at_tile_edges(gpu_available, rp, shape, independent):
     ref = O.filter_rgb(img, img, list(log[0]), _op(5, rp), independent)
     ref = O.filter_rgb(img, ref, list(log[1]), _op(5, rp), independent)
     assert np.array_equal(_bits(out), _bits(ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rp,independent,pixels", [(1, False, 65536), (1, True, 98304), (2, True, 32768), (3, True, 20480)])
+@pytest.mark.parametrize("more", [-1, 0])
+def test_small_images_either_side_of_the_tiles(gpu_available, rp, independent, pixels, more):
+    """Per pixel below the rule's number of pixels, tiled from there on: the
+    oracle's bits on both sides."""
+    shape = (128 + more, pixels // 128)
+    img = _image(*shape, seed=9)
+    p = _rgb_params(2, rp, 1, sigma=(14.0, 9.0))
+    print(f"[gpu] rgb rp={rp} independent={independent} {shape}", flush=True)
+    out, _ = denoise_rgb(img, p, independent_channels=independent, stabilize_variance=False, average_channelsigma=False)
+    ref = O.filter_rgb(img, img, [14.0] * 3, _op(2, rp), independent)
+    assert np.array_equal(_bits(out), _bits(ref))
+
+
+@pytest.mark.gpu
+def test_independent_channels_of_a_small_image_run_per_pixel(gpu_available):
+    """A small image at radius 1: independent channels take about the joint
+    call's time (1.05 times it; tiled 1.33 times the tiled joint call's, 1.6
+    times the per-pixel one's)."""
+    img = _image(64, 64, seed=9)
+    p = _rgb_params(10, 1, 4, sigma=(14.0, 9.0))
+    best = {False: 1e9, True: 1e9}
+    for _ in range(60):
+        for independent in best:
+            t = time.perf_counter()
+            denoise_rgb(img, p, independent_channels=independent)
+            best[independent] = min(best[independent], time.perf_counter() - t)
+    print(f"[gpu] rgb 64x64: joint {best[False] * 1e6:.0f} us, independent {best[True] * 1e6:.0f} us", flush=True)
+    assert best[True] < 1.18 * best[False], best
 
 
 @pytest.mark.gpu
