@@ -154,3 +154,30 @@ def test_few_samples_cost_no_more_than_the_host_clustering(gpu_available, mode, 
     g.free_device()
     print(f"[gpu] {mode} n={n}: estimate {best[whole] * 1e6:.1f} us, parts {best[parts] * 1e6:.1f} us", flush=True)
     assert best[whole] < 1.15 * best[parts], best
+
+
+@pytest.mark.parametrize("shape,n", [((70, 40, 9), 700_001), ((70, 40, 9), 1_100_003), ((70, 40, 64), 1_100_003)])
+def test_large_windows_on_the_gpu_equal_the_host(gpu_available, shape, n):
+    """z windows of one list: 7e5 samples, whose bits take more than 64 KB of
+    LDS, and 1.1e6, for which the kernel derives the last assignment again
+    instead of keeping bits; the sums of a window's 6e5 terms differ by 1e-10
+    relative at most."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(7)
+    raw = rng.normal(size=(nz, ny, nx)).astype(np.float32) * 50 + 1000
+    raw[:, :, 35:] *= 40
+    samples = _capi.draw_samples([nx, ny, nz], n, 15, 5)
+    p = DenoiseParameters(radius_searchspace=[2, 2, 2], radius_patchspace=[1, 1, 1])
+    p.noiselevel.mode = "z-adaptive"
+    p.noiselevel.zwindow = 4
+    p.noiselevel.n_samples = n
+    print(f"[gpu] clustering {shape} n={n}", flush=True)
+    g = IterativeNLM_GPU()
+    assert g.configure_device([nx, ny, nz], p) == nz
+    g.load_raw(raw)
+    stds = g.patchstd(samples)
+    got = g.estimate_noise(samples)
+    g.free_device()
+    want = _capi.sigma_from_patchstd(p.to_c(), [nx, ny, nz], samples, stds)
+    assert np.unique(want).size > 1
+    assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
