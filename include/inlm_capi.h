@@ -272,11 +272,12 @@ INLM_API inlm_status inlm_iterate_slabs(const inlm_params *p, const int32_t shap
 INLM_API inlm_status inlm_tables(const inlm_params *p, const int32_t shape[3], int32_t cap, int32_t *n_search,
                                  int32_t *search_dxyz, int32_t *n_patch, int32_t *patch_dxyz, float *weights);
 
-/* Self-test of the division inside the FP32 parity kernel's Pade weight: on
- * `device`, evaluates the weight for every float exponent from -0 down to the
- * cutoff -3.56648 (about 1.08e9 values) with the kernel's division and with
- * IEEE division and counts the results that differ.  It has no counterpart
- * in the reference; it backs the bit-exactness claim of INLM_PREC_FP32. */
+/* Self-test of the FP32 kernels' divisions: on `device`, evaluates the Pade
+ * weight for every float exponent from -0 down to the cutoff -3.56648 (about
+ * 1.08e9 values) and the joint colour filter's third of every float (2^32)
+ * with the kernels' divisions and with IEEE division and counts the results
+ * that differ.  It has no counterpart in the reference; it backs the
+ * bit-exactness claims of INLM_PREC_FP32 and of the colour filter. */
 INLM_API inlm_status inlm_selftest_division(int32_t device, uint64_t *mismatches, uint64_t *checked,
                                             uint32_t *example);
 

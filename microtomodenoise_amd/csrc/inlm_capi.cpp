@@ -920,13 +920,14 @@ inlm_status inlm_selftest_division(int32_t device, uint64_t *mismatches, uint64_
     const unsigned count = (cb - 0x80000000u) + 1u;
     hipError_t e = hipMemset(cnt, 0, 16);
     if (e == hipSuccess) e = inlm::launch_selftest_div(0u, count, cnt, reinterpret_cast<unsigned *>(cnt + 1), nullptr);
+    if (e == hipSuccess) e = inlm::launch_selftest_third(cnt, reinterpret_cast<unsigned *>(cnt + 1), nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     unsigned long long host[2] = {0, 0};
     if (e == hipSuccess) e = hipMemcpy(host, cnt, 16, hipMemcpyDeviceToHost);
     (void)hipFree(cnt);
     if (e != hipSuccess) return hip_fail(nullptr, e, "division self-test");
     *mismatches = host[0];
-    *checked = count;
+    *checked = ((uint64_t)1 << 32) + count;
     if (example) *example = (uint32_t)host[1];
     return INLM_OK;
 }

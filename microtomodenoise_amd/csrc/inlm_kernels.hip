@@ -175,7 +175,7 @@ struct TiledArgs {
 // (n in [0, 120], d in [120, 600]: no overflow, underflow or special value):
 // the quotient by the hardware reciprocal and one correction with the exact
 // fused remainder.  Both are functions of one float, and
-// filter_selftest_div compares the weight with IEEE division on every float
+// selftest_div_kernel compares the weight with IEEE division on every float
 // of its domain, so neither a refined reciprocal nor a second correction
 // (four more instructions, as a general division needs) is kept.
 __device__ __forceinline__ float div_pade(float n, float d)
@@ -624,9 +624,9 @@ __global__ __launch_bounds__(NT) void filter_rgb_fp32(RgbArgs a)
 }
 
 // x / 3, correctly rounded: the product with the rounded reciprocal and one
-// correction with the exact fused remainder (checked on every float: only -0
-// gives +0, which weighs alike), about half the instructions of a general
-// division; infinities stay as they are.
+// correction with the exact fused remainder (only -0 gives +0, which weighs
+// alike; selftest_third_kernel checks every float), about half the
+// instructions of a general division; infinities stay as they are.
 __device__ __forceinline__ float third(float x)
 {
     constexpr float r3 = 1.f / 3.f;
@@ -1288,7 +1288,31 @@ __global__ __launch_bounds__(NT) void selftest_div_kernel(unsigned first, unsign
     if (bad) atomicAdd(mismatch, (unsigned long long)bad);
 }
 
+// Every float, by bit pattern: the joint colour filter's division by three
+// against IEEE division.
+__global__ __launch_bounds__(NT) void selftest_third_kernel(unsigned long long *mismatch, unsigned *example)
+{
+    const unsigned long stride = (unsigned long)gridDim.x * NT;
+    unsigned bad = 0;
+    for (unsigned long i = (unsigned long)blockIdx.x * NT + threadIdx.x; i < (1ul << 32); i += stride) {
+        const float x = __uint_as_float((unsigned)i), got = third(x), want = x / 3.f;
+        const bool same = __float_as_uint(got) == __float_as_uint(want) || (got != got && want != want) ||
+                          ((unsigned)i == 0x80000000u && got == 0.f);
+        if (!same) {
+            bad++;
+            *example = (unsigned)i;
+        }
+    }
+    if (bad) atomicAdd(mismatch, (unsigned long long)bad);
+}
+
 }  // namespace
+
+hipError_t launch_selftest_third(unsigned long long *mismatch, unsigned *example, hipStream_t st)
+{
+    hipLaunchKernelGGL(selftest_third_kernel, dim3(8192), dim3(NT), 0, st, mismatch, example);
+    return hipGetLastError();
+}
 
 hipError_t launch_selftest_div(unsigned first, unsigned count, unsigned long long *mismatch, unsigned *example,
                                hipStream_t st)

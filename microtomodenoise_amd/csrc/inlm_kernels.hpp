@@ -69,6 +69,9 @@ bool tiled_pays(int shape, int nx, int ny, int nz);
 // first+count).
 hipError_t launch_selftest_div(unsigned first, unsigned count, unsigned long long *mismatch, unsigned *example,
                                hipStream_t st);
+// The same for the joint colour filter's division by three, over every float;
+// adds to the counts.
+hipError_t launch_selftest_third(unsigned long long *mismatch, unsigned *example, hipStream_t st);
 
 // Patch standard deviation per sample (one wavefront per sample).  Sample
 // indices are linear in the unpadded volume (nx, nslice = nx*ny); the volume

@@ -10,6 +10,7 @@ channels do not mix, and with two flat channels the joint filter is the
 volume filter at sigma * sqrt(3).  The GPU tests compare the HIP path with
 the oracle bit for bit (FP32) and the schedule with a restatement built on
 the oracle's filter."""
+import ctypes as C
 import os
 import time
 
@@ -244,6 +245,16 @@ def test_filter_bit_exact_vs_oracle(gpu_available, rs, rp, shape, independent):
     ref = O.filter_rgb(img, img, [14.0] * 3, _op(rs, rp), independent)
     assert np.array_equal(log, np.full((1, 3), 14.0, F))
     assert np.array_equal(_bits(out), _bits(ref))
+
+
+@pytest.mark.gpu
+def test_third_selftest_exhaustive(gpu_available):
+    """The joint filter's division by three equals IEEE division on every
+    float (-0 gives +0); counted with the Pade weight's division."""
+    mism, checked, ex = C.c_uint64(), C.c_uint64(), C.c_uint32()
+    _capi.check(_capi.lib().inlm_selftest_division(0, C.byref(mism), C.byref(checked), C.byref(ex)))
+    assert checked.value > 2 ** 32 + 1_000_000_000
+    assert mism.value == 0, f"{mism.value} mismatches, e.g. bits {ex.value:#x}"
 
 
 @pytest.mark.gpu
