@@ -200,8 +200,8 @@ INLM_API inlm_status inlm_patchstd_noalloc(const float *vol, const int32_t shape
                                            const int64_t *samples, int64_t n, double *out, int32_t device);
 
 /* Noise level per slice (NoiseLevel::get_noiselevel, noiselevel.cpp:9-95):
- * patch std and two-cluster EM (FP64) on the GPU, global or
- * z-adaptive, sigma = mean + stds_from_mean * std.  Writes nz floats. */
+ * patch std and two-cluster EM (FP64) on the GPU (the EM of few samples on
+ * the host), global or z-adaptive, sigma = mean + stds_from_mean * std.  Writes nz floats. */
 INLM_API inlm_status inlm_estimate_noise(inlm_handle *h, int32_t which, const int64_t *samples, int64_t n,
                                          float *sigma_out);
 

@@ -476,8 +476,9 @@ filter_tiled_fp32(TiledArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Per-voxel kernel for any tap table without a tiled kernel: one thread per voxel, gathers straight from global memory, the
-// same operation sequence as the tiled kernel.
+// Per-voxel kernel for any tap table without a tiled kernel, and for volumes
+// too thin for the tiles (tiled_pays): one thread per voxel, gathers straight
+// from global memory, the same operation sequence as the tiled kernel.
 // ---------------------------------------------------------------------------
 struct VoxelArgs {
     const float *R;

@@ -12,9 +12,9 @@
 // act[((z+1)*(ny+2) + (y+1))*(nx+2) + (x+1)][16].  Convolutions 2..4 (forward
 // and the gradient with respect to their input) are implicit GEMMs on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation: 16 consecutive voxels x
-// 16 output channels, K = 27 taps x 16 channels in 14 chunks of two taps.  Their weight gradients (a reduction over all voxels)
-// run there too; the first layer (one input channel) runs on the vector ALUs
-// in FP32.
+// 16 output channels, K = 27 taps x 16 channels in 14 chunks of two taps.
+// Their weight gradients (a reduction over all voxels) run there too; the
+// first layer (one input channel) runs on the vector ALUs in FP32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -91,8 +91,8 @@ __global__ __launch_bounds__(256) void conv1_fwd(const float *__restrict__ in, c
 // a 16-byte read at 32-byte voxel pitch hits 16 distinct bank groups in each
 // 16-lane service group.  One wave per 16 voxels reading the input and the
 // weights of every product from global memory took 1.22 ms a layer on a
-// 256^3 volume, bound by the L1; this takes 0.42 ms forward (550 TFLOP/s)
-// and 0.57 ms backward, where each row's mask is loaded one row ahead.
+// 256^3 volume, bound by the L1; this takes 0.43 ms forward (535 TFLOP/s)
+// and 0.56 ms backward, where each row's mask is loaded one row ahead.
 // ---------------------------------------------------------------------------
 constexpr int kConvBlocks = 512;
 constexpr int CTX = 32, CTY = 8, CTZ = 4;
@@ -230,7 +230,7 @@ static_assert(kHeadShares * (C + 1) * (long)kMaxProposalOffsets <= (long)kWgradB
 // 39 KB) and G (16 KB) per tile, two blocks per CU.  The form before it, one
 // thread per (k, n) pair with 27 shifted copies of X in LDS, read one LDS
 // dword per multiply-add and one block filled a CU's LDS: 37.7 ms a layer on
-// a 256^3 volume against 0.34 ms (680 TFLOP/s), which the tiles' loads
+// a 256^3 volume against 0.37 ms (630 TFLOP/s), which the tiles' loads
 // through L2 (1.8 GB) and the LDS reads (56 per 28 MFMAs) bound together.
 constexpr int WTX = 32, WTY = 4, WTZ = 4;
 constexpr int WRX = WTX + 2, WRY = WTY + 2, WRZ = WTZ + 2;
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256, 2) void conv16_wgrad(const __bf16 *__restrict_
 // vector ALUs bound it (14.5 GFLOP on a 256^3 volume: 0.18 ms at their rate);
 // the loads of the next 64 voxels are in flight meanwhile, two waves a SIMD.
 // A thread per channel with X in LDS read one dword per multiply-add and used
-// 16 of 256 threads: 4.2 ms with 2048 blocks there, 0.77 ms here.
+// 16 of 256 threads: 4.2 ms with 2048 blocks there, 0.89 ms here.
 __global__ __launch_bounds__(192, 2) void conv1_wgrad(const float *__restrict__ X, const __bf16 *__restrict__ G,
                                                       float *__restrict__ part, ActGeom g)
 {
