@@ -149,7 +149,7 @@ inlm_status denoise_rgb(const inlm_params *pin, const inlm_rgb_options *c, const
     inlm_params pc = p;
     if (pc.noise_mode == INLM_NOISE_ZADAPTIVE) pc.noise_mode = INLM_NOISE_GLOBAL;
     int64_t semi_ref[3] = {-1, -1, -1};
-    const bool cluster = 3 * ns > kHostClusterSamples && pc.noise_mode == INLM_NOISE_GLOBAL;
+    const bool cluster = ns > 0 && pc.noise_mode == INLM_NOISE_GLOBAL;
     if (cluster) {  // a window of the clustering per channel
         const int64_t bounds[6] = {0, ns - 1, ns, 2 * ns - 1, 2 * ns, 3 * ns - 1};
         RGB_HIP(hipMalloc(&bC.p, sizeof(bounds) + 6 * sizeof(double)));
