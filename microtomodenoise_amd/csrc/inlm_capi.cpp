@@ -90,13 +90,15 @@ size_t cluster_bytes(int nz) { return kClusterWorkBytes + (size_t)nz * 2 * (size
 bool clusters_on_host(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n)
 {
     if (p.noise_mode != INLM_NOISE_GLOBAL && p.noise_mode != INLM_NOISE_ZADAPTIVE) return true;
-    if (n > kHostClusterSamples) return false;  // every sample lies in a window
-    if (p.noise_mode == INLM_NOISE_GLOBAL || n <= 0) return true;
+    if (n <= 0) return true;
+    if (n > kHostClusterCost) return false;  // every sample lies in a window
+    auto cost = [](int64_t len) { return len > 0 ? len * (64 - __builtin_clzll((unsigned long long)len)) : 0; };
+    if (p.noise_mode == INLM_NOISE_GLOBAL) return cost(n) <= kHostClusterCost;
     std::vector<int64_t> bounds;
     zwindow_bounds(samples, n, shape, p.zwindow, bounds);
     int64_t total = 0;
-    for (size_t i = 0; i < bounds.size(); i += 2) total += bounds[i + 1] - bounds[i] + 1;
-    return total <= kHostClusterSamples;
+    for (size_t i = 0; i < bounds.size(); i += 2) total += cost(bounds[i + 1] - bounds[i] + 1);
+    return total <= kHostClusterCost;
 }
 
 inlm_status sigma_on_device(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n,

@@ -21,13 +21,15 @@ void set_global_error(const std::string &msg);
 inlm_status sigma_from_std(const inlm_params &p, const int shape[3], const int64_t *samples, const double *sd,
                            int64_t n, int which, int64_t &semi_ref, float *sig, std::string &err);
 
-// Whether sigma_from_std is the quicker one: no clustering, or one whose
-// windows hold at most kHostClusterSamples in all (a sample of several windows
-// counts in each).  The GPU takes about 25 us more than the host for a few
-// samples, the host 35 us for 1000: an estimate of 300 samples in one window
-// takes 38 us by the host and 54 by the GPU, of 1000 57 to 70 and 60 to 68, of
-// 300 in the 16 windows of 5 slices of 64x64x16 (1500 in all) 65 and 62.
-constexpr int64_t kHostClusterSamples = 1024;
+// Whether sigma_from_std is the quicker one: no clustering, or one of few
+// samples.  Its time goes with the samples of all windows, times their
+// iterations, which grow with a window: samples times their count's bits.  The
+// GPU takes 10 to 30 us more than the host for a few samples.  An estimate by
+// the host and the GPU, us: one window of 300 samples (cost 2700) 38 / 54, of
+// 700 (7000) 48 / 56, of 1000 (10000) 57 to 70 / 60 to 68; 64 windows of about
+// 24 (7800) 51 / 62, 256 of 5 (3900) 39 / 49, 16 of 94 (10600) 65 / 62, 16 of
+// 100 (11300) 88 / 59.
+constexpr int64_t kHostClusterCost = 9000;
 bool clusters_on_host(const inlm_params &p, const int shape[3], const int64_t *samples, int64_t n);
 
 // The same in the global and z-adaptive modes from standard deviations on the

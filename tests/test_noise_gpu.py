@@ -121,7 +121,7 @@ def test_clustering_beyond_the_bits_in_lds(gpu_available):
     assert np.allclose(got, want, rtol=2e-7, atol=0), (got, want)
 
 
-@pytest.mark.parametrize("mode,window,n", [("global", 0, 20), ("global", 0, 200), ("z-adaptive", 4, 50)])
+@pytest.mark.parametrize("mode,window,n", [("global", 0, 20), ("global", 0, 200), ("z-adaptive", 4, 50), ("z-adaptive", 1, 300)])
 def test_few_samples_cost_no_more_than_the_host_clustering(gpu_available, mode, window, n):
     """An estimate of a few samples takes the time of their patch statistics
     and the host's clustering (1.3 to 1.8 times that when clustered on the
